@@ -502,11 +502,13 @@ int launch_erosion(fs_model *m, const std::vector<Span> &spans) {
 }
 
 int launch_receivers(fs_model *m) {
-  const unsigned gx = static_cast<unsigned>((m->W - 4 + 255) / 256);
-  const int strips = (m->H - 4 + kRecvRows - 1) / kRecvRows;
-  const unsigned gy = static_cast<unsigned>(std::min((strips + kRecvStrips - 1) / kRecvStrips, 65535));
+  // a wave's 64 columns x kRecvShort rows, four waves down a workgroup
+  const unsigned gx = static_cast<unsigned>((m->W - 4 + kWave - 1) / kWave);
+  const int groups = (m->H - 4 + kRecvShort - 1) / kRecvShort;
+  const unsigned gyz = static_cast<unsigned>((groups + 256 / kWave - 1) / (256 / kWave));
+  const unsigned gy = std::min(gyz, 65535u), gz = (gyz + gy - 1) / gy;   // grid.y's limit
   FS_TRY(kt_begin(m, FS_K_RECEIVERS));
-  hipLaunchKernelGGL(k_receivers, dim3(gx, gy), dim3(256), 0, m->stream, m->h, m->rcv, m->W, m->H,
+  hipLaunchKernelGGL(k_receivers, dim3(gx, gy, gz), dim3(256), 0, m->stream, m->h, m->rcv, m->W, m->H,
                      m->d_card, m->d_diag, m->hdr);
   FS_TRY(check_launch());
   return kt_end(m);

@@ -195,7 +195,6 @@ __global__ void k_fill_counts(int32_t *hdr, int n_counts) {
 // built per row in scalar registers: the lane's column is a constant offset,
 // so the loop spends no vector instructions on addresses.
 constexpr int kRecvRows = 16;
-constexpr int kRecvStrips = 2;                  // strips per thread in k_receivers
 constexpr int kRsrcWord3 = 0x00020000;          // raw (unformatted) buffer, gfx9
 using v4u = unsigned __attribute__((ext_vector_type(4)));
 using v2u = unsigned __attribute__((ext_vector_type(2)));
@@ -276,24 +275,49 @@ __device__ __forceinline__ void receivers_strips(const double *__restrict__ h,
   if (n > 0) receivers_rows(h, rcv, W, x, y0, n, d_card, d_diag);
 }
 
+// Receivers of one grid: each wave owns 64 columns x kRecvShort rows, with all
+// its kRecvShort + 2 rows requested before the first is used, so a cell waits
+// for memory once.  The rolling window above (32 rows per thread, one row
+// ahead) left small grids to a chain of 32 dependent row loads on a few
+// waves: 15 us at 101^2 and at 1000^2 alike.  Six rows were the best of 1 to
+// 16 at every size: 19.1 -> 9.0 us at 1000^2, 22.4 -> 15.9 at 2048^2, 93.5 ->
+// 86.3 at 6000^2, 227 -> 223.5 at 10000^2 (HIP events, their own 4 us
+// included); four rows read 1.5 rows per row decided (241 us at 10000^2),
+// sixteen leave too few waves (12.1 at 1000^2).  Bound by VALU issue at the
+// largest sizes (1.04 GB in 0.22 ms).
 // Also clears the header words the tile path's accumulation reports into
-// (hdr[0], hdr[1], hdr[3]; as k_fill_counts with no level counts).  Compiled
-// for eight waves per SIMD (its waves wait on memory most of their cycles;
-// 106 scalar registers held it to fewer).
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_receivers(const double *__restrict__ h,
+// (hdr[0], hdr[1], hdr[3]; as k_fill_counts with no level counts).
+constexpr int kRecvShort = 6;
+__global__ __launch_bounds__(256) void k_receivers(const double *__restrict__ h,
                                                    uint8_t *__restrict__ rcv, int W, int H,
                                                    double d_card, double d_diag,
                                                    int32_t *__restrict__ hdr) {
+  constexpr int ROWS = kRecvShort;
   if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
     hdr[0] = 0;
     hdr[1] = 0;
     hdr[3] = 0;
   }
-  const int x = blockIdx.x * 256 + threadIdx.x + 2;
-  if (x >= W - 2) return;
-  const int nstrips = (H - 4 + kRecvRows - 1) / kRecvRows;
-  for (int s = blockIdx.y * kRecvStrips; s < nstrips; s += gridDim.y * kRecvStrips)
-    receivers_strips(h, rcv, W, H, x, s, min(s + kRecvStrips, nstrips), d_card, d_diag);
+  const int x = blockIdx.x * kWave + static_cast<int>(threadIdx.x % kWave) + 2;
+  const int group = __builtin_amdgcn_readfirstlane(
+      (blockIdx.z * gridDim.y + blockIdx.y) * (256 / kWave) + threadIdx.x / kWave);
+  const int y0 = group * ROWS + 2;
+  if (x >= W - 2 || y0 >= H - 2) return;
+  const bool div_ok = fs::divisors_in_range(d_card, d_diag);
+  const uint32_t rowb = static_cast<uint32_t>(W) * 8u;
+  const uint32_t xo = static_cast<uint32_t>(x - 1) * 8u;
+  double l[ROWS + 2], c[ROWS + 2], r[ROWS + 2];
+#pragma unroll
+  for (int k = 0; k < ROWS + 2; k++)   // past the grid's last row: that row again
+    load_cols(row_rsrc(h + static_cast<size_t>(min(y0 - 1 + k, H - 1)) * W, rowb), xo, l[k], c[k],
+              r[k]);
+#pragma unroll
+  for (int k = 0; k < ROWS; k++) {
+    if (y0 + k >= H - 2) break;
+    const double nb[8] = {l[k + 1], l[k], c[k], r[k], r[k + 1], r[k + 2], c[k + 2], l[k + 2]};
+    rcv[static_cast<size_t>(y0 + k) * W + x] =
+        static_cast<uint8_t>(fs::receiver_fast(c[k + 1], nb, d_card, d_diag, div_ok));
+  }
 }
 
 // Donor bitmask and level of every cell.  Rows are strided over the grid so
