@@ -87,8 +87,6 @@ struct fs_model {
   ErodeConst ek{};
   int nmode = 1;
   hipStream_t stream = nullptr;
-  hipStream_t side = nullptr;     // header read-back of the tile path
-  hipEvent_t acc_done = nullptr;  // tile accumulation finished on `stream`
 
   // device state; h and h_alt swap after each tile-path step
   double *h = nullptr, *h_alt = nullptr;
@@ -133,9 +131,19 @@ struct fs_model {
   double stage_ms[FS_NUM_TIMERS] = {};
   hipEvent_t ev[2][7] = {};
   bool ev_pending[2] = {false, false};
-  bool ev_tile[2] = {false, false};   // that step took the tile path
-  int ev_cur = 0;
-  double tile_acc_ms = 0, tile_ero_ms = 0;   // tile kernels' time not yet split
+  int ev_cur = 0;                     // level-path steps alternate the two sets
+  // Tile and tile-graph steps are not bracketed by events one by one: a batch
+  // (or a run of tile-graph steps) is, and its first step's kernels are the
+  // sample its time is split by.
+  hipEvent_t tev[5] = {};             // batch: start, the sampled step's kernels, end
+  double tile_ms = 0;                 // tile batches' time not yet split over the stages
+  double samp_ms[3] = {};             // sampled receivers, accumulation, erosion
+  long long since_sample = 0;         // tile steps since the last sampled one
+  hipEvent_t gev[8] = {};             // tile-graph run: its first step's stages, end
+  bool graph_open = false, graph_pending = false;
+  int batch = 4;                      // tile steps launched before the host looks
+  bool hdr_fresh = false;             // hdr_h holds the header, nothing launched since
+  bool err_left = false;              // the header may hold an earlier call's error bits
 
   // false for a model whose device buffers are lent to it (the entry point
   // that allocates nothing): no lazy allocations, no events, no side stream
@@ -224,31 +232,54 @@ int stage_collect(fs_model *m, int set) {
   float ms[6] = {};
   for (int i = 0; i < 6; i++)
     FS_HIP_TRY(hipEventElapsedTime(&ms[i], m->ev[set][i], m->ev[set][i + 1]));
-  if (m->ev_tile[set]) {
-    // donors..erosion ran fused in the two tile kernels; split_tile_time
-    // assigns their time to the stages
-    m->stage_ms[FS_T_RECEIVERS] += ms[0];
-    m->tile_acc_ms += ms[1] + ms[2] + ms[3] + ms[4];
-    m->tile_ero_ms += ms[5];
-  } else {
-    for (int i = 0; i < 6; i++) m->stage_ms[FS_T_RECEIVERS + i] += ms[i];
-  }
+  for (int i = 0; i < 6; i++) m->stage_ms[FS_T_RECEIVERS + i] += ms[i];
   m->ev_pending[set] = false;
   return FS_OK;
 }
 
-// Split the tile kernels' event time over the reference's stages in
-// proportion to the phase ticks their sampled workgroups recorded on the
-// timed steps:
+// Ends a run of tile-graph steps for the stage timers (its time is collected
+// once the stream has passed this point).
+int graph_close(fs_model *m) {
+  if (!m->graph_open) return FS_OK;
+  m->graph_open = false;
+  FS_HIP_TRY(hipEventRecord(m->gev[7], m->stream));
+  m->graph_pending = true;
+  return FS_OK;
+}
+
+// The time of a finished run of tile-graph steps, split over the stages in
+// proportion to its first step's.
+int graph_collect(fs_model *m) {
+  if (!m->graph_pending) return FS_OK;
+  FS_HIP_TRY(hipEventSynchronize(m->gev[7]));
+  m->graph_pending = false;
+  float ms[6] = {}, all = 0.f;
+  double sum = 0;
+  for (int i = 0; i < 6; i++) {
+    FS_HIP_TRY(hipEventElapsedTime(&ms[i], m->gev[i], m->gev[i + 1]));
+    sum += ms[i];
+  }
+  FS_HIP_TRY(hipEventElapsedTime(&all, m->gev[0], m->gev[7]));
+  for (int i = 0; i < 6 && sum > 0; i++)
+    m->stage_ms[FS_T_RECEIVERS + i] += static_cast<double>(all) * ms[i] / sum;
+  return FS_OK;
+}
+
+// Split the tile batches' event time over the reference's stages: over the
+// three kernels in proportion to the sampled steps' event times, and the two
+// tile kernels' shares in proportion to the phase ticks their sampled
+// workgroups recorded on those steps:
 // k_tile_acc's region load -> DetermineDonors, its chain walks and
 // count/level stores -> FlowAcc, its halo-chain marking and erosion plan ->
 // GenerateOrder; k_tile_erode's level bucketing -> GenerateOrder, its outlet
 // uplift -> Uplift, its wavefront and stores -> Erosion.
 int split_tile_time(fs_model *m) {
-  if (m->tile_acc_ms <= 0 && m->tile_ero_ms <= 0) return FS_OK;
+  if (m->tile_ms <= 0) return FS_OK;
   double ph[kPhaseStride] = {};
   if (m->phase) {
     std::vector<unsigned long long> raw(static_cast<size_t>(kPhaseSlots) * kPhaseStride);
+    FS_HIP_TRY(hipSetDevice(m->device));
+    FS_HIP_TRY(hipStreamSynchronize(m->stream));
     FS_HIP_TRY(hipMemcpy(raw.data(), m->phase, raw.size() * sizeof(raw[0]),
                          hipMemcpyDeviceToHost));
     for (int r = 0; r < kPhaseSlots; r++)
@@ -256,23 +287,40 @@ int split_tile_time(fs_model *m) {
         ph[i] += static_cast<double>(raw[static_cast<size_t>(r) * kPhaseStride + i]);
     FS_HIP_TRY(hipMemset(m->phase, 0, raw.size() * sizeof(raw[0])));
   }
+  const double samp = m->samp_ms[0] + m->samp_ms[1] + m->samp_ms[2];
+  const double per = samp > 0 ? m->tile_ms / samp : 0;
+  m->stage_ms[FS_T_RECEIVERS] += per * m->samp_ms[0];
+  const double acc_ms = per * m->samp_ms[1], ero_ms = per * m->samp_ms[2];
   const double acc = ph[kPhAccLoad] + ph[kPhAccWalk] + ph[kPhAccPlan] + ph[kPhAccStore];
   if (acc > 0) {
-    m->stage_ms[FS_T_DONORS] += m->tile_acc_ms * ph[kPhAccLoad] / acc;
-    m->stage_ms[FS_T_FLOWACC] += m->tile_acc_ms * (ph[kPhAccWalk] + ph[kPhAccStore]) / acc;
-    m->stage_ms[FS_T_ORDER] += m->tile_acc_ms * ph[kPhAccPlan] / acc;
+    m->stage_ms[FS_T_DONORS] += acc_ms * ph[kPhAccLoad] / acc;
+    m->stage_ms[FS_T_FLOWACC] += acc_ms * (ph[kPhAccWalk] + ph[kPhAccStore]) / acc;
+    m->stage_ms[FS_T_ORDER] += acc_ms * ph[kPhAccPlan] / acc;
   } else {
-    m->stage_ms[FS_T_FLOWACC] += m->tile_acc_ms;
+    m->stage_ms[FS_T_FLOWACC] += acc_ms;
   }
   const double ero = ph[kPhEroBucket] + ph[kPhEroRoots] + ph[kPhEroLoop] + ph[kPhEroStore];
   if (ero > 0) {
-    m->stage_ms[FS_T_ORDER] += m->tile_ero_ms * ph[kPhEroBucket] / ero;
-    m->stage_ms[FS_T_UPLIFT] += m->tile_ero_ms * ph[kPhEroRoots] / ero;
-    m->stage_ms[FS_T_EROSION] += m->tile_ero_ms * (ph[kPhEroLoop] + ph[kPhEroStore]) / ero;
+    m->stage_ms[FS_T_ORDER] += ero_ms * ph[kPhEroBucket] / ero;
+    m->stage_ms[FS_T_UPLIFT] += ero_ms * ph[kPhEroRoots] / ero;
+    m->stage_ms[FS_T_EROSION] += ero_ms * (ph[kPhEroLoop] + ph[kPhEroStore]) / ero;
   } else {
-    m->stage_ms[FS_T_EROSION] += m->tile_ero_ms;
+    m->stage_ms[FS_T_EROSION] += ero_ms;
   }
-  m->tile_acc_ms = m->tile_ero_ms = 0;
+  m->tile_ms = 0;
+  for (double &v : m->samp_ms) v = 0;
+  return FS_OK;
+}
+
+// The stage times of every step so far, into the timers.
+int fold_timers(fs_model *m) {
+  FS_TRY(split_tile_time(m));
+  for (int i = 0; i < 6; i++) {
+    const double ms = m->stage_ms[FS_T_RECEIVERS + i];
+    const uint64_t whole = static_cast<uint64_t>(ms * 1000.0);
+    m->timer_us[FS_T_RECEIVERS + i] += whole;
+    m->stage_ms[FS_T_RECEIVERS + i] = ms - static_cast<double>(whole) / 1000.0;
+  }
   return FS_OK;
 }
 
@@ -333,8 +381,10 @@ void free_model(fs_model *m) {
     (void)hipEventDestroy(t.b);
   }
   for (auto e : m->kfree) (void)hipEventDestroy(e);
-  if (m->acc_done) (void)hipEventDestroy(m->acc_done);
-  if (m->side) (void)hipStreamDestroy(m->side);
+  for (auto e : m->tev)
+    if (e) (void)hipEventDestroy(e);
+  for (auto e : m->gev)
+    if (e) (void)hipEventDestroy(e);
   if (m->stream) (void)hipStreamDestroy(m->stream);
   delete m;
 }
@@ -366,10 +416,10 @@ int create_model(int W, int H, const fs_params *p, const double *h_init, uint32_
   m->ek = make_erode_const(*p, &m->nmode);
   FS_HIP_TRY(hipSetDevice(device));
   FS_HIP_TRY(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking));
-  FS_HIP_TRY(hipStreamCreateWithFlags(&m->side, hipStreamNonBlocking));
-  FS_HIP_TRY(hipEventCreateWithFlags(&m->acc_done, hipEventDisableTiming));
   for (auto &set : m->ev)
     for (auto &e : set) FS_HIP_TRY(hipEventCreate(&e));
+  for (auto &e : m->tev) FS_HIP_TRY(hipEventCreate(&e));
+  for (auto &e : m->gev) FS_HIP_TRY(hipEventCreate(&e));
 
   const size_t N = static_cast<size_t>(m->N);
   const size_t ntiles = (N + kBfsTile - 1) / kBfsTile + 1;
@@ -501,15 +551,18 @@ int launch_erosion(fs_model *m, const std::vector<Span> &spans) {
   return FS_OK;
 }
 
-int launch_receivers(fs_model *m) {
+// prev and slot: the tile batch's slots of the previous step and this one
+// (null off the tile path).
+int launch_receivers(fs_model *m, const double *h, const int32_t *prev = nullptr,
+                     int32_t *slot = nullptr, int shallow = -1) {
   // a wave's 64 columns x kRecvShort rows, four waves down a workgroup
   const unsigned gx = static_cast<unsigned>((m->W - 4 + kWave - 1) / kWave);
   const int groups = (m->H - 4 + kRecvShort - 1) / kRecvShort;
   const unsigned gyz = static_cast<unsigned>((groups + 256 / kWave - 1) / (256 / kWave));
   const unsigned gy = std::min(gyz, 65535u), gz = (gyz + gy - 1) / gy;   // grid.y's limit
   FS_TRY(kt_begin(m, FS_K_RECEIVERS));
-  hipLaunchKernelGGL(k_receivers, dim3(gx, gy, gz), dim3(256), 0, m->stream, m->h, m->rcv, m->W, m->H,
-                     m->d_card, m->d_diag, m->hdr);
+  hipLaunchKernelGGL(k_receivers, dim3(gx, gy, gz), dim3(256), 0, m->stream, h, m->rcv, m->W,
+                     m->H, m->d_card, m->d_diag, m->hdr, prev, slot, shallow);
   FS_TRY(check_launch());
   return kt_end(m);
 }
@@ -668,43 +721,35 @@ int level_path(fs_model *m, hipEvent_t *ev) {
 }
 
 template <int NMODE, bool kTimed>
-int launch_tile_erode(fs_model *m, int tiles, int tiles_x, int halo) {
+int launch_tile_erode(fs_model *m, int halo, const double *h_in, double *h_out,
+                      const int32_t *slot) {
+  const int tiles_x = (m->W + kTile - 1) / kTile, tiles = tiles_x * ((m->H + kTile - 1) / kTile);
   if (halo == kHalo)
     hipLaunchKernelGGL((k_tile_erode<NMODE, kTimed>), dim3(tiles), dim3(kEroBlock), 0, m->stream,
-                       m->h, m->h_alt, m->plan, m->lvl, m->cnt, m->ftab, m->W, m->H, tiles_x,
-                       tiles, m->ek, m->hdr, m->phase);
+                       h_in, h_out, m->plan, m->lvl, m->cnt, m->ftab, m->W, m->H, tiles_x,
+                       tiles, m->ek, m->hdr, slot, m->phase);
   else
     hipLaunchKernelGGL((tile32::k_tile_erode<NMODE, kTimed>), dim3(tiles), dim3(tile32::kEroBlock),
-                       0, m->stream, m->h, m->h_alt, m->plan32, m->lvl, m->cnt, m->ftab, m->W,
-                       m->H, tiles_x, tiles, m->ek, m->hdr, m->phase);
+                       0, m->stream, h_in, h_out, m->plan32, m->lvl, m->cnt, m->ftab, m->W,
+                       m->H, tiles_x, tiles, m->ek, m->hdr, slot, m->phase);
   return check_launch();
 }
 
 template <int NMODE>
-int launch_tile_erode(fs_model *m, int tiles, int tiles_x, int halo, bool timed) {
-  return timed ? launch_tile_erode<NMODE, true>(m, tiles, tiles_x, halo)
-               : launch_tile_erode<NMODE, false>(m, tiles, tiles_x, halo);
+int launch_tile_erode(fs_model *m, int halo, const double *h_in, double *h_out,
+                      const int32_t *slot, bool timed) {
+  return timed ? launch_tile_erode<NMODE, true>(m, halo, h_in, h_out, slot)
+               : launch_tile_erode<NMODE, false>(m, halo, h_in, h_out, slot);
 }
 
-// Accumulation with the given halo (16 or 32), then the erosion with the
-// same halo launched behind it at once: the erosion grid does nothing when a
-// tile was too deep, so the host reads the accumulation's header on a side
-// stream while the erosion runs.  *fits = false when some level exceeds the
-// halo (or a tile's chains need more halo cells than its plan holds); the
-// erosion was then empty and hdr_h[0] is the deepest level among the cells
-// that reach an outlet within the region.  clear: reset the header first
-// (k_receivers already did for the first accumulation of a step).
-int tile_attempt(fs_model *m, int halo, int tiles, int tiles_x, bool clear, hipEvent_t *ev,
-                 bool *fits) {
+// One tile step's accumulation with the given halo (16 or 32) and the erosion
+// right behind it, on the receivers in rcv; both report into and obey the
+// step's slot.  timed: the instantiations that sample the phase ticks.
+// after_acc: an event to record between the two, or null.
+int launch_tile_step(fs_model *m, int halo, const double *h_in, double *h_out, int32_t *slot,
+                     bool timed, hipEvent_t after_acc) {
   hipStream_t s = m->stream;
-  *fits = false;
-  if (clear) {
-    hipLaunchKernelGGL(k_fill_counts, dim3(1), dim3(64), 0, s, m->hdr, 0);
-    FS_TRY(check_launch());
-  }
-  // one step in kPhaseEvery (and the first of each call) runs the timed
-  // instantiations that sample the phase ticks of the stage timers
-  const bool timed = m->phase && (m->steps_in_call == 0 || m->tile_steps % kPhaseEvery == 0);
+  const int tiles_x = (m->W + kTile - 1) / kTile, tiles = tiles_x * ((m->H + kTile - 1) / kTile);
   if (!m->ncu)
     FS_HIP_TRY(hipDeviceGetAttribute(&m->ncu, hipDeviceAttributeMultiprocessorCount, m->device));
   FS_TRY(kt_begin(m, FS_K_TILE_ACC));
@@ -714,18 +759,18 @@ int tile_attempt(fs_model *m, int halo, int tiles, int tiles_x, bool clear, hipE
     const bool wide = tiles < 4 * m->ncu;
     if (wide && timed)
       hipLaunchKernelGGL((k_tile_acc<true, kAccBlockWide>), dim3(tiles), dim3(kAccBlockWide), 0, s,
-                         m->rcv, m->cnt, m->lvl, m->plan, m->hdr, m->W, m->H, tiles_x, tiles,
+                         m->rcv, m->cnt, m->lvl, m->plan, slot, m->W, m->H, tiles_x, tiles,
                          m->phase);
     else if (wide)
       hipLaunchKernelGGL((k_tile_acc<false, kAccBlockWide>), dim3(tiles), dim3(kAccBlockWide), 0,
-                         s, m->rcv, m->cnt, m->lvl, m->plan, m->hdr, m->W, m->H, tiles_x, tiles,
+                         s, m->rcv, m->cnt, m->lvl, m->plan, slot, m->W, m->H, tiles_x, tiles,
                          m->phase);
     else if (timed)
       hipLaunchKernelGGL(k_tile_acc<true>, dim3(tiles), dim3(kAccBlock), 0, s, m->rcv, m->cnt,
-                         m->lvl, m->plan, m->hdr, m->W, m->H, tiles_x, tiles, m->phase);
+                         m->lvl, m->plan, slot, m->W, m->H, tiles_x, tiles, m->phase);
     else
       hipLaunchKernelGGL(k_tile_acc<false>, dim3(tiles), dim3(kAccBlock), 0, s, m->rcv, m->cnt,
-                         m->lvl, m->plan, m->hdr, m->W, m->H, tiles_x, tiles, m->phase);
+                         m->lvl, m->plan, slot, m->W, m->H, tiles_x, tiles, m->phase);
   } else {
     if (!m->plan32) {
       if (!m->owns_memory) return FS_ERR_INTERNAL;   // lent buffers include plan32
@@ -733,73 +778,127 @@ int tile_attempt(fs_model *m, int halo, int tiles, int tiles_x, bool clear, hipE
     }
     if (timed)
       hipLaunchKernelGGL(tile32::k_tile_acc<true>, dim3(tiles), dim3(tile32::kAccBlock), 0, s,
-                         m->rcv, m->cnt, m->lvl, m->plan32, m->hdr, m->W, m->H, tiles_x, tiles,
+                         m->rcv, m->cnt, m->lvl, m->plan32, slot, m->W, m->H, tiles_x, tiles,
                          m->phase);
     else
       hipLaunchKernelGGL(tile32::k_tile_acc<false>, dim3(tiles), dim3(tile32::kAccBlock), 0, s,
-                         m->rcv, m->cnt, m->lvl, m->plan32, m->hdr, m->W, m->H, tiles_x, tiles,
+                         m->rcv, m->cnt, m->lvl, m->plan32, slot, m->W, m->H, tiles_x, tiles,
                          m->phase);
   }
   FS_TRY(check_launch());
   FS_TRY(kt_end(m));
-  FS_TRY(mark(ev[2], s));
-  if (m->side) {
-    FS_HIP_TRY(hipEventRecord(m->acc_done, s));
-    FS_HIP_TRY(hipStreamWaitEvent(m->side, m->acc_done, 0));
-    FS_HIP_TRY(hipMemcpyAsync(m->hdr_h, m->hdr, kHdrInts * sizeof(int32_t),
-                              hipMemcpyDeviceToHost, m->side));
-  }
-  FS_TRY(mark(ev[3], s));
-  FS_TRY(mark(ev[4], s));
-  FS_TRY(mark(ev[5], s));
+  FS_TRY(mark(after_acc, s));
   FS_TRY(kt_begin(m, FS_K_TILE_ERODE));
-  if (m->nmode == 1) FS_TRY(launch_tile_erode<1>(m, tiles, tiles_x, halo, timed));
-  else if (m->nmode == 2) FS_TRY(launch_tile_erode<2>(m, tiles, tiles_x, halo, timed));
-  else FS_TRY(launch_tile_erode<0>(m, tiles, tiles_x, halo, timed));
-  FS_TRY(kt_end(m));
-  if (m->side) {
-    FS_HIP_TRY(hipStreamSynchronize(m->side));
-  } else {
-    // no side stream: read the header behind the erosion on the model's stream
-    FS_HIP_TRY(hipMemcpyAsync(m->hdr_h, m->hdr, kHdrInts * sizeof(int32_t),
-                              hipMemcpyDeviceToHost, s));
-    FS_HIP_TRY(hipStreamSynchronize(s));
-  }
-  FS_TRY(device_error_status(m->hdr_h[2]));
-  *fits = m->hdr_h[3] == 0;
-  return FS_OK;
+  if (m->nmode == 1) FS_TRY(launch_tile_erode<1>(m, halo, h_in, h_out, slot, timed));
+  else if (m->nmode == 2) FS_TRY(launch_tile_erode<2>(m, halo, h_in, h_out, slot, timed));
+  else FS_TRY(launch_tile_erode<0>(m, halo, h_in, h_out, slot, timed));
+  return kt_end(m);
 }
 
-// The tile path (every level <= 32): accumulation with a 16-cell halo, or a
-// 32-cell one when the drainage is deeper, and erosion with the same halo.
-// Returns FS_OK with *done = false when the levels are too deep for either
-// (both erosions were empty); the caller then runs the level path on the
-// same receivers.  The halo that fitted is tried first at the next step.
-int tile_path(fs_model *m, hipEvent_t *ev, bool *done) {
-  *done = false;
-  const int tiles_x = (m->W + kTile - 1) / kTile, tiles_y = (m->H + kTile - 1) / kTile;
-  const int tiles = tiles_x * tiles_y;
-  int halo = m->tile_halo == tile32::kHalo ? tile32::kHalo : kHalo;
-  bool fits = false;
-  FS_TRY(tile_attempt(m, halo, tiles, tiles_x, false, ev, &fits));
-  FS_TRY(stage_collect(m, m->ev_cur ^ 1));
-  FS_TRY(kt_collect(m));
-  if (!fits && halo == kHalo) {
-    halo = tile32::kHalo;
-    FS_TRY(tile_attempt(m, halo, tiles, tiles_x, true, ev, &fits));
+// The outcome of the tile steps launched so far: waits for them, reads the
+// header and adds the batch's time (bracketed by tev[0] and tev[4]).
+int finish_batch(fs_model *m, bool sampled) {
+  FS_TRY(mark(m->tev[4], m->stream));
+  FS_TRY(fetch_header(m, 0));
+  m->hdr_fresh = true;
+  if (m->tev[0]) {
+    float ms = 0.f;
+    FS_HIP_TRY(hipEventElapsedTime(&ms, m->tev[0], m->tev[4]));
+    m->tile_ms += ms;
+    for (int i = 0; i < 3 && sampled; i++) {
+      FS_HIP_TRY(hipEventElapsedTime(&ms, m->tev[i], m->tev[i + 1]));
+      m->samp_ms[i] += ms;
+    }
   }
-  if (!fits) {
-    m->tile_halo = kHalo;                   // the level path sets it from the depth it finds
-    return FS_OK;
-  }
-  // a 32-halo step whose levels all fit 16 tries the 16-cell halo next
-  m->tile_halo = (halo == tile32::kHalo && m->hdr_h[0] <= kHalo) ? kHalo : halo;
+  FS_TRY(graph_collect(m));
+  return kt_collect(m);
+}
+
+void take_tile_steps(fs_model *m, int n, int halo) {
+  if (n <= 0) return;
+  if (n & 1) std::swap(m->h, m->h_alt);
   m->order_current = false;                 // levels, stack, donor masks on request
   m->cnt_stack = false;
-  std::swap(m->h, m->h_alt);
-  m->tile_steps++;
-  if (halo != kHalo) m->tile32_steps++;
-  *done = true;
+  m->have_step = true;
+  m->tile_steps += static_cast<uint64_t>(n);
+  if (halo != kHalo) m->tile32_steps += static_cast<uint64_t>(n);
+}
+
+// Tile-path steps (every level <= 32): receivers, accumulation with a 16-cell
+// halo, or a 32-cell one when the drainage is deeper, and erosion with the
+// same halo, launched back to back for up to `want` steps; the host looks at
+// the outcome once per batch.  A step whose tiles are too deep for the halo
+// does not erode, and the steps behind it do nothing; so do the steps behind
+// a 32-halo step whose levels would fit the 16-cell halo, and those behind a
+// failed solve.  *done steps were taken; with *stuck the next one's receivers
+// are in rcv and its levels fit neither halo: the caller takes it another
+// way.  The halo that fitted is tried first at the next step.
+//
+// Waiting for the header at every step, and seven timer events a step, took
+// more than half of a small run: 73 -> 30 us a step at 101^2, 72 -> 36 at
+// 1000^2, 120 -> 84 at 1500x1101.  A batch that ends early wastes the launches
+// behind its end, so batches start at four steps and double while they end
+// well.
+int tile_steps(fs_model *m, long long want, int *done, bool *stuck) {
+  *done = 0;
+  *stuck = false;
+  const int halo = m->tile_halo == tile32::kHalo ? tile32::kHalo : kHalo;
+  // per-kernel timing counts launches, and a fill comes before every step
+  const int n = m->ktiming || m->fill_mode
+                    ? 1
+                    : static_cast<int>(std::min<long long>(want, std::min(m->batch, kMaxBatch)));
+  // the first step of each call and then one in kPhaseEvery is the timers' sample
+  const bool sample = m->phase && (m->steps_in_call == 0 || m->since_sample >= kPhaseEvery);
+  const hipEvent_t none = nullptr;
+  FS_TRY(mark(m->tev[0], m->stream));
+  double *h_in = m->h, *h_out = m->h_alt;
+  for (int i = 0; i < n; i++) {
+    int32_t *slot = m->hdr + kHdrSlots + i * kSlotInts;
+    const bool timed = sample && i == 0;
+    FS_TRY(launch_receivers(m, h_in, i ? slot - kSlotInts : nullptr, slot,
+                            halo == kHalo ? -1 : kHalo));
+    if (timed) FS_TRY(mark(m->tev[1], m->stream));
+    FS_TRY(launch_tile_step(m, halo, h_in, h_out, slot, timed, timed ? m->tev[2] : none));
+    if (timed) FS_TRY(mark(m->tev[3], m->stream));
+    std::swap(h_in, h_out);
+  }
+  FS_TRY(finish_batch(m, sample));
+  const int32_t *slots = m->hdr_h + kHdrSlots;
+  int taken = 0;
+  while (taken < n && slots[taken * kSlotInts + kSlotOver] == 0 &&
+         slots[taken * kSlotInts + kSlotStop] == 0)
+    taken++;
+  take_tile_steps(m, taken, halo);   // a failed solve's step was taken, none behind it
+  *done = taken;
+  FS_TRY(device_error_status(m->hdr_h[2]));
+  m->since_sample = sample ? n : m->since_sample + n;
+  m->batch = taken == n ? std::min(2 * m->batch, kMaxBatch) : 4;
+  if (taken == n || slots[taken * kSlotInts + kSlotStop] != 0) {
+    // a 32-halo step whose levels all fit 16 tries the 16-cell halo next
+    m->tile_halo = halo == tile32::kHalo && taken > 0 &&
+                           slots[(taken - 1) * kSlotInts + kSlotDeepest] <= kHalo
+                       ? kHalo
+                       : halo;
+    return FS_OK;
+  }
+  if (halo == kHalo) {
+    // the same step again with the 32-cell halo
+    int32_t *slot = m->hdr + kHdrSlots;
+    FS_TRY(mark(m->tev[0], m->stream));
+    hipLaunchKernelGGL(k_slot_reset, dim3(1), dim3(64), 0, m->stream, slot);
+    FS_TRY(check_launch());
+    FS_TRY(launch_tile_step(m, tile32::kHalo, m->h, m->h_alt, slot, false, none));
+    FS_TRY(finish_batch(m, false));
+    if (slots[kSlotOver] == 0) {
+      take_tile_steps(m, 1, tile32::kHalo);
+      m->tile_halo = slots[kSlotDeepest] <= kHalo ? kHalo : tile32::kHalo;
+      *done = taken + 1;
+    }
+    FS_TRY(device_error_status(m->hdr_h[2]));
+    if (*done > taken) return FS_OK;
+  }
+  m->tile_halo = kHalo;                     // the path that takes the step sets it again
+  *stuck = true;
   return FS_OK;
 }
 
@@ -885,8 +984,9 @@ int launch_graph_erosion(fs_model *m, int tiles) {
 
 // The tile-graph path (fs_deep.h): any depth, no halo, no host round trip.
 // Receivers are already in rcv.  Errors (a tier beyond kTierCap, a receiver
-// cycle, a wait that timed out) surface when the call finishes.
-int graph_path(fs_model *m, hipEvent_t *ev) {
+// cycle, a wait that timed out) surface when the call finishes.  ev: events
+// to record between the stages (null handles: none).
+int graph_path(fs_model *m, const hipEvent_t *ev) {
   FS_TRY(ensure_graph(m));
   hipStream_t s = m->stream;
   const int tiles = ((m->W + deep::kSide - 1) / deep::kSide) *
@@ -981,46 +1081,63 @@ int fill_depressions(fs_model *m) {
   return FS_OK;
 }
 
-// One time-step.
-int step_once(fs_model *m) {
-  hipEvent_t *ev = m->ev[m->ev_cur];
+// Up to `want` time-steps (at least one); *took receives how many.
+int advance(fs_model *m, long long want, int *took) {
+  *took = 0;
+  bool stuck = false;   // the step's receivers are in rcv
   if (m->fill_mode) FS_TRY(fill_depressions(m));
-  FS_TRY(mark(ev[0], m->stream));
-  FS_TRY(launch_receivers(m));
-  FS_TRY(mark(ev[1], m->stream));
-  bool done = false;
-  if (m->path == FS_PATH_AUTO && m->tile_halo != 0) FS_TRY(tile_path(m, ev, &done));
-  const bool tiled = done;
-  if (!done && (m->path == FS_PATH_TILE_GRAPH || (m->path == FS_PATH_AUTO && m->owns_memory))) {
+  if (m->path == FS_PATH_AUTO && m->tile_halo != 0) {
+    FS_TRY(graph_close(m));
+    FS_TRY(tile_steps(m, want, took, &stuck));
+    if (!stuck) return FS_OK;
+  }
+  m->hdr_fresh = false;
+  if (m->path == FS_PATH_TILE_GRAPH || (m->path == FS_PATH_AUTO && m->owns_memory)) {
+    // the first of a run of tile-graph steps is the timers' sample
+    static const hipEvent_t none[8] = {};
+    const hipEvent_t *ev = none;
+    if (!m->graph_open) {
+      FS_TRY(graph_collect(m));
+      m->graph_open = true;
+      ev = m->gev;
+    }
+    FS_TRY(mark(ev[0], m->stream));
+    if (!stuck) FS_TRY(launch_receivers(m, m->h));
+    FS_TRY(mark(ev[1], m->stream));
     FS_TRY(graph_path(m, ev));
-    done = true;
+    FS_TRY(mark(ev[6], m->stream));
     if (m->path == FS_PATH_AUTO) {
       // drainage this deep rarely shallows again: try the 32-cell halo
       // every kGraphRetry graph steps
       m->tile_halo = ++m->graph_run % kGraphRetry == 0 ? tile32::kHalo : 0;
     }
-  }
-  if (!done) {
+  } else {
+    FS_TRY(graph_close(m));
+    hipEvent_t *ev = m->ev[m->ev_cur];
+    FS_TRY(mark(ev[0], m->stream));
+    if (!stuck) FS_TRY(launch_receivers(m, m->h));
+    FS_TRY(mark(ev[1], m->stream));
     FS_TRY(level_path(m, ev));
     // the next step tries the tile halo this step's depth would have fitted
     const int D = static_cast<int>(m->counts.size()) - 1;
     m->tile_halo = D <= kHalo ? kHalo : D <= tile32::kHalo ? tile32::kHalo : 0;
+    FS_TRY(mark(ev[6], m->stream));
+    m->ev_pending[m->ev_cur] = ev[0] != nullptr;
+    m->ev_cur ^= 1;
   }
-  FS_TRY(mark(ev[6], m->stream));
-  m->ev_pending[m->ev_cur] = ev[0] != nullptr;
-  m->ev_tile[m->ev_cur] = tiled;
-  m->ev_cur ^= 1;
   m->have_step = true;
+  (*took)++;
   return FS_OK;
 }
 
 int finish(fs_model *m) {
-  FS_HIP_TRY(hipStreamSynchronize(m->stream));
+  FS_TRY(graph_close(m));
+  if (!m->hdr_fresh) FS_TRY(fetch_header(m, 0));   // waits for every step
   FS_TRY(stage_collect(m, 0));
   FS_TRY(stage_collect(m, 1));
+  FS_TRY(graph_collect(m));
   FS_TRY(kt_collect(m));
   FS_TRY(graph_status(m));
-  FS_TRY(fetch_header(m, 0));
   return device_error_status(m->hdr_h[2]);
 }
 
@@ -1029,29 +1146,24 @@ int run_steps(fs_model *m, long long iterations) {
   if (iterations < 0) return FS_ERR_INVALID_ARGUMENT;
   FS_HIP_TRY(hipSetDevice(m->device));
   const auto t0 = std::chrono::steady_clock::now();
-  // clear the device error word left by a previous call
-  FS_HIP_TRY(hipMemcpyAsync(m->hdr_h, m->hdr, kHdrInts * sizeof(int32_t), hipMemcpyDeviceToHost,
-                            m->stream));
-  FS_HIP_TRY(hipStreamSynchronize(m->stream));
-  if (m->hdr_h[2] != 0) {
+  m->hdr_fresh = false;
+  if (m->err_left) {
+    // clear the device error word left by a previous call
     const int32_t zero = 0;
+    FS_HIP_TRY(hipStreamSynchronize(m->stream));
     FS_HIP_TRY(hipMemcpy(m->hdr + 2, &zero, sizeof(zero), hipMemcpyHostToDevice));
+    m->err_left = false;
   }
   int st = FS_OK;
-  for (long long i = 0; i < iterations && st == FS_OK; i++) {
+  for (long long i = 0; i < iterations && st == FS_OK;) {
+    int took = 0;
     m->steps_in_call = i;
-    st = step_once(m);
+    st = advance(m, iterations - i, &took);
+    i += took;
   }
   const int fst = finish(m);
   if (st == FS_OK) st = fst;
-  const int sst = split_tile_time(m);
-  if (st == FS_OK) st = sst;
-  for (int i = 0; i < 6; i++) {
-    const double ms = m->stage_ms[FS_T_RECEIVERS + i];
-    const uint64_t whole = static_cast<uint64_t>(ms * 1000.0);
-    m->timer_us[FS_T_RECEIVERS + i] += whole;
-    m->stage_ms[FS_T_RECEIVERS + i] = ms - static_cast<double>(whole) / 1000.0;
-  }
+  if (st != FS_OK) m->err_left = true;
   m->timer_us[FS_T_OVERALL] += static_cast<uint64_t>(
       std::chrono::duration_cast<std::chrono::microseconds>(std::chrono::steady_clock::now() - t0)
           .count());
@@ -1071,6 +1183,7 @@ int check_model(fs_model *m) {
 // Rebuild the stack and donor masks of the last step if it took the tile path.
 int ensure_order(fs_model *m) {
   if (m->order_current || !m->have_step) return FS_OK;
+  m->err_left = true;   // until the next call has looked
   FS_HIP_TRY(hipStreamSynchronize(m->stream));
   FS_TRY(build_order(m, nullptr));
   FS_HIP_TRY(hipStreamSynchronize(m->stream));
@@ -1150,12 +1263,14 @@ int fs_set_h(fs_model *m, const double *in, size_t count) {
 
 int fs_get_timers(fs_model *m, uint64_t us[FS_NUM_TIMERS]) {
   if (!m || !us) return FS_ERR_INVALID_ARGUMENT;
+  FS_TRY(fold_timers(m));
   for (int i = 0; i < FS_NUM_TIMERS; i++) us[i] = m->timer_us[i];
   return FS_OK;
 }
 
 int fs_reset_timers(fs_model *m) {
   if (!m) return FS_ERR_INVALID_ARGUMENT;
+  FS_TRY(fold_timers(m));
   for (int i = 0; i < FS_NUM_TIMERS; i++) {
     m->timer_us[i] = 0;
     m->stage_ms[i] = 0;

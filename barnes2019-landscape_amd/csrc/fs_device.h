@@ -29,7 +29,16 @@ constexpr int kSmallBlock = 1024;
 constexpr int kSmallItems = 4;
 constexpr int kSmallLevel = kSmallBlock * kSmallItems;  // one-workgroup levels
 constexpr int kNewtonCap = 100;
-constexpr int kHdrInts = 4;            // maxdepth, n_unfinished, err, spare
+// Tile-path steps are launched in batches of up to kMaxBatch without a host
+// round trip; each step reports into a slot of its own.
+constexpr int kMaxBatch = 32;
+constexpr int kSlotOver = 0;           // tiles deeper than the halo: the step was not taken
+constexpr int kSlotDeepest = 1;        // deepest level (32-cell halo)
+constexpr int kSlotStop = 2;           // the step was not reached
+constexpr int kSlotInts = 4;
+constexpr int kHdrSlots = 4;
+// header: maxdepth, n_unfinished, err, spare; the batch's slots
+constexpr int kHdrInts = kHdrSlots + kMaxBatch * kSlotInts;
 constexpr int kHdrCounts = 1024;       // level counts fetched with the header
 // After the level counts: one "cells still unfinished" flag per pointer-
 // jumping pass, so the passes after the last needed one return at once.
@@ -171,12 +180,16 @@ __device__ uint32_t lookback(uint64_t *status, uint32_t tile, uint32_t epoch,
 // ---------------------------------------------------------------------------
 // kernels
 // ---------------------------------------------------------------------------
+// Opens a slot for another attempt of its step.
+__global__ void k_slot_reset(int32_t *slot) {
+  if (threadIdx.x < kSlotInts) slot[threadIdx.x] = 0;
+}
+
 __global__ void k_fill_counts(int32_t *hdr, int n_counts) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i == 0) {
     hdr[0] = 0;   // maxdepth
     hdr[1] = 0;   // n_unfinished
-    hdr[3] = 0;   // tiles whose levels exceed the tile halo
   }
   if (i < n_counts) hdr[kHdrInts + i] = 0;
   if (i <= kJumpPasses) hdr[kHdrJump + i] = 0;
@@ -285,19 +298,19 @@ __device__ __forceinline__ void receivers_strips(const double *__restrict__ h,
 // included); four rows read 1.5 rows per row decided (241 us at 10000^2),
 // sixteen leave too few waves (12.1 at 1000^2).  Bound by VALU issue at the
 // largest sizes (1.04 GB in 0.22 ms).
-// Also clears the header words the tile path's accumulation reports into
-// (hdr[0], hdr[1], hdr[3]; as k_fill_counts with no level counts).
+// On the tile path it also opens its step's slot.  prev is the slot of the
+// batch's previous step (null for its first): when that step was not taken, a
+// solve failed, or its drainage was no deeper than `shallow` levels (the
+// smaller halo fits again; -1: no such limit), this step is not taken either,
+// and nothing is written but the slot.
 constexpr int kRecvShort = 6;
 __global__ __launch_bounds__(256) void k_receivers(const double *__restrict__ h,
                                                    uint8_t *__restrict__ rcv, int W, int H,
                                                    double d_card, double d_diag,
-                                                   int32_t *__restrict__ hdr) {
+                                                   const int32_t *__restrict__ hdr,
+                                                   const int32_t *prev, int32_t *slot,
+                                                   int shallow) {
   constexpr int ROWS = kRecvShort;
-  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
-    hdr[0] = 0;
-    hdr[1] = 0;
-    hdr[3] = 0;
-  }
   const int x = blockIdx.x * kWave + static_cast<int>(threadIdx.x % kWave) + 2;
   const int group = __builtin_amdgcn_readfirstlane(
       (blockIdx.z * gridDim.y + blockIdx.y) * (256 / kWave) + threadIdx.x / kWave);
@@ -311,6 +324,14 @@ __global__ __launch_bounds__(256) void k_receivers(const double *__restrict__ h,
   for (int k = 0; k < ROWS + 2; k++)   // past the grid's last row: that row again
     load_cols(row_rsrc(h + static_cast<size_t>(min(y0 - 1 + k, H - 1)) * W, rowb), xo, l[k], c[k],
               r[k]);
+  const bool stop = prev != nullptr && (prev[kSlotOver] != 0 || prev[kSlotStop] != 0 ||
+                                        hdr[2] != 0 || prev[kSlotDeepest] <= shallow);
+  if (slot != nullptr && x == 2 && group == 0) {   // one thread of the grid
+    slot[kSlotOver] = 0;
+    slot[kSlotDeepest] = 0;
+    slot[kSlotStop] = stop ? 1 : 0;
+  }
+  if (stop) return;
 #pragma unroll
   for (int k = 0; k < ROWS; k++) {
     if (y0 + k >= H - 2) break;

@@ -77,7 +77,8 @@ __device__ __forceinline__ int region_offset(int r) {
 // adds 1 to each cell it passes, itself included, so a cell's count is the
 // number of region cells draining through it -- its whole upstream area when
 // every level is at most kHalo.  A tile cell deeper than that (or whose chain
-// leaves the region) raises hdr[3]; the host then runs the level path.
+// leaves the region) raises the step's slot; a larger halo, the tile graph or
+// the level path then takes the step.
 // Halo cells the erosion pass solves per tile at most: those on the receiver
 // chains of the tile's cells (with a 16-cell halo: mean 60-66, at most 92 per
 // tile of 5120 over 120 steps at the benchmark preset).
@@ -546,17 +547,18 @@ template <bool kTimed, int BLOCK = kAccBlock>
 __global__ __launch_bounds__(BLOCK) void k_tile_acc(const uint8_t *__restrict__ rcv,
                                                         uint32_t *__restrict__ cnt,
                                                         uint8_t *__restrict__ lvl,
-                                                        TilePlan *__restrict__ plan, int32_t *hdr,
+                                                        TilePlan *__restrict__ plan, int32_t *slot,
                                                         int W, int H, int tiles_x, int ntiles,
                                                         unsigned long long *phase) {
   __shared__ AccShared sh;
+  if (slot[kSlotStop] != 0) return;   // the batch ended before this step
   const int t = xcd_tile(blockIdx.x, ntiles);
-  // with the deep halo, hdr[0] (cleared by k_fill_counts) receives the
-  // deepest tile-cell level, so the host can step back to the 16-cell halo
+  // with the deep halo, the slot receives the deepest tile-cell level, so
+  // the next step can go back to the 16-cell halo
   const int over = tile_acc_body<BLOCK>(sh, rcv, cnt, lvl, plan + t, W, H, t, tiles_x, nullptr,
-                                            kHalo > 16 ? hdr : nullptr,
+                                            kHalo > 16 ? slot + kSlotDeepest : nullptr,
                                             kTimed ? phase : nullptr);
-  if (threadIdx.x == 0 && over) atomicAdd(&hdr[3], 1);
+  if (threadIdx.x == 0 && over) atomicAdd(&slot[kSlotOver], 1);
 }
 
 // Pass 2: uplift and erosion (AddUplift RB:285-296, Erode RB:306-328) of the
@@ -810,12 +812,13 @@ __global__ __launch_bounds__(kEroBlock) void k_tile_erode(
     const double *__restrict__ h_old, double *__restrict__ h_new,
     const TilePlan *__restrict__ plan, const uint8_t *__restrict__ lvl,
     const uint32_t *__restrict__ cnt, const double *__restrict__ ftab, int W, int H,
-    int tiles_x, int ntiles, ErodeConst k, int32_t *hdr, unsigned long long *phase) {
+    int tiles_x, int ntiles, ErodeConst k, int32_t *hdr, const int32_t *slot,
+    unsigned long long *phase) {
   __shared__ EroShared sh;
   // launched right behind the accumulation, before the host has read its
-  // outcome: when a tile was too deep (hdr[3], the plans are incomplete)
-  // the whole grid does nothing
-  if (hdr[3] != 0) return;
+  // outcome: when a tile was too deep (the plans are incomplete) or the
+  // batch ended before this step, the whole grid does nothing
+  if (slot[kSlotOver] != 0 || slot[kSlotStop] != 0) return;
   const int t = xcd_tile(blockIdx.x, ntiles);
   tile_erode_body<NMODE>(sh, h_old, h_new, plan + t, lvl, cnt, ftab, W, H, t, tiles_x, k, hdr,
                          kTimed ? phase : nullptr);
