@@ -55,176 +55,395 @@ __device__ __forceinline__ f32x4 mfma16(uint4 a, uint4 b, f32x4 c) {
 // ---------------------------------------------------------------------------
 // 3x3 convolution, stride 1, zero padding, as an implicit GEMM:
 //   out[p][n] = bias[n] + sum_{t, c} in[p + off_t][c] * wt[t][n][c]
-// M = pixels (64 per workgroup, 16 per wave), N = NT*16 outputs per
-// workgroup, K = 9 taps x cin in 32-channel steps.  MFMA operand A is the
-// input patch (row = pixel lane%16, 8 channels per lane group lane/16),
-// operand B the weights (column = output lane%16), D[4*(lane/16)+i][lane%16].
-// Pixels at or beyond M (the last workgroup's tail) read zeros and store
-// nothing.  Needs nout % (NT*16) == 0 and cin % 8 == 0.
+// A wave computes 16 columns x R rows x 32 outputs of one image on
+// v_mfma_f32_16x16x32_bf16: operand A the weights (row = output), operand B
+// the pixels (column = pixel lane%16, 8 channels per lane group lane/16), so a
+// lane ends with 8 consecutive outputs of one pixel (one 16-byte store).
+//
+// Per step of 32 input channels the wave holds its 9 taps' weights in
+// registers and walks down the R + 2 input rows: a row is loaded once (16
+// bytes per lane, straight from memory: no staging), its two column shifts
+// are lane shifts within the 16 lanes of a row (DPP; the edge pixel comes from
+// a second load that only lanes 0 and 15 take), and it feeds three output
+// rows.  That is 9 * 2 * R MFMAs for R + 2 row loads and 18 weight reads; the
+// kernel it replaces read two operands from LDS per MFMA pair and was bound by
+// LDS (9 * 6 reads for 72 MFMAs per wave).  Row p of the next step (or of the
+// wave's next tile) is requested as soon as row p of this one is used.
+//
+// The upsampled and concatenated decoder inputs are read where they lie, and
+// the pooling, the ReLU gradient and the gradient of the upsampling happen on
+// the finished tile, so none of them is a pass over memory of its own.
+// Ranking 256 candidates at 256 x 256: 12.75 -> 7.43 ms (391 -> 672 TFLOP/s);
+// the widest layers run at 820 to 990 TFLOP/s, the 32-channel layers of the
+// top level at 3.4 TB/s, bound by memory.
+//
+// Each accumulator adds its taps in order 0..8 within a step and the
+// steps in order, so the sums are those of a plain loop over (channel step,
+// tap), bit for bit, at every R.  kTapOuter (levels smaller than 8 x 16,
+// few and latency-bound): the loop over (tap, channel step).
 // ---------------------------------------------------------------------------
-template <int NT>
-__global__ __launch_bounds__(256) void k_conv3x3(const uint16_t *__restrict__ in, int cin,
-                                                 const uint16_t *__restrict__ wt,
-                                                 const float *__restrict__ bias,
-                                                 uint16_t *__restrict__ out, int nout, int H,
-                                                 int W, int relu, long M) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int g = lane >> 4, r = lane & 15;
-  const long m0 = static_cast<long>(blockIdx.x) * 64 + wave * 16;
-  const int n0 = blockIdx.y * (NT * 16);
-  const long p = m0 + r;
-  const int x = static_cast<int>(p % W);
-  const long q = p / W;
-  const int y = static_cast<int>(q % H);
-  const long b = q / H;
-  f32x4 acc[NT];
+constexpr int kNB = 32;            // outputs per wave
+constexpr int kKC = 32;            // input channels per step
+constexpr int kWaves = 4;          // waves per workgroup
+constexpr int kWFrags = 9 * (kNB / 16);
+constexpr int kRsrc = 0x00020000;  // raw (unformatted) buffer, gfx9
+constexpr uint32_t kOob = 0x80000000u;   // beyond every row: loads give zero
+
+// The input: channels [0, ca) from a -- at half the resolution when up (a 2x
+// nearest upsampling) -- and then cb channels from b.
+struct ConvSrc {
+  const uint16_t *a, *b;
+  int ca, cb, up;
+};
+// The output.  Outputs [0, c1) (c1 = 0 but for the gradient of a
+// concatenation) are summed over 2 x 2 pixels into lo, the others go to out;
+// mask / lo_mask: zero where that tensor is not positive (ReLU gradient);
+// pool: also the 2 x 2 averages of out.
+struct ConvDst {
+  uint16_t *out, *pool, *lo;
+  const uint16_t *mask, *lo_mask;
+  int c1;
+};
+
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ u32x4 load_px(const char *row, int bytes, uint32_t off) {
+  return __builtin_amdgcn_raw_buffer_load_b128(
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(row), 0, bytes, kRsrc),
+      static_cast<int>(off), 0, 0);
+}
+// lane r's value from lane r-1 / r+1 of its 16; lanes 0 / 15 take edge's own
+__device__ __forceinline__ u32x4 from_left(u32x4 v, u32x4 edge) {
+  u32x4 o;
 #pragma unroll
-  for (int nt = 0; nt < NT; nt++) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int t = 0; t < 9; t++) {
-    const int yy = y + t / 3 - 1, xx = x + t % 3 - 1;
-    const bool ok = p < M && yy >= 0 && yy < H && xx >= 0 && xx < W;
-    const uint16_t *src = in + ((b * H + (ok ? yy : 0)) * W + (ok ? xx : 0)) * cin;
-    const uint16_t *wrow = wt + (static_cast<long>(t) * nout + n0 + r) * cin;
-    for (int c0 = 0; c0 < cin; c0 += 32) {
-      const int c = c0 + 8 * g;
-      const bool cok = c < cin;
-      uint4 av = make_uint4(0u, 0u, 0u, 0u);
-      if (ok && cok) av = *reinterpret_cast<const uint4 *>(src + c);
+  for (int k = 0; k < 4; k++)
+    o[k] = __builtin_amdgcn_update_dpp(edge[k], v[k], 0x111, 0xF, 0xF, false);
+  return o;
+}
+__device__ __forceinline__ u32x4 from_right(u32x4 v, u32x4 edge) {
+  u32x4 o;
 #pragma unroll
-      for (int nt = 0; nt < NT; nt++) {
-        uint4 bv = make_uint4(0u, 0u, 0u, 0u);
-        if (cok) bv = *reinterpret_cast<const uint4 *>(wrow + static_cast<long>(nt) * 16 * cin + c);
-        acc[nt] = mfma16(av, bv, acc[nt]);
-      }
-    }
+  for (int k = 0; k < 4; k++)
+    o[k] = __builtin_amdgcn_update_dpp(edge[k], v[k], 0x101, 0xF, 0xF, false);
+  return o;
+}
+__device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
+                                                 __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+// two floats to bf16 (round to nearest even), low half first
+__device__ __forceinline__ uint32_t pack_bf(float lo, float hi) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  const bf16x2 v = {static_cast<__bf16>(lo), static_cast<__bf16>(hi)};
+  return __builtin_bit_cast(uint32_t, v);
+}
+// halves of g where the same half of y is positive, zero elsewhere
+__device__ __forceinline__ uint32_t relu_mask(uint32_t g, uint32_t y) {
+  const uint32_t lo = y & 0xFFFFu, hi = y >> 16;
+  return ((lo != 0 && lo < 0x8000u) ? (g & 0xFFFFu) : 0u) |
+         ((hi != 0 && hi < 0x8000u) ? (g & 0xFFFF0000u) : 0u);
+}
+__device__ __forceinline__ float bf_lo(uint32_t v) { return __uint_as_float(v << 16); }
+__device__ __forceinline__ float bf_hi(uint32_t v) { return __uint_as_float(v & 0xFFFF0000u); }
+// sum of a 2 x 2 pixel block (this lane and the next, two rows), in the order
+// (0,0), (0,1), (1,0), (1,1), times scale; right in the even lanes
+__device__ __forceinline__ u32x4 block2x2(u32x4 r0, u32x4 r1, float scale) {
+  u32x4 o;
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const uint32_t n0 = __builtin_amdgcn_mov_dpp(r0[k], 0xB1, 0xF, 0xF, true);
+    const uint32_t n1 = __builtin_amdgcn_mov_dpp(r1[k], 0xB1, 0xF, 0xF, true);
+    const float l = 0.f + bf_lo(r0[k]) + bf_lo(n0) + bf_lo(r1[k]) + bf_lo(n1);
+    const float h = 0.f + bf_hi(r0[k]) + bf_hi(n0) + bf_hi(r1[k]) + bf_hi(n1);
+    o[k] = pack_bf(scale * l, scale * h);
   }
+  return o;
+}
+
+// Position of a wave's tile: image, first row and column.
+struct TileAt {
+  long b;
+  int y0, x0;
+  bool valid;
+};
+template <int R>
+__device__ __forceinline__ TileAt tile_at(int tile, int ntiles, int tiles_x, int tiles_y) {
+  TileAt t;
+  t.valid = tile < ntiles;
+  const int q = t.valid ? tile : 0;
+  const int row = q / tiles_x;
+  t.x0 = (q - row * tiles_x) * 16;
+  t.b = row / tiles_y;
+  t.y0 = (row % tiles_y) * R;
+  return t;
+}
+
+// Bias, ReLU, rounding and the stores of a finished tile: acc[y][nt][i] is
+// output n0 + 8 * (lane / 16) + 4 * nt + i of pixel (t.y0 + y, t.x0 + lane % 16).
+template <int R>
+__device__ __forceinline__ void store_tile(const f32x4 (&acc)[R][2], const TileAt &t,
+                                           const ConvDst &dst, const float *bias, int relu,
+                                           int n0, int nout, int H, int W) {
+  if (!t.valid) return;
+  const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
+  float bb[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (bias) {
 #pragma unroll
-  for (int nt = 0; nt < NT; nt++) {
-    const int n = n0 + nt * 16 + r;
-    const float bb = bias ? bias[n] : 0.f;
+    for (int k = 0; k < 8; k++) bb[k] = bias[n0 + 8 * g + k];
+  }
+  const bool to_lo = n0 < dst.c1;                 // uniform
+  const int C = nout - dst.c1, n = n0 - dst.c1 + 8 * g;
+  const int xx = t.x0 + r;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      float v = acc[nt][i] + bb;
-      if (relu) v = fmaxf(v, 0.f);
-      if (m0 + 4 * g + i < M) out[(m0 + 4 * g + i) * nout + n] = f2bf(v);
+  for (int y = 0; y < R; y += 2) {
+    u32x4 v[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      float f[8];
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        f[k] = acc[y + h][k >> 2][k & 3] + bb[k];
+        if (relu) f[k] = fmaxf(f[k], 0.f);
+      }
+#pragma unroll
+      for (int k = 0; k < 4; k++) v[h][k] = pack_bf(f[2 * k], f[2 * k + 1]);
+    }
+    if (t.y0 + y >= H) break;                     // H is even
+    const long px = (t.b * H + t.y0 + y) * W + xx;
+    const long half = ((t.b * (H >> 1)) + ((t.y0 + y) >> 1)) * (W >> 1) + (xx >> 1);
+    if (to_lo) {
+      u32x4 s = block2x2(v[0], v[1], 1.f);
+      if (xx < W && (r & 1) == 0) {
+        const long at = half * dst.c1 + n0 + 8 * g;
+        if (dst.lo_mask) {
+          const u32x4 m = *reinterpret_cast<const u32x4 *>(dst.lo_mask + at);
+#pragma unroll
+          for (int k = 0; k < 4; k++) s[k] = relu_mask(s[k], m[k]);
+        }
+        *reinterpret_cast<u32x4 *>(dst.lo + at) = s;
+      }
+      continue;
+    }
+    if (dst.pool) {
+      const u32x4 s = block2x2(v[0], v[1], 0.25f);
+      if (xx < W && (r & 1) == 0) *reinterpret_cast<u32x4 *>(dst.pool + half * C + n) = s;
+    }
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      if (xx >= W) continue;
+      const long at = (px + static_cast<long>(h) * W) * C + n;
+      if (dst.mask) {
+        const u32x4 m = *reinterpret_cast<const u32x4 *>(dst.mask + at);
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[h][k] = relu_mask(v[h][k], m[k]);
+      }
+      *reinterpret_cast<u32x4 *>(dst.out + at) = v[h];
     }
   }
 }
 
-// ---------------------------------------------------------------------------
-// The same convolution with operands staged in LDS: a workgroup computes an
-// 8 x 16 pixel tile (one image) x NB outputs.  For each 32-channel step the
-// 10 x 18 input patch (tile + one-pixel halo, zero padded) and the 9 taps'
-// weights go to LDS once and every tap's MFMA operands are read from there,
-// so each input value is fetched once per tile instead of once per tap and
-// wave.  Wave w owns tile rows 2w and 2w+1 (two 16-pixel MFMA rows) and all
-// NB outputs.  Rows are padded to 40 bf16 (80 bytes) against bank conflicts.
-// Needs nout % NB == 0 and cin % 8 == 0.
-// ---------------------------------------------------------------------------
-constexpr int kTPH = 8, kTPW = 16;               // pixel tile
-constexpr int kPatchH = kTPH + 2, kPatchW = kTPW + 2;
-constexpr int kKC = 32;                           // input channels per step
-constexpr int kCS = kKC + 8;                      // padded channel stride in LDS
+// output of MFMA row m in weight tile nt (see store_tile)
+__device__ __forceinline__ int frag_out(int m, int nt) { return 8 * (m >> 2) + 4 * nt + (m & 3); }
 
-template <int NB>
-__global__ __launch_bounds__(256) void k_conv3x3_t(const uint16_t *__restrict__ in, int cin,
-                                                   const uint16_t *__restrict__ wt,
-                                                   const float *__restrict__ bias,
-                                                   uint16_t *__restrict__ out, int nout, int H,
-                                                   int W, int relu, int tiles_y) {
-  constexpr int NT = NB / 16;
-  __shared__ __attribute__((aligned(16))) uint16_t patch[kPatchH * kPatchW * kCS];
-  __shared__ __attribute__((aligned(16))) uint16_t ws[9 * NB * kCS];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// A workgroup keeps one block of 32 outputs and takes groups of kWaves tiles
+// in turn; each XCD gets one contiguous run of groups (tiles that share input
+// rows share an L2) for every block of outputs.  gridDim.x is a multiple of
+// 8 * nout / 32.
+template <int R>
+__global__ __launch_bounds__(64 * kWaves, 2) void k_conv(ConvSrc src,
+                                                         const uint16_t *__restrict__ wt,
+                                                         const float *__restrict__ bias, int relu,
+                                                         ConvDst dst, int nout, int H, int W,
+                                                         int tiles_x, int tiles_y, int ntiles,
+                                                         int groups) {
+  // the step's weights in fragment order: [buffer][frag][lane]
+  __shared__ u32x4 ws[2][kWFrags * 64];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, r = lane & 15;
-  const int x0 = blockIdx.x * kTPW;
-  const int ty = blockIdx.y % tiles_y;
-  const long b = blockIdx.y / tiles_y;
-  const int y0 = ty * kTPH;
-  const int n0 = blockIdx.z * NB;
-  f32x4 acc[2][NT];
+  const int nblk = nout / kNB;
+  const int xcd = blockIdx.x & 7, q = blockIdx.x >> 3;
+  const int n0 = (q % nblk) * kNB, per = gridDim.x / (8 * nblk);
+  const int g1 = static_cast<int>(static_cast<long>(groups) * (xcd + 1) / 8);
+  const int first = static_cast<int>(static_cast<long>(groups) * xcd / 8) + q / nblk;
+  if (first >= g1) return;
+  const int cin = src.ca + src.cb;
+  const int csteps = (cin + kKC - 1) / kKC;
+
+  // ---- weights: global -> registers -> LDS, one step ahead ----
+  constexpr int kWVec = 9 * kNB * 4;               // 16-byte vectors per step
+  constexpr int kWPer = (kWVec + 64 * kWaves - 1) / (64 * kWaves);
+  u32x4 wreg[kWPer];
+  auto fetch_weights = [&](int c0) {
 #pragma unroll
-  for (int mt = 0; mt < 2; mt++)
-#pragma unroll
-    for (int nt = 0; nt < NT; nt++) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // the next step's patch and weights are loaded into registers while the
-  // current step is computed from LDS
-  constexpr int kPV = (kPatchH * kPatchW * 4 + 255) / 256;
-  constexpr int kWV = (9 * NB * 4 + 255) / 256;
-  uint4 pv[kPV], wv[kWV];
-  auto load = [&](int c0) {
-#pragma unroll
-    for (int k = 0; k < kPV; k++) {
-      const int v = k * 256 + threadIdx.x;
-      const int pix = v >> 2, c8 = v & 3;
-      const int py = pix / kPatchW, px = pix % kPatchW;
-      const int yy = y0 - 1 + py, xx = x0 - 1 + px;
-      const int c = c0 + 8 * c8;
-      pv[k] = make_uint4(0u, 0u, 0u, 0u);
-      if (v < kPatchH * kPatchW * 4 && yy >= 0 && yy < H && xx >= 0 && xx < W && c < cin)
-        pv[k] = *reinterpret_cast<const uint4 *>(in + ((b * H + yy) * W + xx) * cin + c);
-    }
-#pragma unroll
-    for (int k = 0; k < kWV; k++) {
-      const int v = k * 256 + threadIdx.x;
-      const int row = v >> 2, c8 = v & 3;           // row = tap * NB + output
-      const int t = row / NB, o = row % NB;
-      const int c = c0 + 8 * c8;
-      wv[k] = make_uint4(0u, 0u, 0u, 0u);
-      if (v < 9 * NB * 4 && c < cin)
-        wv[k] = *reinterpret_cast<const uint4 *>(wt + (static_cast<long>(t) * nout + n0 + o) * cin + c);
+    for (int k = 0; k < kWPer; k++) {
+      const int v = k * 64 * kWaves + static_cast<int>(threadIdx.x);
+      const int row = v >> 2, c = c0 + 8 * (v & 3);
+      const int t = row / kNB, o = row % kNB;
+      wreg[k] = u32x4{0u, 0u, 0u, 0u};
+      if (v < kWVec && c < cin)
+        wreg[k] = *reinterpret_cast<const u32x4 *>(
+            wt + (static_cast<long>(t) * nout + n0 + o) * cin + c);
     }
   };
-  load(0);
-  for (int c0 = 0; c0 < cin; c0 += kKC) {
+  auto stage_weights = [&](int buf) {
 #pragma unroll
-    for (int k = 0; k < kPV; k++) {
-      const int v = k * 256 + threadIdx.x;
-      if (v < kPatchH * kPatchW * 4)
-        *reinterpret_cast<uint4 *>(&patch[(v >> 2) * kCS + 8 * (v & 3)]) = pv[k];
+    for (int k = 0; k < kWPer; k++) {
+      const int v = k * 64 * kWaves + static_cast<int>(threadIdx.x);
+      const int row = v >> 2, t = row / kNB, o = row % kNB;
+      const int nt = (o >> 2) & 1, m = 4 * (o >> 3) + (o & 3);   // frag_out(m, nt) == o
+      if (v < kWVec) ws[buf][(2 * t + nt) * 64 + 16 * (v & 3) + m] = wreg[k];
     }
+  };
+
+  // ---- input rows ----
+  struct Unit {            // a tile's step of 32 channels
+    const char *base;      // the image's first row in the step's source
+    int rowbytes, up, y0;
+    bool valid;
+    uint32_t oc, oe;       // the lane's offsets in a row: its pixel, the edge pixel
+  };
+  auto make_unit = [&](int grp, int c0) {
+    Unit u;
+    const TileAt t = tile_at<R>(grp * kWaves + wave, ntiles, tiles_x, tiles_y);
+    const bool first_src = c0 < src.ca;
+    const int C = first_src ? src.ca : src.cb, c = first_src ? c0 : c0 - src.ca;
+    u.up = first_src ? src.up : 0;
+    u.rowbytes = (W >> u.up) * C * 2;
+    u.base = reinterpret_cast<const char *>(first_src ? src.a : src.b) +
+             t.b * (H >> u.up) * static_cast<long>(u.rowbytes);
+    u.y0 = t.y0;
+    u.valid = t.valid && grp < g1;
+    const bool cok = c + 8 * g < C;
+    const int xc = (t.x0 + r) >> u.up, xe = (r == 0 ? t.x0 - 1 : t.x0 + 16) >> u.up;
+    u.oc = cok ? static_cast<uint32_t>(xc * C + c + 8 * g) * 2u : kOob;
+    u.oe = cok && (r == 0 || r == 15) ? static_cast<uint32_t>(xe * C + c + 8 * g) * 2u : kOob;
+    return u;
+  };
+  // rows in flight: row p sits in slot p % kRing
+  constexpr int kRing = R == 8 ? 5 : R + 2;
+  static_assert((R + 2) % kRing == 0, "slots line up from step to step");
+  u32x4 pc[kRing], pe[kRing];
+  auto load_row = [&](const Unit &u, int p) {
+    const int yy = u.y0 - 1 + p;
+    const bool ok = u.valid && static_cast<unsigned>(yy) < static_cast<unsigned>(H);
+    const char *row = u.base + static_cast<long>(ok ? yy >> u.up : 0) * u.rowbytes;
+    pc[p % kRing] = load_px(row, ok ? u.rowbytes : 0, u.oc);
+    pe[p % kRing] = load_px(row, ok ? u.rowbytes : 0, u.oe);
+  };
+
+  f32x4 acc[R][2];
 #pragma unroll
-    for (int k = 0; k < kWV; k++) {
-      const int v = k * 256 + threadIdx.x;
-      if (v < 9 * NB * 4) *reinterpret_cast<uint4 *>(&ws[(v >> 2) * kCS + 8 * (v & 3)]) = wv[k];
-    }
-    __syncthreads();
-    if (c0 + kKC < cin) load(c0 + kKC);
+  for (int y = 0; y < R; y++) acc[y][0] = acc[y][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  fetch_weights(0);
+  Unit cur = make_unit(first, 0);
 #pragma unroll
-    for (int t = 0; t < 9; t++) {
-      const int dy = t / 3, dx = t % 3;
-      uint4 av[2];
+  for (int p = 0; p < kRing; p++) load_row(cur, p);
+  stage_weights(0);
+  __syncthreads();
+  u32x4 w[9][2];
 #pragma unroll
-      for (int mt = 0; mt < 2; mt++) {
-        const int pr = 2 * wave + mt;
-        av[mt] = *reinterpret_cast<const uint4 *>(&patch[((pr + dy) * kPatchW + r + dx) * kCS + 8 * g]);
+  for (int f = 0; f < kWFrags; f++) w[f >> 1][f & 1] = ws[0][f * 64 + lane];
+  int buf = 0;
+  for (int grp = first; grp < g1; grp += per) {
+    for (int cs = 0; cs < csteps; cs++) {
+      const bool last = cs + 1 == csteps;
+      const bool more = !last || grp + per < g1;
+      const int cnext = last ? 0 : (cs + 1) * kKC;
+      const Unit next = make_unit(last ? grp + per : grp, cnext);
+      if (csteps > 1 && more) fetch_weights(cnext);
+#pragma unroll
+      for (int p = 0; p < R + 2; p++) {
+        const u32x4 c = pc[p % kRing], e = pe[p % kRing];
+        const u32x4 f[3] = {from_left(c, e), c, from_right(c, e)};
+        if (p + kRing < R + 2) load_row(cur, p + kRing);
+        else load_row(next, p + kRing - (R + 2));
+#pragma unroll
+        for (int dx = 0; dx < 3; dx++)
+#pragma unroll
+          for (int dy = 0; dy < 3; dy++) {
+            const int y = p - dy;
+            if (y < 0 || y >= R) continue;
+#pragma unroll
+            for (int nt = 0; nt < 2; nt++)
+              acc[y][nt] = mfma16(w[3 * dy + dx][nt], f[dx], acc[y][nt]);
+          }
       }
+      cur = next;
+      if (csteps > 1 && more) {
+        // the other buffer's readers passed the previous barrier; only LDS is
+        // waited for, the rows requested above stay in flight
+        buf ^= 1;
+        stage_weights(buf);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
-      for (int nt = 0; nt < NT; nt++) {
-        const uint4 bv = *reinterpret_cast<const uint4 *>(&ws[(t * NB + 16 * nt + r) * kCS + 8 * g]);
-#pragma unroll
-        for (int mt = 0; mt < 2; mt++) acc[mt][nt] = mfma16(av[mt], bv, acc[mt][nt]);
+        for (int f = 0; f < kWFrags; f++) w[f >> 1][f & 1] = ws[buf][f * 64 + lane];
       }
     }
-    __syncthreads();
+    store_tile<R>(acc, tile_at<R>(grp * kWaves + wave, ntiles, tiles_x, tiles_y), dst, bias, relu,
+                  n0, nout, H, W);
+#pragma unroll
+    for (int y = 0; y < R; y++) acc[y][0] = acc[y][1] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
+}
+
+// Levels smaller than 8 x 16: one wave per workgroup, 16 columns x 2 rows x 32
+// outputs, the loop over (tap, channel step) with kAhead iterations' operands
+// in flight.  cin is a multiple of 32.
+__global__ __launch_bounds__(64) void k_conv_small(ConvSrc src, const uint16_t *__restrict__ wt,
+                                                   const float *__restrict__ bias, int relu,
+                                                   ConvDst dst, int nout, int H, int W,
+                                                   int tiles_x, int tiles_y, int ntiles) {
+  constexpr int R = 2, kAhead = 9;
+  const int lane = threadIdx.x, g = lane >> 4, r = lane & 15;
+  const int n0 = blockIdx.y * kNB;
+  const TileAt t = tile_at<R>(blockIdx.x, ntiles, tiles_x, tiles_y);
+  const int cin = src.ca + src.cb, csteps = cin / kKC, steps = 9 * csteps;
+  u32x4 px[kAhead][R], wv[kAhead][2];
+  int lt = 0, lc = 0;    // tap and first channel of the next iteration to load
+  auto load = [&](int slot) {
+    const bool first_src = lc < src.ca, ok = lt < 9;
+    const int C = first_src ? src.ca : src.cb, c = first_src ? lc : lc - src.ca;
+    const int up = first_src ? src.up : 0;
+    const int rowbytes = (W >> up) * C * 2;
+    const char *base = reinterpret_cast<const char *>(first_src ? src.a : src.b) +
+                       t.b * (H >> up) * static_cast<long>(rowbytes);
+    const int tt = ok ? lt : 0;
+    const int x = t.x0 + r + tt % 3 - 1;
+    const uint32_t off = static_cast<uint32_t>((x >> up) * C + c + 8 * g) * 2u;
 #pragma unroll
-  for (int mt = 0; mt < 2; mt++) {
-    const int yy = y0 + 2 * wave + mt;
+    for (int y = 0; y < R; y++) {
+      const int yy = t.y0 + y + tt / 3 - 1;
+      const bool in = ok && static_cast<unsigned>(yy) < static_cast<unsigned>(H);
+      px[slot][y] = load_px(base + static_cast<long>(in ? yy >> up : 0) * rowbytes,
+                            in ? rowbytes : 0, off);
+    }
 #pragma unroll
-    for (int nt = 0; nt < NT; nt++) {
-      const int n = n0 + 16 * nt + r;
-      const float bb = bias ? bias[n] : 0.f;
+    for (int nt = 0; nt < 2; nt++)
+      wv[slot][nt] = *reinterpret_cast<const u32x4 *>(
+          wt + (static_cast<long>(tt) * nout + n0 + frag_out(r, nt)) * cin + lc + 8 * g);
+    lc += kKC;
+    if (lc >= cin) {
+      lc = 0;
+      lt++;
+    }
+  };
+  f32x4 acc[R][2];
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int xx = x0 + 4 * g + i;
-        if (yy >= H || xx >= W) continue;
-        float v = acc[mt][nt][i] + bb;
-        if (relu) v = fmaxf(v, 0.f);
-        out[((b * H + yy) * W + xx) * nout + n] = f2bf(v);
-      }
+  for (int y = 0; y < R; y++) acc[y][0] = acc[y][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int d = 0; d < kAhead; d++) load(d);
+  for (int s = 0; s < steps; s += kAhead) {   // steps is a multiple of kAhead
+#pragma unroll
+    for (int d = 0; d < kAhead; d++) {
+#pragma unroll
+      for (int nt = 0; nt < 2; nt++)
+#pragma unroll
+        for (int y = 0; y < R; y++) acc[y][nt] = mfma16(wv[d][nt], px[d][y], acc[y][nt]);
+      load(d);
     }
   }
+  store_tile<R>(acc, t, dst, bias, relu, n0, nout, H, W);
 }
 
 // ---------------------------------------------------------------------------
@@ -237,11 +456,11 @@ __global__ __launch_bounds__(256) void k_conv3x3_t(const uint16_t *__restrict__ 
 constexpr int kDwStride = 40;   // LDS row: 32 pixels + 8 pad (80 bytes)
 
 __global__ __launch_bounds__(256) void k_conv3x3_dw(const uint16_t *__restrict__ dz, int cout,
-                                                    const uint16_t *__restrict__ x, int cin,
-                                                    float *__restrict__ part, int H, int W,
-                                                    long chunk_pix, long M) {
+                                                    ConvSrc src, float *__restrict__ part, int H,
+                                                    int W, long chunk_pix, long M) {
   __shared__ __attribute__((aligned(16))) uint16_t As[64 * kDwStride];
   __shared__ __attribute__((aligned(16))) uint16_t Bs[64 * kDwStride];
+  const int cin = src.ca + src.cb;
   const int tiles_ci = (cin + 63) / 64;
   const int co0 = (blockIdx.x / tiles_ci) * 64, ci0 = (blockIdx.x % tiles_ci) * 64;
   const int t = blockIdx.y, chunk = blockIdx.z;
@@ -252,6 +471,9 @@ __global__ __launch_bounds__(256) void k_conv3x3_dw(const uint16_t *__restrict__
   const int rb = (wave >> 1) * 32, cb = (wave & 1) * 32;
   // loader: pixel lp = tid/8, channels 8*(tid%8) .. +7
   const int lp = threadIdx.x >> 3, lc = (threadIdx.x & 7) * 8;
+  const bool first_src = ci0 + lc < src.ca;
+  const int up = first_src ? src.up : 0, xC = first_src ? src.ca : src.cb;
+  const uint16_t *const x = first_src ? src.a + ci0 + lc : src.b + (ci0 + lc - src.ca);
   f32x4 acc[2][2];
 #pragma unroll
   for (int a = 0; a < 2; a++)
@@ -268,7 +490,8 @@ __global__ __launch_bounds__(256) void k_conv3x3_dw(const uint16_t *__restrict__
       const long pb = pq / H;
       const int yy = py + dy, xx = px + dx;
       if (ci0 + lc < cin && yy >= 0 && yy < H && xx >= 0 && xx < W)
-        xv = *reinterpret_cast<const uint4 *>(x + ((pb * H + yy) * W + xx) * cin + ci0 + lc);
+        xv = *reinterpret_cast<const uint4 *>(
+            x + ((pb * (H >> up) + (yy >> up)) * (W >> up) + (xx >> up)) * xC);
     }
     const uint16_t *zs = reinterpret_cast<const uint16_t *>(&zv);
     const uint16_t *xs = reinterpret_cast<const uint16_t *>(&xv);
@@ -349,9 +572,9 @@ __device__ __forceinline__ void transpose8(const uint4 (&v)[8], uint4 (&o)[8]) {
 
 template <int CB>
 __global__ __launch_bounds__(kDwThreads) void k_conv3x3_dw_t(
-    const uint16_t *__restrict__ dz, int cout, const uint16_t *__restrict__ x, int cin,
-    float *__restrict__ part, float *__restrict__ db, int H, int W, int tiles_img, int tiles_x,
-    long ntiles, int tiles_per_chunk, int ci_blocks) {
+    const uint16_t *__restrict__ dz, int cout, ConvSrc src, float *__restrict__ part,
+    float *__restrict__ db, int H, int W, int tiles_img, int tiles_x, long ntiles,
+    int tiles_per_chunk, int ci_blocks) {
   constexpr int NA = CB / 16;
   constexpr int kABlocks = (kDwTP / 8) * (CB / 8);
   static_assert(kABlocks <= kDwThreads, "one dz block per thread");
@@ -360,6 +583,12 @@ __global__ __launch_bounds__(kDwThreads) void k_conv3x3_dw_t(
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int g = lane >> 4, r = lane & 15;
   const int co0 = (blockIdx.x / ci_blocks) * CB, ci0 = (blockIdx.x % ci_blocks) * 32;
+  const int cin = src.ca + src.cb;
+  // the block's 32 inputs lie in one of the two sources (ca is a multiple of 32
+  // where there are two)
+  const bool first_src = ci0 < src.ca;
+  const int up = first_src ? src.up : 0, xC = first_src ? src.ca : src.cb;
+  const uint16_t *const x = first_src ? src.a + ci0 : src.b + (ci0 - src.ca);
   const long t0 = static_cast<long>(blockIdx.y) * tiles_per_chunk;
   const long t1 = min(ntiles, t0 + tiles_per_chunk);
   f32x4 acc[3][NA][2];
@@ -407,13 +636,15 @@ __global__ __launch_bounds__(kDwThreads) void k_conv3x3_dw_t(
       const int cg = blk & 3, h = (blk >> 2) & 1, pr = (blk >> 3) % kDwBR, dx = blk / (8 * kDwBR);
       const int yy = y0 - 1 + pr, xs = x0 - 1 + dx + 8 * h;
       const bool row_ok = yy >= 0 && yy < H && ci0 + 8 * cg < cin;
-      const uint16_t *src = x + ((b * H + (row_ok ? yy : 0)) * W) * cin + ci0 + 8 * cg;
+      const uint16_t *row =
+          x + (b * (H >> up) + (row_ok ? yy >> up : 0)) * static_cast<long>(W >> up) * xC + 8 * cg;
       uint4 v[8], o[8];
 #pragma unroll
       for (int i = 0; i < 8; i++) {
         const int xx = xs + i;
         v[i] = make_uint4(0u, 0u, 0u, 0u);
-        if (row_ok && xx >= 0 && xx < W) v[i] = *reinterpret_cast<const uint4 *>(src + static_cast<long>(xx) * cin);
+        if (row_ok && xx >= 0 && xx < W)
+          v[i] = *reinterpret_cast<const uint4 *>(row + static_cast<long>(xx >> up) * xC);
       }
       transpose8(v, o);
 #pragma unroll
@@ -520,58 +751,13 @@ __global__ __launch_bounds__(256) void k_bias_grad(const uint16_t *__restrict__ 
   for (int c = threadIdx.x; c < C; c += 256) atomicAdd(&db[c], red[c]);
 }
 
-// dz = dy where y > 0 (ReLU gradient from the stored output), 8 per thread
-__global__ __launch_bounds__(256) void k_relu_grad(const uint16_t *__restrict__ dy,
-                                                   const uint16_t *__restrict__ y,
-                                                   uint16_t *__restrict__ dz, long n8) {
-  for (long i = blockIdx.x * 256l + threadIdx.x; i < n8; i += gridDim.x * 256l) {
-    const uint4 g = reinterpret_cast<const uint4 *>(dy)[i];
-    const uint4 v = reinterpret_cast<const uint4 *>(y)[i];
-    const uint32_t gw[4] = {g.x, g.y, g.z, g.w}, vw[4] = {v.x, v.y, v.z, v.w};
-    uint32_t o[4];
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-      const uint32_t lo = vw[k] & 0xFFFFu, hi = vw[k] >> 16;
-      const bool plo = lo != 0 && !(lo & 0x8000u), phi = hi != 0 && !(hi & 0x8000u);
-      o[k] = (plo ? (gw[k] & 0xFFFFu) : 0u) | (phi ? (gw[k] & 0xFFFF0000u) : 0u);
-    }
-    reinterpret_cast<uint4 *>(dz)[i] = make_uint4(o[0], o[1], o[2], o[3]);
-  }
-}
-
-// 2x2 average pooling, NHWC, C % 8 == 0
-__global__ __launch_bounds__(256) void k_pool(const uint16_t *__restrict__ in,
-                                              uint16_t *__restrict__ out, int B, int H, int W,
-                                              int C) {
-  const int Ho = H / 2, Wo = W / 2, C8 = C / 8;
-  const long n = static_cast<long>(B) * Ho * Wo * C8;
-  for (long i = blockIdx.x * 256l + threadIdx.x; i < n; i += gridDim.x * 256l) {
-    const int c8 = static_cast<int>(i % C8);
-    const long q = i / C8;
-    const int xo = static_cast<int>(q % Wo);
-    const long q2 = q / Wo;
-    const int yo = static_cast<int>(q2 % Ho);
-    const long b = q2 / Ho;
-    float s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-    for (int d = 0; d < 4; d++) {
-      const long src = ((b * H + 2 * yo + d / 2) * W + 2 * xo + d % 2) * C + 8 * c8;
-      const uint4 v = *reinterpret_cast<const uint4 *>(in + src);
-      const uint16_t *h = reinterpret_cast<const uint16_t *>(&v);
-#pragma unroll
-      for (int k = 0; k < 8; k++) s[k] += bf2f(h[k]);
-    }
-    uint16_t o[8];
-#pragma unroll
-    for (int k = 0; k < 8; k++) o[k] = f2bf(0.25f * s[k]);
-    *reinterpret_cast<uint4 *>(out + q * C + 8 * c8) = *reinterpret_cast<const uint4 *>(o);
-  }
-}
-
-// gradient of the pooling: dx[b,y,x,c] (+)= dy[b,y/2,x/2,c] / 4
+// gradient of the pooling, added to the skip connection's:
+// dx[b,y,x,c] = dx[b,y,x,c] + dy[b,y/2,x/2,c] / 4 where act[b,y,x,c] > 0, else 0
+// (act: the pooled tensor, a ReLU's output)
 __global__ __launch_bounds__(256) void k_pool_grad(const uint16_t *__restrict__ dy,
-                                                   uint16_t *__restrict__ dx, int B, int H,
-                                                   int W, int C, int accumulate) {
+                                                   uint16_t *__restrict__ dx,
+                                                   const uint16_t *__restrict__ act, int B, int H,
+                                                   int W, int C) {
   const int C8 = C / 8;
   const long n = static_cast<long>(B) * H * W * C8;
   for (long i = blockIdx.x * 256l + threadIdx.x; i < n; i += gridDim.x * 256l) {
@@ -582,81 +768,15 @@ __global__ __launch_bounds__(256) void k_pool_grad(const uint16_t *__restrict__ 
     const int y = static_cast<int>(q2 % H);
     const long b = q2 / H;
     const long src = ((b * (H / 2) + y / 2) * (W / 2) + x / 2) * C + 8 * c8;
-    const uint4 v = *reinterpret_cast<const uint4 *>(dy + src);
-    const uint16_t *h = reinterpret_cast<const uint16_t *>(&v);
-    uint16_t *dst = dx + q * C + 8 * c8;
-    uint16_t o[8];
-    if (accumulate) {
-      const uint4 w = *reinterpret_cast<const uint4 *>(dst);
-      const uint16_t *e = reinterpret_cast<const uint16_t *>(&w);
+    const u32x4 v = *reinterpret_cast<const u32x4 *>(dy + src);
+    u32x4 *const dst = reinterpret_cast<u32x4 *>(dx + q * C + 8 * c8);
+    const u32x4 e = *dst, m = *reinterpret_cast<const u32x4 *>(act + q * C + 8 * c8);
+    u32x4 o;
 #pragma unroll
-      for (int k = 0; k < 8; k++) o[k] = f2bf(bf2f(e[k]) + 0.25f * bf2f(h[k]));
-    } else {
-#pragma unroll
-      for (int k = 0; k < 8; k++) o[k] = f2bf(0.25f * bf2f(h[k]));
-    }
-    *reinterpret_cast<uint4 *>(dst) = *reinterpret_cast<const uint4 *>(o);
-  }
-}
-
-// out[b,y,x] = [lo[b,y/2,x/2, 0:c1], skip[b,y,x, 0:c2]]
-__global__ __launch_bounds__(256) void k_upcat(const uint16_t *__restrict__ lo, int c1,
-                                               const uint16_t *__restrict__ skip, int c2,
-                                               uint16_t *__restrict__ out, int B, int H, int W) {
-  const int C = c1 + c2, C8 = C / 8;
-  const long n = static_cast<long>(B) * H * W * C8;
-  for (long i = blockIdx.x * 256l + threadIdx.x; i < n; i += gridDim.x * 256l) {
-    const int c = static_cast<int>(i % C8) * 8;
-    const long q = i / C8;
-    const int x = static_cast<int>(q % W);
-    const long q2 = q / W;
-    const int y = static_cast<int>(q2 % H);
-    const long b = q2 / H;
-    uint4 v;
-    if (c < c1) v = *reinterpret_cast<const uint4 *>(lo + ((b * (H / 2) + y / 2) * (W / 2) + x / 2) * c1 + c);
-    else v = *reinterpret_cast<const uint4 *>(skip + q * c2 + (c - c1));
-    *reinterpret_cast<uint4 *>(out + q * C + c) = v;
-  }
-}
-
-// gradient of k_upcat: dlo[b,Y,X,c] = sum of the 2x2 block's dout[.., c];
-// dskip[b,y,x,c] = dout[b,y,x,c1+c]
-__global__ __launch_bounds__(256) void k_upcat_grad(const uint16_t *__restrict__ dout, int c1,
-                                                    int c2, uint16_t *__restrict__ dlo,
-                                                    uint16_t *__restrict__ dskip, int B, int H,
-                                                    int W) {
-  const int C = c1 + c2;
-  const int Hl = H / 2, Wl = W / 2;
-  const long nlo = static_cast<long>(B) * Hl * Wl * (c1 / 8);
-  const long nsk = static_cast<long>(B) * H * W * (c2 / 8);
-  for (long i = blockIdx.x * 256l + threadIdx.x; i < nlo + nsk; i += gridDim.x * 256l) {
-    if (i < nlo) {
-      const int c = static_cast<int>(i % (c1 / 8)) * 8;
-      const long q = i / (c1 / 8);
-      const int X = static_cast<int>(q % Wl);
-      const long q2 = q / Wl;
-      const int Y = static_cast<int>(q2 % Hl);
-      const long b = q2 / Hl;
-      float s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-      for (int d = 0; d < 4; d++) {
-        const long src = ((b * H + 2 * Y + d / 2) * W + 2 * X + d % 2) * C + c;
-        const uint4 v = *reinterpret_cast<const uint4 *>(dout + src);
-        const uint16_t *h = reinterpret_cast<const uint16_t *>(&v);
-#pragma unroll
-        for (int k = 0; k < 8; k++) s[k] += bf2f(h[k]);
-      }
-      uint16_t o[8];
-#pragma unroll
-      for (int k = 0; k < 8; k++) o[k] = f2bf(s[k]);
-      *reinterpret_cast<uint4 *>(dlo + q * c1 + c) = *reinterpret_cast<const uint4 *>(o);
-    } else {
-      const long j = i - nlo;
-      const int c = static_cast<int>(j % (c2 / 8)) * 8;
-      const long q = j / (c2 / 8);
-      *reinterpret_cast<uint4 *>(dskip + q * c2 + c) =
-          *reinterpret_cast<const uint4 *>(dout + q * C + c1 + c);
-    }
+    for (int k = 0; k < 4; k++)
+      o[k] = relu_mask(pack_bf(bf_lo(e[k]) + 0.25f * bf_lo(v[k]), bf_hi(e[k]) + 0.25f * bf_hi(v[k])),
+                       m[k]);
+    *dst = o;
   }
 }
 
@@ -716,8 +836,8 @@ __global__ __launch_bounds__(256) void k_head(const uint16_t *__restrict__ f,
 }
 
 // loss = mean (yhat - t)^2 over M pixels; gy = 2 (yhat - t) / M; head
-// gradients; df[p][c] = gy[p] * hw[c].  acc[0] += loss, acc[1..32] += dhw,
-// acc[33] += dhb.
+// gradients; df[p][c] = gy[p] * hw[c] where f[p][c] > 0, else 0 (f is a ReLU's
+// output).  acc[0] += loss, acc[1..32] += dhw, acc[33] += dhb.
 __global__ __launch_bounds__(256) void k_head_grad(const uint16_t *__restrict__ f,
                                                    const float *__restrict__ hw,
                                                    const float *__restrict__ yhat,
@@ -744,7 +864,7 @@ __global__ __launch_bounds__(256) void k_head_grad(const uint16_t *__restrict__ 
 #pragma unroll
       for (int k = 0; k < 8; k++) {
         gw[8 * c8 + k] += gy * bf2f(h[k]);
-        o[k] = f2bf(gy * hw[8 * c8 + k]);
+        o[k] = h[k] != 0 && h[k] < 0x8000u ? f2bf(gy * hw[8 * c8 + k]) : 0;
       }
       *reinterpret_cast<uint4 *>(df + p * 32 + 8 * c8) = *reinterpret_cast<const uint4 *>(o);
     }
@@ -823,10 +943,11 @@ struct fs_unet {
   float *part = nullptr;
   size_t part_n = 0;
   // activations and their gradients
-  Tensor x0, e_a[kLevels], e[kLevels], p[kLevels - 1], u[kLevels - 1], d_a[kLevels - 1],
-      d[kLevels - 1];
-  Tensor ge_a[kLevels], ge[kLevels], gp[kLevels - 1], gu[kLevels - 1], gd_a[kLevels - 1],
-      gd[kLevels - 1], gz;   // gz: ReLU-masked gradient scratch (largest tensor)
+  Tensor x0, e_a[kLevels], e[kLevels], p[kLevels - 1], d_a[kLevels - 1], d[kLevels - 1];
+  // gradients of the convolutions' outputs before their ReLU; gp: of the
+  // pooled tensors
+  Tensor ge_a[kLevels], ge[kLevels], gp[kLevels - 1], gd_a[kLevels - 1], gd[kLevels - 1];
+  int ncu = 0;
   float *yhat = nullptr, *tgt = nullptr, *head_acc = nullptr, *terrain = nullptr,
         *params_in = nullptr;
   // resident training set
@@ -857,33 +978,52 @@ long pixels(const fs_unet *u, int level, int B) {
   return static_cast<long>(B) * (u->H >> level) * (u->W >> level);
 }
 
-// out = conv3x3(in) with weights wt [tap][nout][cin]: the LDS-tiled kernel
-// for images of at least one 8 x 16 tile, the direct one for the small
-// deep levels.
-int launch_conv(fs_unet *u, const uint16_t *in, int cin, const uint16_t *wt, const float *bias,
-                uint16_t *out, int nout, int Hl, int Wl, int relu, int B) {
-  const long M = static_cast<long>(B) * Hl * Wl;
-  if (Hl >= kTPH && Wl >= kTPW) {
-    const int tx = (Wl + kTPW - 1) / kTPW, ty = (Hl + kTPH - 1) / kTPH;
-    if (nout % 64 == 0)
-      hipLaunchKernelGGL(k_conv3x3_t<64>, dim3(tx, ty * B, nout / 64), dim3(256), 0, u->stream,
-                         in, cin, wt, bias, out, nout, Hl, Wl, relu, ty);
-    else
-      hipLaunchKernelGGL(k_conv3x3_t<32>, dim3(tx, ty * B, nout / 32), dim3(256), 0, u->stream,
-                         in, cin, wt, bias, out, nout, Hl, Wl, relu, ty);
-  } else if (nout % 64 == 0) {
-    hipLaunchKernelGGL(k_conv3x3<4>, dim3((M + 63) / 64, nout / 64), dim3(256), 0, u->stream, in,
-                       cin, wt, bias, out, nout, Hl, Wl, relu, M);
-  } else {
-    hipLaunchKernelGGL(k_conv3x3<2>, dim3((M + 63) / 64, nout / 32), dim3(256), 0, u->stream, in,
-                       cin, wt, bias, out, nout, Hl, Wl, relu, M);
-  }
+ConvSrc src_of(const Tensor &t) { return ConvSrc{t.d, nullptr, t.C, 0, 0}; }
+// [lo upsampled, skip]
+ConvSrc src_of(const Tensor &lo, const Tensor &skip) {
+  return ConvSrc{lo.d, skip.d, lo.C, skip.C, 1};
+}
+ConvDst dst_of(const Tensor &t) {
+  return ConvDst{t.d, nullptr, nullptr, nullptr, nullptr, 0};
+}
+
+template <int R>
+int launch_conv_rows(fs_unet *u, const ConvSrc &src, const uint16_t *wt, const float *bias,
+                     const ConvDst &dst, int nout, int Hl, int Wl, int relu, int B) {
+  const int tx = (Wl + 15) / 16, ty = (Hl + R - 1) / R, tiles = tx * ty * B;
+  const int groups = (tiles + kWaves - 1) / kWaves, nblk = nout / kNB;
+  // two workgroups per CU in all; no more of them than groups to take
+  const int per_xcd = std::max(1, std::min((groups + 7) / 8, 2 * u->ncu / 8 / nblk));
+  hipLaunchKernelGGL(k_conv<R>, dim3(8 * nblk * per_xcd), dim3(64 * kWaves), 0, u->stream, src, wt,
+                     bias, relu, dst, nout, Hl, Wl, tx, ty, tiles, groups);
   return check_launch_u();
 }
 
-int conv_fwd(fs_unet *u, const Conv &c, const Tensor &in, Tensor &out, int B) {
-  const int Hl = u->H >> c.level, Wl = u->W >> c.level;
-  return launch_conv(u, in.d, c.cin, c.wf, u->w + c.boff, out.d, c.cout, Hl, Wl, 1, B);
+// dst = conv3x3(src) with weights wt [tap][nout][cin].
+int launch_conv(fs_unet *u, const ConvSrc &src, const uint16_t *wt, const float *bias,
+                const ConvDst &dst, int nout, int Hl, int Wl, int relu, int B) {
+  if (Hl < 8 || Wl < 16) {
+    const int tx = (Wl + 15) / 16, ty = (Hl + 1) / 2, tiles = tx * ty * B;
+    hipLaunchKernelGGL(k_conv_small, dim3(tiles, nout / kNB), dim3(64), 0, u->stream, src, wt, bias,
+                       relu, dst, nout, Hl, Wl, tx, ty, tiles);
+    return check_launch_u();
+  }
+  // 8 rows a wave wherever that gives every SIMD a wave (1024 of them); below,
+  // 2 rows: one sample of 64 x 64 takes 187 us against 202 with 4 rows, and 32
+  // of 256 x 256 take as long with 4 rows as with 8
+  const long waves = static_cast<long>((Wl + 15) / 16) * (Hl / 8) * B * (nout / kNB);
+  if (waves >= 4l * u->ncu)
+    return launch_conv_rows<8>(u, src, wt, bias, dst, nout, Hl, Wl, relu, B);
+  return launch_conv_rows<2>(u, src, wt, bias, dst, nout, Hl, Wl, relu, B);
+}
+
+// conv + bias + ReLU into out; with pooled, also its 2 x 2 averages
+int conv_fwd(fs_unet *u, const Conv &c, const ConvSrc &in, Tensor &out, const Tensor *pooled,
+             int B) {
+  ConvDst dst = dst_of(out);
+  if (pooled) dst.pool = pooled->d;
+  return launch_conv(u, in, c.wf, u->w + c.boff, dst, c.cout, u->H >> c.level, u->W >> c.level, 1,
+                     B);
 }
 
 // Work split of the nine-tap weight-gradient kernel: about kDwTargetGroups
@@ -912,15 +1052,12 @@ DwPlan dw_plan(int cout, int cin, int Hl, int Wl, int B) {
   return p;
 }
 
-// Gradients of one conv+ReLU layer from gout (gradient of its output):
-// weight and bias gradients, and the input gradient into gin (if given).
-int conv_bwd(fs_unet *u, const Conv &c, const Tensor &in, const Tensor &out, const Tensor &gout,
-             Tensor *gin, int B) {
+// Gradients of one conv layer from gz, the gradient of its output before the
+// ReLU: weight and bias gradients, and the input gradient into gin (if given).
+int conv_bwd(fs_unet *u, const Conv &c, const ConvSrc &in, const Tensor &gz, const ConvDst *gin,
+             int B) {
   const int Hl = u->H >> c.level, Wl = u->W >> c.level;
   const long M = pixels(u, c.level, B);
-  hipLaunchKernelGGL(k_relu_grad, dim3(grid_for(M * c.cout / 8)), dim3(256), 0, u->stream,
-                     gout.d, out.d, u->gz.d, M * c.cout / 8);
-  FS_TRY(check_launch_u());
   // weight gradient, split over pixel chunks
   const size_t wn = 9ul * c.cout * c.cin;
   const DwPlan dp = dw_plan(c.cout, c.cin, Hl, Wl, B);
@@ -931,11 +1068,11 @@ int conv_bwd(fs_unet *u, const Conv &c, const Tensor &in, const Tensor &out, con
                        static_cast<long>(c.cout), 0.f);
     if (dp.cb == 64)
       hipLaunchKernelGGL(k_conv3x3_dw_t<64>, dim3(dp.blocks, dp.nchunks), dim3(kDwThreads), 0,
-                         u->stream, u->gz.d, c.cout, in.d, c.cin, u->part, u->g + c.boff, Hl, Wl,
+                         u->stream, gz.d, c.cout, in, u->part, u->g + c.boff, Hl, Wl,
                          dp.tiles_img, dp.tiles_x, dp.ntiles, dp.tpc, dp.ci_blocks);
     else
       hipLaunchKernelGGL(k_conv3x3_dw_t<32>, dim3(dp.blocks, dp.nchunks), dim3(kDwThreads), 0,
-                         u->stream, u->gz.d, c.cout, in.d, c.cin, u->part, u->g + c.boff, Hl, Wl,
+                         u->stream, gz.d, c.cout, in, u->part, u->g + c.boff, Hl, Wl,
                          dp.tiles_img, dp.tiles_x, dp.ntiles, dp.tpc, dp.ci_blocks);
     FS_TRY(check_launch_u());
     hipLaunchKernelGGL(k_reduce_chunks_wide, dim3(static_cast<unsigned>((wn + 63) / 64)),
@@ -947,8 +1084,8 @@ int conv_bwd(fs_unet *u, const Conv &c, const Tensor &in, const Tensor &out, con
     const int nchunks = static_cast<int>((M + chunk - 1) / chunk);
     if (static_cast<size_t>(nchunks) * wn > u->part_n) return FS_ERR_INTERNAL;
     const int tiles = ((c.cout + 63) / 64) * ((c.cin + 63) / 64);
-    hipLaunchKernelGGL(k_conv3x3_dw, dim3(tiles, 9, nchunks), dim3(256), 0, u->stream, u->gz.d,
-                       c.cout, in.d, c.cin, u->part, Hl, Wl, chunk, M);
+    hipLaunchKernelGGL(k_conv3x3_dw, dim3(tiles, 9, nchunks), dim3(256), 0, u->stream, gz.d,
+                       c.cout, in, u->part, Hl, Wl, chunk, M);
     FS_TRY(check_launch_u());
     hipLaunchKernelGGL(k_reduce_chunks, dim3(grid_for(static_cast<long>(wn))), dim3(256), 0,
                        u->stream, u->part, u->g + c.woff, static_cast<long>(wn), nchunks);
@@ -959,10 +1096,10 @@ int conv_bwd(fs_unet *u, const Conv &c, const Tensor &in, const Tensor &out, con
     hipLaunchKernelGGL(k_fill_f32, dim3(1), dim3(256), 0, u->stream, u->g + c.boff,
                        static_cast<long>(c.cout), 0.f);
     hipLaunchKernelGGL(k_bias_grad, dim3((M + bchunk - 1) / bchunk), dim3(256), 0, u->stream,
-                       u->gz.d, c.cout, u->g + c.boff, M, bchunk);
+                       gz.d, c.cout, u->g + c.boff, M, bchunk);
     FS_TRY(check_launch_u());
   }
-  if (gin) FS_TRY(launch_conv(u, u->gz.d, c.cout, c.wb, nullptr, gin->d, c.cin, Hl, Wl, 0, B));
+  if (gin) FS_TRY(launch_conv(u, src_of(gz), c.wb, nullptr, *gin, c.cin, Hl, Wl, 0, B));
   return FS_OK;
 }
 
@@ -988,23 +1125,15 @@ int forward(fs_unet *u, const float *terrain_d, const float *params_d, int B,
   FS_TRY(check_launch_u());
   const Tensor *in = &u->x0;
   for (int L = 0; L < kLevels; L++) {
-    FS_TRY(conv_fwd(u, u->conv[enc(L, 0)], *in, u->e_a[L], B));
-    FS_TRY(conv_fwd(u, u->conv[enc(L, 1)], u->e_a[L], u->e[L], B));
-    if (L < kLevels - 1) {
-      hipLaunchKernelGGL(k_pool, dim3(grid_for(pixels(u, L + 1, B) * u->e[L].C / 8)), dim3(256),
-                         0, u->stream, u->e[L].d, u->p[L].d, B, u->H >> L, u->W >> L, u->e[L].C);
-      FS_TRY(check_launch_u());
-      in = &u->p[L];
-    }
+    const Tensor *pooled = L < kLevels - 1 ? &u->p[L] : nullptr;
+    FS_TRY(conv_fwd(u, u->conv[enc(L, 0)], src_of(*in), u->e_a[L], nullptr, B));
+    FS_TRY(conv_fwd(u, u->conv[enc(L, 1)], src_of(u->e_a[L]), u->e[L], pooled, B));
+    in = pooled;
   }
   const Tensor *lo = &u->e[kLevels - 1];
   for (int L = kLevels - 2; L >= 0; L--) {
-    hipLaunchKernelGGL(k_upcat, dim3(grid_for(pixels(u, L, B) * u->u[L].C / 8)), dim3(256), 0,
-                       u->stream, lo->d, lo->C, u->e[L].d, u->e[L].C, u->u[L].d, B, u->H >> L,
-                       u->W >> L);
-    FS_TRY(check_launch_u());
-    FS_TRY(conv_fwd(u, u->conv[dec(L, 0)], u->u[L], u->d_a[L], B));
-    FS_TRY(conv_fwd(u, u->conv[dec(L, 1)], u->d_a[L], u->d[L], B));
+    FS_TRY(conv_fwd(u, u->conv[dec(L, 0)], src_of(*lo, u->e[L]), u->d_a[L], nullptr, B));
+    FS_TRY(conv_fwd(u, u->conv[dec(L, 1)], src_of(u->d_a[L]), u->d[L], nullptr, B));
     lo = &u->d[L];
   }
   const long M = pixels(u, 0, B);
@@ -1026,29 +1155,35 @@ int backward(fs_unet *u, int B) {
                             hipMemcpyDeviceToDevice, u->stream));
   FS_HIP_TRY(hipMemcpyAsync(u->g + u->head_b, u->head_acc + 33, sizeof(float),
                             hipMemcpyDeviceToDevice, u->stream));
-  // decoder, top level first
+  // decoder, top level first; the gradient of the concatenated input goes to
+  // the level below (summed over the upsampling) and to the skip connection
   for (int L = 0; L <= kLevels - 2; L++) {
-    FS_TRY(conv_bwd(u, u->conv[dec(L, 1)], u->d_a[L], u->d[L], u->gd[L], &u->gd_a[L], B));
-    FS_TRY(conv_bwd(u, u->conv[dec(L, 0)], u->u[L], u->d_a[L], u->gd_a[L], &u->gu[L], B));
-    Tensor &glo = (L + 1 <= kLevels - 2) ? u->gd[L + 1] : u->ge[kLevels - 1];
-    hipLaunchKernelGGL(k_upcat_grad, dim3(grid_for(pixels(u, L, B) * u->u[L].C / 8)), dim3(256),
-                       0, u->stream, u->gu[L].d, glo.C, u->ge[L].C, glo.d, u->ge[L].d, B,
-                       u->H >> L, u->W >> L);
-    FS_TRY(check_launch_u());
+    const bool deepest = L + 1 == kLevels - 1;
+    const Tensor &lo = deepest ? u->e[L + 1] : u->d[L + 1];
+    ConvDst ga = dst_of(u->gd_a[L]);
+    ga.mask = u->d_a[L].d;
+    FS_TRY(conv_bwd(u, u->conv[dec(L, 1)], src_of(u->d_a[L]), u->gd[L], &ga, B));
+    ConvDst gu = dst_of(u->ge[L]);
+    gu.lo = deepest ? u->ge[L + 1].d : u->gd[L + 1].d;
+    gu.lo_mask = lo.d;
+    gu.c1 = lo.C;
+    FS_TRY(conv_bwd(u, u->conv[dec(L, 0)], src_of(lo, u->e[L]), u->gd_a[L], &gu, B));
   }
   // encoder, bottom level first; ge[L] holds the skip gradient, the pooled
   // path's gradient is added
   for (int L = kLevels - 1; L >= 0; L--) {
     if (L < kLevels - 1) {
       hipLaunchKernelGGL(k_pool_grad, dim3(grid_for(pixels(u, L, B) * u->ge[L].C / 8)),
-                         dim3(256), 0, u->stream, u->gp[L].d, u->ge[L].d, B, u->H >> L,
-                         u->W >> L, u->ge[L].C, 1);
+                         dim3(256), 0, u->stream, u->gp[L].d, u->ge[L].d, u->e[L].d, B, u->H >> L,
+                         u->W >> L, u->ge[L].C);
       FS_TRY(check_launch_u());
     }
-    FS_TRY(conv_bwd(u, u->conv[enc(L, 1)], u->e_a[L], u->e[L], u->ge[L], &u->ge_a[L], B));
+    ConvDst ga = dst_of(u->ge_a[L]);
+    ga.mask = u->e_a[L].d;
+    FS_TRY(conv_bwd(u, u->conv[enc(L, 1)], src_of(u->e_a[L]), u->ge[L], &ga, B));
     const Tensor &in = L == 0 ? u->x0 : u->p[L - 1];
-    FS_TRY(conv_bwd(u, u->conv[enc(L, 0)], in, u->e_a[L], u->ge_a[L],
-                    L == 0 ? nullptr : &u->gp[L - 1], B));
+    const ConvDst gp = L == 0 ? ConvDst{} : dst_of(u->gp[L - 1]);
+    FS_TRY(conv_bwd(u, u->conv[enc(L, 0)], src_of(in), u->ge_a[L], L == 0 ? nullptr : &gp, B));
   }
   return FS_OK;
 }
@@ -1059,7 +1194,7 @@ void free_unet(fs_unet *u) {
   if (u->stream) (void)hipStreamSynchronize(u->stream);
   std::vector<void *> ptrs = {u->w, u->g, u->m, u->v, u->part, u->yhat, u->tgt, u->head_acc,
                               u->terrain, u->params_in, u->data_terrain, u->data_params,
-                              u->data_tgt, u->x0.d, u->gz.d};
+                              u->data_tgt, u->x0.d};
   for (int L = 0; L < kLevels; L++) {
     ptrs.push_back(u->e_a[L].d);
     ptrs.push_back(u->e[L].d);
@@ -1067,8 +1202,7 @@ void free_unet(fs_unet *u) {
     ptrs.push_back(u->ge[L].d);
   }
   for (int L = 0; L < kLevels - 1; L++)
-    for (Tensor *t : {&u->p[L], &u->u[L], &u->d_a[L], &u->d[L], &u->gp[L], &u->gu[L],
-                      &u->gd_a[L], &u->gd[L]})
+    for (Tensor *t : {&u->p[L], &u->d_a[L], &u->d[L], &u->gp[L], &u->gd_a[L], &u->gd[L]})
       ptrs.push_back(t->d);
   for (Conv &c : u->conv) {
     ptrs.push_back(c.wf);
@@ -1127,6 +1261,7 @@ int fs_unet_create(int height, int width, int max_batch, uint64_t seed, int devi
   u->device = device;
   FS_HIP_TRY(hipSetDevice(device));
   FS_HIP_TRY(hipStreamCreateWithFlags(&u->stream, hipStreamNonBlocking));
+  FS_HIP_TRY(hipDeviceGetAttribute(&u->ncu, hipDeviceAttributeMultiprocessorCount, device));
   // layers
   auto add = [&](int cin, int cout, int level) {
     Conv c;
@@ -1188,21 +1323,13 @@ int fs_unet_create(int height, int width, int max_batch, uint64_t seed, int devi
     FS_TRY(alloc_tensor(u, u->ge[L], kWidth[L], L));
   }
   for (int L = 0; L < kLevels - 1; L++) {
-    const int below = L == kLevels - 2 ? kWidth[kLevels - 1] : kWidth[L + 1];
     FS_TRY(alloc_tensor(u, u->p[L], kWidth[L], L + 1));
     FS_TRY(alloc_tensor(u, u->gp[L], kWidth[L], L + 1));
-    FS_TRY(alloc_tensor(u, u->u[L], below + kWidth[L], L));
-    FS_TRY(alloc_tensor(u, u->gu[L], below + kWidth[L], L));
     FS_TRY(alloc_tensor(u, u->d_a[L], kWidth[L], L));
     FS_TRY(alloc_tensor(u, u->gd_a[L], kWidth[L], L));
     FS_TRY(alloc_tensor(u, u->d[L], kWidth[L], L));
     FS_TRY(alloc_tensor(u, u->gd[L], kWidth[L], L));
   }
-  // gz holds the largest conv output
-  size_t gzn = 0;
-  for (const Conv &c : u->conv)
-    gzn = std::max(gzn, static_cast<size_t>(pixels(u, c.level, max_batch)) * c.cout);
-  FS_TRY(fs::dev_alloc(&u->gz.d, gzn));
   const size_t HWB = static_cast<size_t>(max_batch) * height * width;
   FS_TRY(fs::dev_alloc(&u->yhat, HWB));
   FS_TRY(fs::dev_alloc(&u->tgt, HWB));
