@@ -129,7 +129,7 @@ struct fs_model {
   // timers
   uint64_t timer_us[FS_NUM_TIMERS] = {};
   double stage_ms[FS_NUM_TIMERS] = {};
-  hipEvent_t ev[2][7] = {};
+  hipEvent_t ev[2][7] = {};           // a level-path step's stages (created on first use)
   bool ev_pending[2] = {false, false};
   int ev_cur = 0;                     // level-path steps alternate the two sets
   // Tile and tile-graph steps are not bracketed by events one by one: a batch
@@ -416,10 +416,7 @@ int create_model(int W, int H, const fs_params *p, const double *h_init, uint32_
   m->ek = make_erode_const(*p, &m->nmode);
   FS_HIP_TRY(hipSetDevice(device));
   FS_HIP_TRY(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking));
-  for (auto &set : m->ev)
-    for (auto &e : set) FS_HIP_TRY(hipEventCreate(&e));
   for (auto &e : m->tev) FS_HIP_TRY(hipEventCreate(&e));
-  for (auto &e : m->gev) FS_HIP_TRY(hipEventCreate(&e));
 
   const size_t N = static_cast<size_t>(m->N);
   const size_t ntiles = (N + kBfsTile - 1) / kBfsTile + 1;
@@ -558,7 +555,7 @@ int launch_receivers(fs_model *m, const double *h, const int32_t *prev = nullptr
   // a wave's 64 columns x kRecvShort rows, four waves down a workgroup
   const unsigned gx = static_cast<unsigned>((m->W - 4 + kWave - 1) / kWave);
   const int groups = (m->H - 4 + kRecvShort - 1) / kRecvShort;
-  const unsigned gyz = static_cast<unsigned>((groups + 256 / kWave - 1) / (256 / kWave));
+  const unsigned gyz = static_cast<unsigned>((groups + kRecvGroups - 1) / kRecvGroups);
   const unsigned gy = std::min(gyz, 65535u), gz = (gyz + gy - 1) / gy;   // grid.y's limit
   FS_TRY(kt_begin(m, FS_K_RECEIVERS));
   hipLaunchKernelGGL(k_receivers, dim3(gx, gy, gz), dim3(256), 0, m->stream, h, m->rcv, m->W,
@@ -1098,6 +1095,8 @@ int advance(fs_model *m, long long want, int *took) {
     const hipEvent_t *ev = none;
     if (!m->graph_open) {
       FS_TRY(graph_collect(m));
+      for (auto &e : m->gev)
+        if (!e) FS_HIP_TRY(hipEventCreate(&e));
       m->graph_open = true;
       ev = m->gev;
     }
@@ -1114,6 +1113,8 @@ int advance(fs_model *m, long long want, int *took) {
   } else {
     FS_TRY(graph_close(m));
     hipEvent_t *ev = m->ev[m->ev_cur];
+    for (int i = 0; m->owns_memory && i < 7; i++)
+      if (!ev[i]) FS_HIP_TRY(hipEventCreate(&ev[i]));
     FS_TRY(mark(ev[0], m->stream));
     if (!stuck) FS_TRY(launch_receivers(m, m->h));
     FS_TRY(mark(ev[1], m->stream));

@@ -195,19 +195,12 @@ __global__ void k_fill_counts(int32_t *hdr, int n_counts) {
   if (i <= kJumpPasses) hdr[kHdrJump + i] = 0;
 }
 
-// ComputeReceivers (RB:160-182).  Each thread owns one column of a run of
-// interior rows (whole strips of kRecvRows) and slides a 3x3 window down it,
-// so every elevation is fetched from HBM about once (neighbouring columns
-// come from L1, and a run re-reads only its two halo rows).
-// fs::receiver_try picks the reference's direction -- steepest
-// (hc - h[n]) / dr[n] over n = 0..7 with a strict '>' from 0, ties to the
-// lowest n, flat cells and pits NO_FLOW -- without dividing; the rare cells it
-// leaves undecided (near-ties, extreme magnitudes) send the column's run
-// through fs::receiver_fast again, which divides where it must, so the row
-// loop has no branch.  Rows are read and written through buffer resources
-// built per row in scalar registers: the lane's column is a constant offset,
-// so the loop spends no vector instructions on addresses.
-constexpr int kRecvRows = 16;
+// ComputeReceivers (RB:160-182).  fs::receiver_fast picks the reference's
+// direction -- steepest (hc - h[n]) / dr[n] over n = 0..7 with a strict '>'
+// from 0, ties to the lowest n, flat cells and pits NO_FLOW -- and divides only
+// in the rare cells that need it (near-ties, extreme magnitudes).  Rows are
+// read through buffer resources built per row in scalar registers: the lane's
+// column is a constant offset, so no vector instructions go to addresses.
 constexpr int kRsrcWord3 = 0x00020000;          // raw (unformatted) buffer, gfx9
 using v4u = unsigned __attribute__((ext_vector_type(4)));
 using v2u = unsigned __attribute__((ext_vector_type(2)));
@@ -228,70 +221,10 @@ __device__ __forceinline__ void load_cols(__amdgpu_buffer_rsrc_t r, uint32_t xo,
   rr = __builtin_bit_cast(double, b);
 }
 
-// Rows y0 .. y0+n-1 (all interior: 2 <= y0, y0+n <= H-2) of column x.  The
-// window holds rows y-1, y, y+1 and the next row's load is in flight while
-// row y is decided (row y+2 <= H-1 always exists).
-__device__ __forceinline__ void receivers_rows(const double *__restrict__ h,
-                                               uint8_t *__restrict__ rcv, int W, int x, int y0,
-                                               int n, double d_card, double d_diag) {
-  const bool div_ok = fs::divisors_in_range(d_card, d_diag);
-  const uint32_t rowb = static_cast<uint32_t>(W) * 8u;
-  const uint32_t xo = static_cast<uint32_t>(x - 1) * 8u;
-  const double *row = h + static_cast<size_t>(y0 - 1) * W;   // row y-1 of the first cell
-  uint8_t *out = rcv + static_cast<size_t>(y0) * W;
-  double a0, a1, a2, b0, b1, b2, c0, c1, c2;
-  load_cols(row_rsrc(row, rowb), xo, a0, a1, a2);
-  load_cols(row_rsrc(row + W, rowb), xo, b0, b1, b2);
-  load_cols(row_rsrc(row + 2 * W, rowb), xo, c0, c1, c2);
-  uint32_t undecided = 0;
-  auto one_row = [&]() {
-    double d0, d1, d2;
-    load_cols(row_rsrc(row + 3 * W, rowb), xo, d0, d1, d2);
-    // neighbours in direction order W, NW, N, NE, E, SE, S, SW (RB:79-82)
-    const double nb[8] = {b0, a0, a1, a2, b2, c2, c1, c0};
-    bool ok;
-    const int r = fs::receiver_try(b1, nb, d_card, d_diag, div_ok, &ok);
-    __builtin_amdgcn_raw_buffer_store_b8(static_cast<uint8_t>(r), row_rsrc(out, W), x, 0, 0);
-    undecided |= ok ? 0u : 1u;
-    // settle the flag here: left symbolic, every row's comparison masks stay
-    // live in scalar registers until after the loop
-    asm volatile("" : "+v"(undecided));
-    row += W;
-    out += W;
-    a0 = b0; a1 = b1; a2 = b2;
-    b0 = c0; b1 = c1; b2 = c2;
-    c0 = d0; c1 = d1; c2 = d2;
-  };
-  int k = 0;
-  for (; k + kRecvRows <= n; k += kRecvRows) {
-#pragma unroll
-    for (int u = 0; u < kRecvRows; u++) one_row();
-  }
-  for (; k < n; k++) one_row();
-  if (undecided) {   // rare: the column's rows again, with the divisions where needed
-    for (k = 0; k < n; k++) {
-      const double *up = h + static_cast<size_t>(y0 + k - 1) * W + x;
-      const double *mid = up + W, *dn = mid + W;
-      const double nb[8] = {mid[-1], up[-1], up[0], up[1], mid[1], dn[1], dn[0], dn[-1]};
-      rcv[static_cast<size_t>(y0 + k) * W + x] =
-          static_cast<uint8_t>(fs::receiver_fast(mid[0], nb, d_card, d_diag, div_ok));
-    }
-  }
-}
-
-// Strips s0 .. s1-1 of kRecvRows interior rows each, as one run of rows.
-__device__ __forceinline__ void receivers_strips(const double *__restrict__ h,
-                                                 uint8_t *__restrict__ rcv, int W, int H, int x,
-                                                 int s0, int s1, double d_card, double d_diag) {
-  const int y0 = s0 * kRecvRows + 2;
-  const int n = min(s1 * kRecvRows + 2, H - 2) - y0;
-  if (n > 0) receivers_rows(h, rcv, W, x, y0, n, d_card, d_diag);
-}
-
 // Receivers of one grid: each wave owns 64 columns x kRecvShort rows, with all
 // its kRecvShort + 2 rows requested before the first is used, so a cell waits
-// for memory once.  The rolling window above (32 rows per thread, one row
-// ahead) left small grids to a chain of 32 dependent row loads on a few
+// for memory once.  A rolling window (32 rows per thread, one row ahead)
+// left small grids to a chain of 32 dependent row loads on a few
 // waves: 15 us at 101^2 and at 1000^2 alike.  Six rows were the best of 1 to
 // 16 at every size: 19.1 -> 9.0 us at 1000^2, 22.4 -> 15.9 at 2048^2, 93.5 ->
 // 86.3 at 6000^2, 227 -> 223.5 at 10000^2 (HIP events, their own 4 us
@@ -304,26 +237,49 @@ __device__ __forceinline__ void receivers_strips(const double *__restrict__ h,
 // smaller halo fits again; -1: no such limit), this step is not taken either,
 // and nothing is written but the slot.
 constexpr int kRecvShort = 6;
+constexpr int kRecvGroups = 256 / kWave;   // row groups per workgroup
+struct ShortRows {
+  double l[kRecvShort + 2], c[kRecvShort + 2], r[kRecvShort + 2];
+};
+// Requests the rows of row group `group` in column x (past the grid's last
+// row: that row again).
+__device__ __forceinline__ void load_short(ShortRows &v, const double *__restrict__ h, int W, int H,
+                                           int x, int group) {
+  const uint32_t rowb = static_cast<uint32_t>(W) * 8u;
+  const uint32_t xo = static_cast<uint32_t>(x - 1) * 8u;
+  const int y0 = group * kRecvShort + 2;
+#pragma unroll
+  for (int k = 0; k < kRecvShort + 2; k++)
+    load_cols(row_rsrc(h + static_cast<size_t>(min(y0 - 1 + k, H - 1)) * W, rowb), xo, v.l[k],
+              v.c[k], v.r[k]);
+}
+__device__ __forceinline__ void decide_short(const ShortRows &v, uint8_t *__restrict__ rcv, int W,
+                                             int H, int x, int group, double d_card,
+                                             double d_diag) {
+  const bool div_ok = fs::divisors_in_range(d_card, d_diag);
+  const int y0 = group * kRecvShort + 2;
+#pragma unroll
+  for (int k = 0; k < kRecvShort; k++) {
+    if (y0 + k >= H - 2) break;
+    const double nb[8] = {v.l[k + 1], v.l[k],     v.c[k],     v.r[k],
+                          v.r[k + 1], v.r[k + 2], v.c[k + 2], v.l[k + 2]};
+    rcv[static_cast<size_t>(y0 + k) * W + x] =
+        static_cast<uint8_t>(fs::receiver_fast(v.c[k + 1], nb, d_card, d_diag, div_ok));
+  }
+}
+
 __global__ __launch_bounds__(256) void k_receivers(const double *__restrict__ h,
                                                    uint8_t *__restrict__ rcv, int W, int H,
                                                    double d_card, double d_diag,
                                                    const int32_t *__restrict__ hdr,
                                                    const int32_t *prev, int32_t *slot,
                                                    int shallow) {
-  constexpr int ROWS = kRecvShort;
   const int x = blockIdx.x * kWave + static_cast<int>(threadIdx.x % kWave) + 2;
   const int group = __builtin_amdgcn_readfirstlane(
-      (blockIdx.z * gridDim.y + blockIdx.y) * (256 / kWave) + threadIdx.x / kWave);
-  const int y0 = group * ROWS + 2;
-  if (x >= W - 2 || y0 >= H - 2) return;
-  const bool div_ok = fs::divisors_in_range(d_card, d_diag);
-  const uint32_t rowb = static_cast<uint32_t>(W) * 8u;
-  const uint32_t xo = static_cast<uint32_t>(x - 1) * 8u;
-  double l[ROWS + 2], c[ROWS + 2], r[ROWS + 2];
-#pragma unroll
-  for (int k = 0; k < ROWS + 2; k++)   // past the grid's last row: that row again
-    load_cols(row_rsrc(h + static_cast<size_t>(min(y0 - 1 + k, H - 1)) * W, rowb), xo, l[k], c[k],
-              r[k]);
+      (blockIdx.z * gridDim.y + blockIdx.y) * kRecvGroups + threadIdx.x / kWave);
+  if (x >= W - 2 || group * kRecvShort + 2 >= H - 2) return;
+  ShortRows v;
+  load_short(v, h, W, H, x, group);
   const bool stop = prev != nullptr && (prev[kSlotOver] != 0 || prev[kSlotStop] != 0 ||
                                         hdr[2] != 0 || prev[kSlotDeepest] <= shallow);
   if (slot != nullptr && x == 2 && group == 0) {   // one thread of the grid
@@ -332,13 +288,7 @@ __global__ __launch_bounds__(256) void k_receivers(const double *__restrict__ h,
     slot[kSlotStop] = stop ? 1 : 0;
   }
   if (stop) return;
-#pragma unroll
-  for (int k = 0; k < ROWS; k++) {
-    if (y0 + k >= H - 2) break;
-    const double nb[8] = {l[k + 1], l[k], c[k], r[k], r[k + 1], r[k + 2], c[k + 2], l[k + 2]};
-    rcv[static_cast<size_t>(y0 + k) * W + x] =
-        static_cast<uint8_t>(fs::receiver_fast(c[k + 1], nb, d_card, d_diag, div_ok));
-  }
+  decide_short(v, rcv, W, H, x, group, d_card, d_diag);
 }
 
 // Donor bitmask and level of every cell.  Rows are strided over the grid so

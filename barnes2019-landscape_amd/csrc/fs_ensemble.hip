@@ -1,40 +1,44 @@
 // fs_ensemble.hip -- many FastScape grids ("realizations") of different
-// sizes and parameters advanced by ONE persistent cooperative launch per
-// time-step.
+// sizes and parameters advanced together, every kernel of a time-step
+// launched once for all of them.
 //
 // Every realization takes the reference's time-step (fastscape_RB.cpp:366-376)
 // and gets the same bits as a single-grid model with its size, parameters and
-// initial terrain.  A step is one launch of k_ens_step, a grid of one
-// 1024-thread workgroup per CU, in phases separated by grid barriers:
+// initial terrain.  A step, on one stream:
 //
-//   R  receivers of every realization (RB:160-182), 256-column x recv_rows
-//      work items dealt round-robin; block 0 lists the tile candidates
-//      (realizations whose drainage was at most kHalo levels deep last step)
-//   A  tile accumulation (upstream counts and levels, RB:213-279) of every
-//      candidate's 64x64 tiles; a tile deeper than kHalo marks its
-//      realization deep
-//   -  block 0 lists the erosion work (the shallow realizations' tiles) and
-//      the deep realizations (a tile deeper than kHalo, or deeper than kHalo
-//      last step) for the tile-graph kernels
-//   E  work items claimed in list order from one counter: tile uplift +
-//      erosion in LDS (RB:285-328)
+//   k_ens_receivers  receivers of every realization (RB:160-182)
+//   k_ens_acc        tile accumulation (upstream counts and levels,
+//                    RB:213-279) of every 64x64 tile of the candidates: the
+//                    realizations at most kHalo levels deep last step; a tile
+//                    deeper than kHalo marks its realization deep
+//   k_ens_lists      one workgroup: each realization's path this step, and the
+//                    deep ones' tiles as the tile-graph kernels' work list
+//   k_ens_erode      tile uplift + erosion (RB:285-328) of the others
 //
 // The deep realizations then take one tile-graph step together (fs_deep.h):
 // per 64x64 tile with no halo, every deep realization's tiles in the same
 // launches, the tiles joined by the graph of the cells where drainage leaves
 // a tile; the step also counts their levels, so the next step knows which
-// are shallow again.
+// are shallow again.  The host reads the work list's size while k_ens_erode
+// runs.
 //
-// Results do not depend on the schedule (work item sizes): each cell's
-// elevation depends only on its own inputs and its receiver's final value,
-// and upstream counts are integers.
+// The kernels are the single-grid ones' bodies, with a table from workgroup to
+// realization; workgroups of realizations on the other path return at once.
+// One persistent cooperative kernel for all phases ran one 1024-thread
+// workgroup per CU (the LDS of its largest phase) behind grid barriers: 394 us
+// a step for 32 realizations of 256^2 (512 tiles), which these four kernels
+// step in 64.
+//
+// A cell's elevation depends only on its own inputs and its receiver's final
+// value, and upstream counts are integers, so the order of the work is free.
+// (fs_schedule's work item sizes were the persistent kernel's; they are
+// accepted and have no effect.)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <chrono>
 #include <cmath>
 #include <cstring>
-#include <map>
 #include <new>
 #include <numeric>
 #include <string>
@@ -50,11 +54,9 @@
 
 namespace {
 
-constexpr int kEnsBlock = 1024;
-constexpr int kRecvLanes = 256;                     // columns per receiver work item
-constexpr int kRecvQuarters = kEnsBlock / kRecvLanes;
+constexpr int kEnsBlock = 1024;                     // k_ens_lists
 constexpr int kHistLen = kHalo + 1;
-constexpr int kSpinCap = 1 << 22;                   // bounded waits (seconds)
+constexpr int kRecvRows = 16;                       // schedules name multiples of this
 constexpr int kMaxRealizations = 1 << 20;
 
 // per-realization state words (kRH ints each)
@@ -63,15 +65,8 @@ constexpr int kRhDepth = 0;       // deepest level of the last step
 constexpr int kRhOver = 1;        // tiles deeper than kHalo this step
 constexpr int kRhErr = 2;         // error bits (same slot as a model's hdr[2])
 constexpr int kRhPath = 7;        // path of the last step: 1 tiles, 3 tile graph
-constexpr int kRhCand = 8;        // tile candidate this step
 constexpr int kRhTileSteps = 9;
 constexpr int kRhLevelSteps = 10;   // steps off the tiles (the tile graph)
-
-// global control words
-constexpr int kCtlBarrier = 0, kCtlClaim = 1, kCtlAbort = 2;
-constexpr int kCtlEntriesA = 3, kCtlItemsA = 4, kCtlEntriesE = 5, kCtlItemsE = 6;
-constexpr int kCtlGraph = 8;      // the tile-graph work list's size: [8] entries, [9] tiles
-constexpr int kCtlInts = 10;
 
 struct EnsReal {
   uint64_t off;        // first cell of the realization in the cell arrays
@@ -82,96 +77,42 @@ struct EnsReal {
   int lev_cap;         // level entries available
   int nmode;
   int recv_xb;         // receiver column blocks
-  int pad;
+  int recv_first;      // first receiver workgroup
   double d_card, d_diag;
   ErodeConst ek;
 };
 
+// The realizations and their state.
 struct EnsArgs {
   const EnsReal *real;
   int R;
-  int recv_rows, tiles_per_claim;
   double *h_old, *h_new;
   uint8_t *rcv, *lvl;
   uint32_t *cnt;
   TilePlan *plan;
   const double *ftab;
-  int32_t *rh, *hist, *ctl;
-  const int32_t *recv_first;   // R+1 prefix of receiver work items
-  int32_t *tabA_off, *tabA_real, *tabE_off, *tabE_real;
-  int32_t *tabG_off, *tabG_real;   // the deep realizations (tile-graph work list)
-  uint32_t bar_base;
+  int32_t *rh, *hist;
 };
 
-__device__ __forceinline__ int32_t ld_agent(const int32_t *p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Barrier of `members` workgroups on a monotonically increasing counter;
-// `target` is this workgroup's running arrival target.  The wait is bounded:
-// on expiry the launch is marked aborted and every later wait returns at
-// once, so the grid always drains.
-__device__ __forceinline__ void counter_barrier(int32_t *bar, uint32_t &target, int members,
-                                                int32_t *ctl) {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-  __syncthreads();
-  target += static_cast<uint32_t>(members);
-  if (threadIdx.x == 0) {
-    __hip_atomic_fetch_add(bar, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    int spins = 0;
-    while (static_cast<int32_t>(static_cast<uint32_t>(ld_agent(bar)) - target) < 0) {
-      if (ld_agent(&ctl[kCtlAbort])) break;
-      if (++spins > kSpinCap) {
-        atomicOr(&ctl[kCtlAbort], 1);
-        break;
-      }
-      __builtin_amdgcn_s_sleep(2);
-    }
-  }
-  __syncthreads();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-}
-
-// Last index i in [0, n) with off[i] <= v (off ascending, off[0] <= v).
-__device__ __forceinline__ int find_entry(const int32_t *off, int n, int v) {
-  int lo = 0, hi = n - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (off[mid] <= v) lo = mid;
-    else hi = mid - 1;
-  }
-  return lo;
-}
-
-struct TableShared {
-  uint32_t scan[kEnsBlock / kWave + 1];
-};
-
-union EnsShared {
-  AccShared acc;
-  EroShared ero;
-  TableShared tab;
-};
-
-// Block 0: list the realizations with count(r) > 0, in increasing r among
-// those with pick(r), appending after `entries`/`items`; off[e] is the first
-// work item of entry e.
-template <class Pick, class Count>
-__device__ void append_entries(int R, Pick pick, Count count, int32_t *off, int32_t *real,
-                               int &entries, int &items, TableShared &ts) {
+// Lists the realizations r in [0, R) with pick(r): real[e] is entry e's
+// realization, off[e] its first tile in the list.  One workgroup of kEnsBlock
+// threads; sh holds kEnsBlock / kWave + 1 words.
+template <class Pick>
+__device__ void list_entries(int R, const EnsReal *rl, Pick pick, int32_t *off, int32_t *real,
+                             int &entries, int &tiles, uint32_t *sh) {
+  entries = tiles = 0;
   for (int base = 0; base < R; base += kEnsBlock) {
     const int r = base + threadIdx.x;
-    int v = 0;
-    if (r < R && pick(r)) v = count(r);
+    const int v = r < R && pick(r) ? rl[r].ntiles : 0;
     uint32_t te, ti;
-    const uint32_t ee = block_excl_scan<kEnsBlock>(v > 0 ? 1u : 0u, &te, ts.scan);
-    const uint32_t ei = block_excl_scan<kEnsBlock>(static_cast<uint32_t>(v), &ti, ts.scan);
+    const uint32_t ee = block_excl_scan<kEnsBlock>(v > 0 ? 1u : 0u, &te, sh);
+    const uint32_t ei = block_excl_scan<kEnsBlock>(static_cast<uint32_t>(v), &ti, sh);
     if (v > 0) {
-      off[entries + ee] = items + static_cast<int>(ei);
+      off[entries + ee] = tiles + static_cast<int>(ei);
       real[entries + ee] = r;
     }
     entries += static_cast<int>(te);
-    items += static_cast<int>(ti);
+    tiles += static_cast<int>(ti);
   }
 }
 
@@ -186,143 +127,108 @@ __device__ __forceinline__ void with_nmode(int nm, F f) {
   }
 }
 
-// One time-step of every realization.  NM is the pow mode shared by all
-// realizations, or -1 for a mix.
-template <int NM>
-__global__ __launch_bounds__(kEnsBlock) void k_ens_step(EnsArgs a) {
-  __shared__ EnsShared sh;
-  __shared__ int s_item;
-  const int R = a.R;
-  uint32_t bar = a.bar_base;
-  // ---- phase R: per-step state, the tile candidates, receivers -----------
-  for (int r = blockIdx.x * kEnsBlock + threadIdx.x; r < R; r += gridDim.x * kEnsBlock) {
-    int32_t *q = a.rh + static_cast<size_t>(r) * kRH;
-    q[kRhOver] = 0;
-    for (int l = 0; l < kHistLen; l++) a.hist[static_cast<size_t>(r) * kHistLen + l] = 0;
+// Workgroup number in a grid of ens_grid's shape.
+__device__ __forceinline__ int ens_block() {
+  return static_cast<int>(blockIdx.y * gridDim.x + blockIdx.x);
+}
+
+// recv_real: each workgroup's realization (nblocks of them).
+__global__ __launch_bounds__(256) void k_ens_receivers(EnsArgs a,
+                                                       const int32_t *__restrict__ recv_real,
+                                                       int nblocks) {
+  const int b = ens_block();
+  if (b >= nblocks) return;
+  const int r = recv_real[b];
+  const EnsReal &g = a.real[r];
+  const int local = b - g.recv_first;
+  if (local == 0) {   // the realization's per-step state
+    if (threadIdx.x == 0) a.rh[static_cast<size_t>(r) * kRH + kRhOver] = 0;
+    if (threadIdx.x < kHistLen) a.hist[static_cast<size_t>(r) * kHistLen + threadIdx.x] = 0;
   }
-  if (blockIdx.x == 0) {
-    if (threadIdx.x == 0) a.ctl[kCtlClaim] = 0;
-    int entries = 0, items = 0;
-    append_entries(
-        R, [&](int r) { return a.rh[static_cast<size_t>(r) * kRH + kRhDepth] <= kHalo; },
-        [&](int r) { return a.real[r].ntiles; }, a.tabA_off, a.tabA_real, entries, items,
-        sh.tab);
-    if (threadIdx.x == 0) {
-      a.tabA_off[entries] = items;
-      a.ctl[kCtlEntriesA] = entries;
-      a.ctl[kCtlItemsA] = items;
-    }
-    for (int r = threadIdx.x; r < R; r += kEnsBlock)
-      a.rh[static_cast<size_t>(r) * kRH + kRhCand] =
-          a.rh[static_cast<size_t>(r) * kRH + kRhDepth] <= kHalo;
-  }
-  {
-    const int quarter = threadIdx.x / kRecvLanes, lane = threadIdx.x % kRecvLanes;
-    const int nitems = a.recv_first[R];
-    const int spi = a.recv_rows / kRecvRows;
-    for (int item = blockIdx.x * kRecvQuarters + quarter; item < nitems;
-         item += gridDim.x * kRecvQuarters) {
-      const int r = find_entry(a.recv_first, R + 1, item);
-      const EnsReal &g = a.real[r];
-      const int local = item - a.recv_first[r];
-      const int x = (local % g.recv_xb) * kRecvLanes + lane + 2;
-      if (x >= g.W - 2) continue;
-      const int nstrips = (g.H - 4 + kRecvRows - 1) / kRecvRows;
-      const int s0 = (local / g.recv_xb) * spi, s1 = min(nstrips, s0 + spi);
-      receivers_strips(a.h_old + g.off, a.rcv + g.off, g.W, g.H, x, s0, s1, g.d_card, g.d_diag);
-    }
-  }
-  counter_barrier(&a.ctl[kCtlBarrier], bar, gridDim.x, a.ctl);
-  // ---- phase A: tile accumulation of the candidates -----------------------
-  {
-    const int entries = ld_agent(&a.ctl[kCtlEntriesA]), nitems = ld_agent(&a.ctl[kCtlItemsA]);
-    for (int b = blockIdx.x; b < nitems; b += gridDim.x) {
-      const int item = xcd_tile(b, nitems);
-      const int e = find_entry(a.tabA_off, entries + 1, item);
-      const int r = a.tabA_real[e];
-      const EnsReal &g = a.real[r];
-      const int t = item - a.tabA_off[e];
-      const int over = tile_acc_body<kEnsBlock>(
-          sh.acc, a.rcv + g.off, a.cnt + g.off, a.lvl + g.off, a.plan + g.plan_off + t, g.W, g.H,
-          t, g.tiles_x, a.hist + static_cast<size_t>(r) * kHistLen, nullptr);
-      if (threadIdx.x == 0 && over) atomicAdd(&a.rh[static_cast<size_t>(r) * kRH + kRhOver], 1);
-      __syncthreads();
-    }
-  }
-  counter_barrier(&a.ctl[kCtlBarrier], bar, gridDim.x, a.ctl);
-  // ---- erosion work list ----------------------------------------------------
-  if (blockIdx.x == 0) {
-    auto deep = [&](int r) {
-      const int32_t *q = a.rh + static_cast<size_t>(r) * kRH;
-      return !q[kRhCand] || q[kRhOver] > 0;
-    };
-    for (int r = threadIdx.x; r < R; r += kEnsBlock) {
-      int32_t *q = a.rh + static_cast<size_t>(r) * kRH;
-      if (deep(r)) {
-        q[kRhPath] = 3;
-        q[kRhLevelSteps]++;
-      } else {
-        int D = 0;
-        for (int l = 0; l < kHistLen; l++)
-          if (a.hist[static_cast<size_t>(r) * kHistLen + l]) D = l;
-        q[kRhDepth] = D;
-        q[kRhPath] = 1;
-        q[kRhTileSteps]++;
-      }
-    }
-    __syncthreads();
-    int entries = 0, items = 0;
-    // the deep realizations' tiles: the tile-graph kernels' work list
-    append_entries(R, deep, [&](int r) { return a.real[r].ntiles; }, a.tabG_off, a.tabG_real,
-                   entries, items, sh.tab);
-    if (threadIdx.x == 0) {
-      a.tabG_off[entries] = items;
-      a.ctl[kCtlGraph] = entries;
-      a.ctl[kCtlGraph + 1] = items;
-    }
-    entries = items = 0;
-    const int tpc = a.tiles_per_claim;
-    append_entries(
-        R, [&](int r) { return !deep(r); },
-        [&](int r) { return (a.real[r].ntiles + tpc - 1) / tpc; }, a.tabE_off, a.tabE_real,
-        entries, items, sh.tab);
-    if (threadIdx.x == 0) {
-      a.tabE_off[entries] = items;
-      a.ctl[kCtlEntriesE] = entries;
-      a.ctl[kCtlItemsE] = items;
+  const int x = (local % g.recv_xb) * kWave + static_cast<int>(threadIdx.x % kWave) + 2;
+  const int group = __builtin_amdgcn_readfirstlane((local / g.recv_xb) * kRecvGroups +
+                                                   threadIdx.x / kWave);
+  if (x >= g.W - 2 || group * kRecvShort + 2 >= g.H - 2) return;
+  ShortRows v;
+  load_short(v, a.h_old + g.off, g.W, g.H, x, group);
+  decide_short(v, a.rcv + g.off, g.W, g.H, x, group, g.d_card, g.d_diag);
+}
+
+// tile_real: each tile's realization (tiles numbered across realizations).
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_ens_acc(EnsArgs a, const int32_t *__restrict__ tile_real,
+                                                   int ntiles) {
+  __shared__ AccShared sh;
+  const int b = ens_block();
+  if (b >= ntiles) return;
+  const int tile = xcd_tile(b, ntiles);
+  const int r = tile_real[tile];
+  int32_t *const q = a.rh + static_cast<size_t>(r) * kRH;
+  if (q[kRhDepth] > kHalo) return;   // no candidate: it takes the tile graph
+  const EnsReal &g = a.real[r];
+  const int over = tile_acc_body<BLOCK>(
+      sh, a.rcv + g.off, a.cnt + g.off, a.lvl + g.off, a.plan + tile, g.W, g.H,
+      tile - static_cast<int>(g.plan_off), g.tiles_x,
+      a.hist + static_cast<size_t>(r) * kHistLen, nullptr);
+  if (threadIdx.x == 0 && over) atomicAdd(&q[kRhOver], 1);
+}
+
+// The path of every realization this step; size[0..1] (and host_size, read by
+// the host once this launch has finished): the tile-graph work list's entries
+// and tiles.
+__global__ __launch_bounds__(kEnsBlock) void k_ens_lists(EnsArgs a, int32_t *tab_off,
+                                                         int32_t *tab_real, int32_t *size,
+                                                         int32_t *host_size) {
+  __shared__ uint32_t sh[kEnsBlock / kWave + 1];
+  for (int r = threadIdx.x; r < a.R; r += kEnsBlock) {
+    int32_t *const q = a.rh + static_cast<size_t>(r) * kRH;
+    int n[kHistLen], D = 0;
+#pragma unroll
+    for (int l = 0; l < kHistLen; l++) n[l] = a.hist[static_cast<size_t>(r) * kHistLen + l];
+#pragma unroll
+    for (int l = 0; l < kHistLen; l++) D = n[l] ? l : D;
+    if (q[kRhDepth] > kHalo || q[kRhOver] > 0) {
+      q[kRhPath] = 3;
+      q[kRhLevelSteps]++;
+    } else {
+      q[kRhDepth] = D;
+      q[kRhPath] = 1;
+      q[kRhTileSteps]++;
     }
   }
-  counter_barrier(&a.ctl[kCtlBarrier], bar, gridDim.x, a.ctl);
-  // ---- phase E: erosion -------------------------------------------------------
-  const int entries = ld_agent(&a.ctl[kCtlEntriesE]), nitems = ld_agent(&a.ctl[kCtlItemsE]);
-  for (;;) {
-    if (threadIdx.x == 0) s_item = atomicAdd(&a.ctl[kCtlClaim], 1);
-    __syncthreads();
-    const int item = s_item;
-    __syncthreads();
-    if (item >= nitems) break;
-    const int e = find_entry(a.tabE_off, entries + 1, item);
-    const int r = a.tabE_real[e];
-    const EnsReal &g = a.real[r];
-    int32_t *q = a.rh + static_cast<size_t>(r) * kRH;
-    const int j = item - a.tabE_off[e];
-    const int t1 = min(g.ntiles, (j + 1) * a.tiles_per_claim);
-    const ErodeConst ek = g.ek;
-    for (int tile = j * a.tiles_per_claim; tile < t1; tile++) {
-      with_nmode<NM>(g.nmode, [&](auto c) {
-        tile_erode_body<decltype(c)::value>(sh.ero, a.h_old + g.off, a.h_new + g.off,
-                                            a.plan + g.plan_off + tile, a.lvl + g.off,
-                                            a.cnt + g.off,
-                                            a.ftab + g.ftab_off, g.W, g.H, tile, g.tiles_x,
-                                            ek, q);
-      });
-      __syncthreads();
-    }
-    __syncthreads();
+  __syncthreads();
+  int entries, tiles;
+  list_entries(a.R, a.real, [&](int r) { return a.rh[static_cast<size_t>(r) * kRH + kRhPath] == 3; },
+               tab_off, tab_real, entries, tiles, sh);
+  if (threadIdx.x == 0) {
+    tab_off[entries] = tiles;
+    size[0] = entries;
+    size[1] = tiles;
+    __hip_atomic_store(&host_size[0], entries, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&host_size[1], tiles, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
-constexpr int kBarriersPerStep = 3;
+template <int NM>
+__global__ __launch_bounds__(kEroBlock) void k_ens_erode(EnsArgs a,
+                                                         const int32_t *__restrict__ tile_real,
+                                                         int ntiles) {
+  __shared__ EroShared sh;
+  const int b = ens_block();
+  if (b >= ntiles) return;
+  const int tile = xcd_tile(b, ntiles);
+  const int r = tile_real[tile];
+  int32_t *const q = a.rh + static_cast<size_t>(r) * kRH;
+  if (q[kRhPath] != 1) return;
+  const EnsReal &g = a.real[r];
+  const ErodeConst ek = g.ek;
+  with_nmode<NM>(g.nmode, [&](auto c) {
+    tile_erode_body<decltype(c)::value>(sh, a.h_old + g.off, a.h_new + g.off, a.plan + tile,
+                                        a.lvl + g.off, a.cnt + g.off, a.ftab + g.ftab_off, g.W,
+                                        g.H, tile - static_cast<int>(g.plan_off), g.tiles_x, ek, q);
+  });
+}
+
 
 }  // namespace
 
@@ -338,7 +244,7 @@ struct fs_ensemble {
   std::vector<int> to_internal;       // user index -> internal index
   std::vector<EnsReal> real;
   int nm_all = -1;                    // shared pow mode, -1 when mixed
-  int grid = 0;
+  int ncu = 0;
 
   EnsReal *real_d = nullptr;
   double *h[2] = {nullptr, nullptr};
@@ -347,10 +253,13 @@ struct fs_ensemble {
   TilePlan *plan = nullptr;
   int32_t *lev = nullptr;                     // per-level counts of tile-graph steps
   double *ftab = nullptr;
-  int32_t *rh = nullptr, *hist = nullptr, *ctl = nullptr;
-  int32_t *tabA_off = nullptr, *tabA_real = nullptr, *tabE_off = nullptr, *tabE_real = nullptr;
-  int32_t *tabG_off = nullptr, *tabG_real = nullptr;
+  int32_t *rh = nullptr, *hist = nullptr;
+  int32_t *recv_real = nullptr, *tile_real = nullptr;   // workgroup -> realization
+  int recv_blocks = 0;
+  int tiles = 0;                              // tiles of every realization
+  int32_t *tabG_off = nullptr, *tabG_real = nullptr, *tabG_size = nullptr;
   int32_t *graph_n_h = nullptr;               // pinned: the tile-graph work list's size
+  hipEvent_t listed = nullptr;                // the list of this step is there
   // the tile-graph step of the deep realizations (fs_deep.h)
   deep::GraphGrid *graph_grid = nullptr;
   uint32_t *dinfo = nullptr, *link = nullptr;
@@ -363,9 +272,7 @@ struct fs_ensemble {
   int32_t *thist = nullptr, *tcur = nullptr, *tstat = nullptr;
   int graph_blocks = 0, graph_queues = 1;
   uint64_t graph_tiles = 0;                   // tile-graph tiles stepped so far
-  std::map<int, int32_t *> recv_first;   // per recv_rows
   int cur = 0;
-  uint32_t bar_base = 0;
   fs_schedule sched{64, 1, 0};
   bool broken = false, have_step = false;
   uint64_t steps = 0;
@@ -389,10 +296,9 @@ void free_ensemble(fs_ensemble *e) {
                   static_cast<void *>(e->lvl), static_cast<void *>(e->cnt),
                   static_cast<void *>(e->plan), static_cast<void *>(e->lev),
                   static_cast<void *>(e->ftab), static_cast<void *>(e->rh),
-                  static_cast<void *>(e->hist), static_cast<void *>(e->ctl),
-                  static_cast<void *>(e->tabA_off), static_cast<void *>(e->tabA_real),
-                  static_cast<void *>(e->tabE_off), static_cast<void *>(e->tabE_real),
-                  static_cast<void *>(e->tabG_off), static_cast<void *>(e->tabG_real),
+                  static_cast<void *>(e->hist), static_cast<void *>(e->recv_real),
+                  static_cast<void *>(e->tile_real), static_cast<void *>(e->tabG_off),
+                  static_cast<void *>(e->tabG_real), static_cast<void *>(e->tabG_size),
                   static_cast<void *>(e->graph_grid), static_cast<void *>(e->dinfo),
                   static_cast<void *>(e->link), static_cast<void *>(e->node_word),
                   static_cast<void *>(e->items), static_cast<void *>(e->node_kids),
@@ -404,10 +310,9 @@ void free_ensemble(fs_ensemble *e) {
                   static_cast<void *>(e->tcur), static_cast<void *>(e->tstat)})
     if (p) (void)hipFree(p);
   if (e->graph_n_h) (void)hipHostFree(e->graph_n_h);
-  for (auto &kv : e->recv_first)
-    if (kv.second) (void)hipFree(kv.second);
   for (auto &ev : e->ev)
     if (ev) (void)hipEventDestroy(ev);
+  if (e->listed) (void)hipEventDestroy(e->listed);
   if (e->stream) (void)hipStreamDestroy(e->stream);
   delete e;
 }
@@ -426,47 +331,13 @@ int check_schedule(const fs_schedule &s) {
   if (s.recv_rows < kRecvRows || s.recv_rows > 256 || s.recv_rows % kRecvRows != 0 ||
       s.tiles_per_claim < 1 || s.tiles_per_claim > 16 || s.group_cells < 0)
     return FS_ERR_INVALID_ARGUMENT;
-  return FS_OK;   // group_cells is accepted and has no effect (no level path any more)
-}
-
-// Receiver work items of every realization for `rows` rows per item.
-int recv_table(fs_ensemble *e, int rows, const int32_t **out) {
-  auto it = e->recv_first.find(rows);
-  if (it == e->recv_first.end()) {
-    std::vector<int32_t> first(e->R + 1);
-    long long run = 0;
-    for (int r = 0; r < e->R; r++) {
-      first[r] = static_cast<int32_t>(run);
-      const EnsReal &g = e->real[r];
-      const long long strips = (g.H - 4 + kRecvRows - 1) / kRecvRows;
-      const long long per = rows / kRecvRows;
-      run += static_cast<long long>(g.recv_xb) * ((strips + per - 1) / per);
-    }
-    if (run >= (1ll << 31)) return FS_ERR_DIMENSIONS;
-    first[e->R] = static_cast<int32_t>(run);
-    int32_t *d = nullptr;
-    FS_TRY(fs::dev_alloc(&d, first.size()));
-    e->recv_first[rows] = d;
-    FS_HIP_TRY(hipMemcpy(d, first.data(), first.size() * sizeof(int32_t), hipMemcpyHostToDevice));
-    it = e->recv_first.find(rows);
-  }
-  *out = it->second;
   return FS_OK;
 }
 
-template <int NM>
-int launch_step_nm(fs_ensemble *e, const EnsArgs &a) {
-  EnsArgs args = a;
-  void *params[] = {&args};
-  FS_HIP_TRY(hipLaunchCooperativeKernel(reinterpret_cast<const void *>(&k_ens_step<NM>),
-                                        dim3(e->grid), dim3(kEnsBlock), params, 0, e->stream));
-  return FS_OK;
-}
-
-// The tile-graph step of the realizations the step kernel listed as deep
+// The tile-graph step of the realizations k_ens_lists listed as deep
 // (fs_deep.h), on the same stream.  The host reads the list's tile count
-// (one wait per step) so every per-tile kernel is launched with exactly one
-// workgroup per tile.
+// (one wait per step, while the erosion runs) so every per-tile kernel is
+// launched with exactly one workgroup per tile.
 template <int NM>
 int graph_launches(fs_ensemble *e, const deep::GraphWork &w, int T) {
   hipStream_t s = e->stream;
@@ -501,30 +372,32 @@ int graph_launches(fs_ensemble *e, const deep::GraphWork &w, int T) {
 }
 
 int graph_step(fs_ensemble *e) {
-  FS_HIP_TRY(hipMemcpyAsync(e->graph_n_h, e->ctl + kCtlGraph, 2 * sizeof(int32_t),
-                            hipMemcpyDeviceToHost, e->stream));
-  FS_HIP_TRY(hipStreamSynchronize(e->stream));
+  FS_HIP_TRY(hipEventSynchronize(e->listed));
   const int T = e->graph_n_h[1];
   if (T <= 0) return FS_OK;
   deep::GraphWork w;
   w.grid = e->graph_grid;
   w.first = e->tabG_off;
   w.which = e->tabG_real;
-  w.size = e->ctl + kCtlGraph;
+  w.size = e->tabG_size;
   e->graph_tiles += static_cast<uint64_t>(T);
   if (e->nm_all == 1) return graph_launches<1>(e, w, T);
   if (e->nm_all == 2) return graph_launches<2>(e, w, T);
   return graph_launches<-1>(e, w, T);
 }
 
-int launch_step(fs_ensemble *e) {
-  const int32_t *rf = nullptr;
-  FS_TRY(recv_table(e, e->sched.recv_rows, &rf));
+// A grid of at least n workgroups (a grid of one row holds fewer than 2^32
+// threads).
+dim3 ens_grid(int n) {
+  const unsigned x = std::min(static_cast<unsigned>(n), 1u << 20);
+  return dim3(x, (static_cast<unsigned>(n) + x - 1) / x);
+}
+
+int tile_launches(fs_ensemble *e) {
+  hipStream_t s = e->stream;
   EnsArgs a{};
   a.real = e->real_d;
   a.R = e->R;
-  a.recv_rows = e->sched.recv_rows;
-  a.tiles_per_claim = e->sched.tiles_per_claim;
   a.h_old = e->h[e->cur];
   a.h_new = e->h[e->cur ^ 1];
   a.rcv = e->rcv;
@@ -534,41 +407,48 @@ int launch_step(fs_ensemble *e) {
   a.ftab = e->ftab;
   a.rh = e->rh;
   a.hist = e->hist;
-  a.ctl = e->ctl;
-  a.recv_first = rf;
-  a.tabA_off = e->tabA_off;
-  a.tabA_real = e->tabA_real;
-  a.tabE_off = e->tabE_off;
-  a.tabE_real = e->tabE_real;
-  a.tabG_off = e->tabG_off;
-  a.tabG_real = e->tabG_real;
-  a.bar_base = e->bar_base;
-  int st;
-  if (e->nm_all == 1) st = launch_step_nm<1>(e, a);
-  else if (e->nm_all == 2) st = launch_step_nm<2>(e, a);
-  else st = launch_step_nm<-1>(e, a);
+  hipLaunchKernelGGL(k_ens_receivers, ens_grid(e->recv_blocks), dim3(256), 0, s, a,
+                     e->recv_real, e->recv_blocks);
+  // as for one grid: 1024-thread workgroups where there are fewer tiles than
+  // four per CU
+  if (e->tiles < 4 * e->ncu)
+    hipLaunchKernelGGL(k_ens_acc<kAccBlockWide>, ens_grid(e->tiles), dim3(kAccBlockWide), 0, s, a,
+                       e->tile_real, e->tiles);
+  else
+    hipLaunchKernelGGL(k_ens_acc<kAccBlock>, ens_grid(e->tiles), dim3(kAccBlock), 0, s, a,
+                       e->tile_real, e->tiles);
+  hipLaunchKernelGGL(k_ens_lists, dim3(1), dim3(kEnsBlock), 0, s, a, e->tabG_off, e->tabG_real,
+                     e->tabG_size, e->graph_n_h);
+  FS_HIP_TRY(hipEventRecord(e->listed, s));
+  if (e->nm_all == 1)
+    hipLaunchKernelGGL(k_ens_erode<1>, ens_grid(e->tiles), dim3(kEroBlock), 0, s, a, e->tile_real,
+                       e->tiles);
+  else if (e->nm_all == 2)
+    hipLaunchKernelGGL(k_ens_erode<2>, ens_grid(e->tiles), dim3(kEroBlock), 0, s, a, e->tile_real,
+                       e->tiles);
+  else
+    hipLaunchKernelGGL(k_ens_erode<-1>, ens_grid(e->tiles), dim3(kEroBlock), 0, s, a, e->tile_real,
+                       e->tiles);
+  FS_HIP_TRY(hipGetLastError());
+  return FS_OK;
+}
+
+int launch_step(fs_ensemble *e) {
+  int st = tile_launches(e);
   if (st == FS_OK) st = graph_step(e);
   if (st != FS_OK) {
     e->broken = true;
     return st;
   }
-  e->bar_base += static_cast<uint32_t>(kBarriersPerStep * e->grid);
   e->cur ^= 1;
   e->steps++;
   e->have_step = true;
   return FS_OK;
 }
 
-// Device error bits of every realization and the abort flag, after a sync.
+// Device error bits of every realization, after a sync.
 int ensemble_errors(fs_ensemble *e) {
   FS_HIP_TRY(hipStreamSynchronize(e->stream));
-  int32_t ctl[kCtlInts];
-  FS_HIP_TRY(hipMemcpy(ctl, e->ctl, sizeof(ctl), hipMemcpyDeviceToHost));
-  if (ctl[kCtlAbort]) {
-    e->broken = true;
-    fs::set_last_error("a grid barrier timed out");
-    return FS_ERR_INTERNAL;
-  }
   int32_t ts[deep::kStWords];
   FS_HIP_TRY(hipMemcpy(ts, e->tstat, sizeof(ts), hipMemcpyDeviceToHost));
   if (ts[deep::kStErr]) {
@@ -725,13 +605,8 @@ int fs_ensemble_create(const fs_realization *reals, int count, int device, fs_en
   e->device = device;
   e->R = count;
   FS_HIP_TRY(hipSetDevice(device));
-  int coop = 0;
-  FS_HIP_TRY(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, device));
-  if (!coop) {
-    fs::set_last_error("device does not support cooperative launches");
-    return FS_ERR_NO_DEVICE;
-  }
-  // largest realizations first: the erosion list starts with them
+  FS_HIP_TRY(hipDeviceGetAttribute(&e->ncu, hipDeviceAttributeMultiprocessorCount, device));
+  // largest realizations first
   std::vector<int> ord(count);
   std::iota(ord.begin(), ord.end(), 0);
   std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) {
@@ -743,6 +618,7 @@ int fs_ensemble_create(const fs_realization *reals, int count, int device, fs_en
   e->real.resize(count);
   size_t cells = 0, ftab_n = 0, lev_n = 0;
   int nm0 = -2;
+  long long recv_total = 0;   // receiver workgroups
   for (int i = 0; i < count; i++) {
     const fs_realization &s = reals[ord[i]];
     e->to_internal[ord[i]] = i;
@@ -754,7 +630,13 @@ int fs_ensemble_create(const fs_realization *reals, int count, int device, fs_en
     g.H = s.height;
     g.tiles_x = (s.width + kTile - 1) / kTile;
     g.ntiles = g.tiles_x * ((s.height + kTile - 1) / kTile);
-    g.recv_xb = (s.width - 4 + kRecvLanes - 1) / kRecvLanes;
+    g.recv_xb = (s.width - 4 + kWave - 1) / kWave;
+    const int groups = (s.height - 4 + kRecvShort - 1) / kRecvShort;
+    const long long blocks =
+        static_cast<long long>(g.recv_xb) * ((groups + kRecvGroups - 1) / kRecvGroups);
+    if (recv_total + blocks >= (1ll << 31)) return FS_ERR_DIMENSIONS;
+    g.recv_first = static_cast<int>(recv_total);
+    recv_total += blocks;
     g.d_card = s.params.dx;
     g.d_diag = s.params.dx * fs::kSqrt2;
     g.ek = make_erode_const(s.params, &g.nmode);
@@ -774,9 +656,12 @@ int fs_ensemble_create(const fs_realization *reals, int count, int device, fs_en
     tiles_total += g.ntiles;
   }
   if (tiles_total >= (1ll << 31)) return FS_ERR_DIMENSIONS;
+  e->tiles = static_cast<int>(tiles_total);
+  e->recv_blocks = static_cast<int>(recv_total);
 
   FS_HIP_TRY(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking));
   for (auto &ev : e->ev) FS_HIP_TRY(hipEventCreate(&ev));
+  FS_HIP_TRY(hipEventCreateWithFlags(&e->listed, hipEventDisableTiming));
   FS_TRY(fs::dev_alloc(&e->real_d, count));
   FS_TRY(fs::dev_alloc(&e->h[0], cells));
   FS_TRY(fs::dev_alloc(&e->h[1], cells));
@@ -788,13 +673,33 @@ int fs_ensemble_create(const fs_realization *reals, int count, int device, fs_en
   FS_TRY(fs::dev_alloc(&e->ftab, ftab_n));
   FS_TRY(fs::dev_alloc(&e->rh, static_cast<size_t>(count) * kRH));
   FS_TRY(fs::dev_alloc(&e->hist, static_cast<size_t>(count) * kHistLen));
-  FS_TRY(fs::dev_alloc(&e->ctl, kCtlInts));
-  FS_TRY(fs::dev_alloc(&e->tabA_off, count + 1));
-  FS_TRY(fs::dev_alloc(&e->tabA_real, count + 1));
-  FS_TRY(fs::dev_alloc(&e->tabE_off, count + 1));
-  FS_TRY(fs::dev_alloc(&e->tabE_real, count + 1));
+  FS_TRY(fs::dev_alloc(&e->recv_real, static_cast<size_t>(recv_total)));
+  FS_TRY(fs::dev_alloc(&e->tile_real, static_cast<size_t>(tiles_total)));
+  {
+    std::vector<int32_t> of;
+    try {
+      of.resize(static_cast<size_t>(std::max(recv_total, tiles_total)));
+    } catch (const std::bad_alloc &) {
+      return FS_ERR_OUT_OF_MEMORY;
+    }
+    for (int r = 0; r < count; r++) {
+      const EnsReal &g = e->real[r];
+      const long long end = r + 1 < count ? e->real[r + 1].recv_first : recv_total;
+      std::fill(of.begin() + g.recv_first, of.begin() + static_cast<std::ptrdiff_t>(end), r);
+    }
+    FS_HIP_TRY(hipMemcpy(e->recv_real, of.data(), static_cast<size_t>(recv_total) * sizeof(int32_t),
+                         hipMemcpyHostToDevice));
+    for (int r = 0; r < count; r++) {
+      const EnsReal &g = e->real[r];
+      std::fill_n(of.begin() + static_cast<std::ptrdiff_t>(g.plan_off), g.ntiles, r);
+    }
+    FS_HIP_TRY(hipMemcpy(e->tile_real, of.data(),
+                         static_cast<size_t>(tiles_total) * sizeof(int32_t),
+                         hipMemcpyHostToDevice));
+  }
   FS_TRY(fs::dev_alloc(&e->tabG_off, count + 1));
   FS_TRY(fs::dev_alloc(&e->tabG_real, count + 1));
+  FS_TRY(fs::dev_alloc(&e->tabG_size, 2));
   // the tile-graph step (deep realizations): the realizations' tiles are
   // numbered by plan_off, so the per-tile arrays cover every tile
   {
@@ -853,7 +758,6 @@ int fs_ensemble_create(const fs_realization *reals, int count, int device, fs_en
   FS_HIP_TRY(hipMemset(e->cnt, 0, cells * sizeof(uint32_t)));
   FS_HIP_TRY(hipMemset(e->rh, 0, static_cast<size_t>(count) * kRH * sizeof(int32_t)));
   FS_HIP_TRY(hipMemset(e->hist, 0, static_cast<size_t>(count) * kHistLen * sizeof(int32_t)));
-  FS_HIP_TRY(hipMemset(e->ctl, 0, kCtlInts * sizeof(int32_t)));
 
   // Initial terrains and erosion factor tables.  Host threads fill host
   // buffers, one realization each per round; this thread alone makes every
@@ -900,28 +804,10 @@ int fs_ensemble_create(const fs_realization *reals, int count, int device, fs_en
     }
   }
 
-  int per_cu = 0;
-  hipError_t oe;
-  if (e->nm_all == 1)
-    oe = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_ens_step<1>, kEnsBlock, 0);
-  else if (e->nm_all == 2)
-    oe = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_ens_step<2>, kEnsBlock, 0);
-  else
-    oe = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_ens_step<-1>, kEnsBlock, 0);
-  FS_HIP_TRY(oe);
-  int ncu = 0;
-  FS_HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device));
-  if (per_cu < 1 || ncu < 1) {
-    fs::set_last_error("the step kernel does not fit on a CU");
-    return FS_ERR_INTERNAL;
-  }
-  e->grid = per_cu * ncu;
-  e->graph_blocks = e->nm_all == 1   ? deep::erode_grid<1>(ncu)
-                    : e->nm_all == 2 ? deep::erode_grid<2>(ncu)
-                                     : deep::erode_grid<-1>(ncu);
+  e->graph_blocks = e->nm_all == 1   ? deep::erode_grid<1>(e->ncu)
+                    : e->nm_all == 2 ? deep::erode_grid<2>(e->ncu)
+                                     : deep::erode_grid<-1>(e->ncu);
   e->graph_queues = deep::erode_queues(e->graph_blocks);
-  const int32_t *rf = nullptr;
-  FS_TRY(recv_table(e, e->sched.recv_rows, &rf));
   FS_HIP_TRY(hipDeviceSynchronize());
   guard.e = nullptr;
   *out = e;
@@ -1056,8 +942,6 @@ int fs_ensemble_set_schedule(fs_ensemble *e, const fs_schedule *s) {
   FS_TRY(check_ensemble(e));
   if (!s) return FS_ERR_INVALID_ARGUMENT;
   FS_TRY(check_schedule(*s));
-  const int32_t *rf = nullptr;
-  FS_TRY(recv_table(e, s->recv_rows, &rf));
   e->sched = *s;
   return FS_OK;
 }
@@ -1074,10 +958,6 @@ int fs_ensemble_autotune(fs_ensemble *e, int trial_steps, int interval) {
   e->tune_trial = trial_steps;
   e->tune_interval = interval;
   e->tuned_at = ~0ull;
-  if (trial_steps > 0) {
-    const int32_t *rf = nullptr;
-    for (int rows : {16, 64, 256}) FS_TRY(recv_table(e, rows, &rf));
-  }
   return FS_OK;
 }
 

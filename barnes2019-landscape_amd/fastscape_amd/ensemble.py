@@ -1,4 +1,4 @@
-"""Ensembles: many FastScape grids stepped by one persistent launch per step.
+"""Ensembles: many FastScape grids stepped together.
 
 Binding of the fs_ensemble_* entry points of include/fastscape.h.  Each
 realization has its own size, parameter block (fs_params, RB:58-65) and

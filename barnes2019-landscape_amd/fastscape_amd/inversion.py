@@ -5,7 +5,7 @@ reference's, fastscape_RB.cpp:366-376) from a known initial terrain with
 hidden (K, U, m); find the candidate set whose exact result fits it best.
 
 * exact-only search: every candidate runs through the exact solver (batched
-  in ensembles, one persistent launch per step) and the best misfit wins;
+  in ensembles) and the best misfit wins;
 * proposal search: the U-Net predicts each candidate's topography, the
   candidates are ranked by predicted misfit, and only the top few run
   through the exact solver, which picks the winner -- the exact solver stays

@@ -265,7 +265,7 @@ int fs_calibrate_copy(size_t nbytes, int device, double *ms);
 
 /* ---- ensembles --------------------------------------------------------------
  * Many independent grids ("realizations") of different sizes and parameters,
- * advanced together by one persistent cooperative launch per time-step.  No
+ * advanced together, each kernel of a time-step launched once for all.  No
  * reference counterpart: the reference runs one grid per process; its README
  * motivates ensembles for inverse problems (README.md:28-29).  Each
  * realization's time-step is the reference's (RB:366-376) and gives the same
@@ -279,13 +279,11 @@ typedef struct fs_realization {
   uint32_t engine_seed;
 } fs_realization;
 
-/* Work schedule of a step; every schedule gives the same results.
- *   recv_rows        rows of 256 columns per receiver work item (16..256,
- *                    a multiple of 16)
- *   tiles_per_claim  64x64 tiles per erosion work item (1..16)
- *   group_cells      accepted (>= 0) and without effect: deep realizations
- *                    take the tile-graph step, whose work spreads over every
- *                    CU */
+/* Work schedule of a step.  The fields are checked and kept and have no
+ * effect: the work is laid out by the realizations' sizes.
+ *   recv_rows        16..256, a multiple of 16
+ *   tiles_per_claim  1..16
+ *   group_cells      >= 0 */
 typedef struct fs_schedule {
   int recv_rows;
   int tiles_per_claim;
