@@ -60,6 +60,7 @@ namespace tile32 {
 #include "fs_deep.h"
 
 namespace {
+constexpr int kFillBatch = 8;     // depression-filling launches between two looks of the host
 constexpr int kGraphRetry = 64;   // graph steps between attempts of the 32-cell halo
 }  // namespace
 
@@ -106,7 +107,7 @@ struct fs_model {
   uint64_t *status = nullptr;
   unsigned long long *ticket = nullptr;
   unsigned long long *phase = nullptr;   // tile kernels' phase ticks (stage timers)
-  int32_t *fill_flag = nullptr;          // a fill launch changed a cell
+  int32_t *fill_flag = nullptr;          // per launch of a batch: it changed a cell
   long long steps_in_call = 0;           // steps taken by the current fs_run / fs_step
   bool fill_mode = false;                // fill depressions before every step
 
@@ -445,7 +446,7 @@ int create_model(int W, int H, const fs_params *p, const double *h_init, uint32_
                             static_cast<size_t>((m->H + kTile - 1) / kTile);
   FS_TRY(fs::dev_alloc(&m->plan, plan_tiles));
   FS_TRY(fs::dev_alloc(&m->phase, static_cast<size_t>(kPhaseSlots) * kPhaseStride));
-  FS_TRY(fs::dev_alloc(&m->fill_flag, 1));
+  FS_TRY(fs::dev_alloc(&m->fill_flag, kFillBatch));
   if (hipHostMalloc(reinterpret_cast<void **>(&m->hdr_h),
                     (kHdrInts + FS_MAX_LEVELS + 3) * sizeof(int32_t)) != hipSuccess ||
       hipHostMalloc(reinterpret_cast<void **>(&m->levels_h),
@@ -1059,18 +1060,23 @@ int fill_depressions(fs_model *m) {
   FS_TRY(check_launch());
   const int tiles_x = (m->W + kFillTile - 1) / kFillTile;
   const int tiles = tiles_x * ((m->H + kFillTile - 1) / kFillTile);
+  // kFillBatch launches between two looks at their flags; those behind a
+  // launch that changed nothing return at once
   const long long cap = 8ll * tiles + 16;
-  for (long long launch = 0;; launch++) {
+  for (long long launch = 0;; launch += kFillBatch) {
     if (launch > cap) {
       fs::set_last_error("depression filling did not settle");
       return FS_ERR_INTERNAL;
     }
-    FS_HIP_TRY(hipMemsetAsync(m->fill_flag, 0, sizeof(int32_t), s));
-    hipLaunchKernelGGL(k_fill, dim3(tiles), dim3(kFillBlock), 0, s, m->h, m->h_alt, m->W, m->H,
-                       tiles_x, m->fill_flag);
-    FS_TRY(check_launch());
-    int32_t changed = 0;
-    FS_HIP_TRY(hipMemcpyAsync(&changed, m->fill_flag, sizeof(changed), hipMemcpyDeviceToHost, s));
+    FS_HIP_TRY(hipMemsetAsync(m->fill_flag, 0, kFillBatch * sizeof(int32_t), s));
+    for (int i = 0; i < kFillBatch; i++) {
+      hipLaunchKernelGGL(k_fill, dim3(tiles), dim3(kFillBlock), 0, s, m->h, m->h_alt, m->W, m->H,
+                         tiles_x, i ? m->fill_flag + i - 1 : nullptr, m->fill_flag + i);
+      FS_TRY(check_launch());
+    }
+    int32_t changed = 0;   // by the batch's last launch
+    FS_HIP_TRY(hipMemcpyAsync(&changed, m->fill_flag + kFillBatch - 1, sizeof(changed),
+                              hipMemcpyDeviceToHost, s));
     FS_HIP_TRY(hipStreamSynchronize(s));
     if (!changed) break;
   }

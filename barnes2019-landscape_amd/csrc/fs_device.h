@@ -778,8 +778,9 @@ __global__ __launch_bounds__(kSmallBlock) void k_erode_small(
 // values.
 constexpr int kFillTile = 64;
 constexpr int kFillReg = kFillTile + 2;
-constexpr int kFillBlock = 256;
-constexpr int kFillSweeps = 512;          // local sweeps per launch at most
+constexpr int kFillBlock = 1024;
+constexpr int kFillInner = 6;             // a wave's relaxations between two votes of the block
+constexpr int kFillVotes = 4096;          // votes per launch at most
 
 // nextafter(x, +inf) for IEEE doubles.
 __device__ __forceinline__ double next_up(double x) {
@@ -787,6 +788,14 @@ __device__ __forceinline__ double next_up(double x) {
   if (x == 0.0) return 0x1p-1074;                      // +-0 -> smallest subnormal
   const long long u = __double_as_longlong(x);
   return __longlong_as_double(x > 0.0 ? u + 1 : u - 1);
+}
+
+// v_min_f64 as it is, without the instruction per operand that fmin spends on
+// quieting signalling NaNs (k_fill quiets what it loads, once)
+__device__ __forceinline__ double raw_min(double a, double b) {
+  double r;
+  asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
 }
 
 // F = h on rings 0 and 1, +inf inside.
@@ -800,71 +809,164 @@ __global__ __launch_bounds__(256) void k_fill_init(const double *__restrict__ h,
   }
 }
 
+// One tile: relaxed to its fixed point in LDS, its border published and the
+// neighbours' borders read again, until such a read brings nothing new.
+//
+// A flood path runs cell by cell and values are corrected several times on
+// the way, so the time is a chain of relaxations.  Each wave owns a patch of 16
+// x 16 cells and relaxes 2 x 2 of them per lane from LDS, up to kFillInner
+// times between two votes of the workgroup, with no barrier in between: values
+// only fall, and any order ends at the same fixed point.  A wave whose patch
+// and whose neighbours have no news rests, which leaves LDS to the others.
+// 256 threads with 16 strided cells each and three barriers a sweep took 266
+// us per launch on a random 700 x 501 terrain and 7.9 ms for the fill; this
+// takes 2.5 (5.0 ms against 16.5 at 1000^2, 14.0 against 37.4 at 3000 x 2000).
+// Two relaxations between votes: 3.2 ms, 16: 2.7; waiting in the launch for
+// further news (40 more reads): 3.0.
 __global__ __launch_bounds__(kFillBlock) void k_fill(const double *__restrict__ h, double *F,
                                                      int W, int H, int tiles_x,
-                                                     int32_t *changed) {
+                                                     const int32_t *before, int32_t *changed) {
+  // the launch before found every tile settled
+  if (before != nullptr && *before == 0) return;
   __shared__ double f_s[kFillReg * kFillReg];
-  __shared__ int s_more, s_any;
-  constexpr int kPer = kFillTile * kFillTile / kFillBlock;
+  __shared__ uint32_t dirty;   // patches with news, one bit per wave
   const int x0 = (blockIdx.x % tiles_x) * kFillTile, y0 = (blockIdx.x / tiles_x) * kFillTile;
-  for (int i = threadIdx.x; i < kFillReg * kFillReg; i += kFillBlock) {
-    const int gx = x0 - 1 + i % kFillReg, gy = y0 - 1 + i / kFillReg;
-    f_s[i] = (gx >= 0 && gx < W && gy >= 0 && gy < H)
-                 ? __hip_atomic_load(&F[static_cast<size_t>(gy) * W + gx], __ATOMIC_RELAXED,
-                                     __HIP_MEMORY_SCOPE_AGENT)
-                 : __builtin_huge_val();
-  }
-  double hv[kPer];
-  bool inner[kPer];
+  if (threadIdx.x == 0) dirty = 0xFFFFu;
+  auto load_f = [&](int gx, int gy) {
+    return (gx >= 0 && gx < W && gy >= 0 && gy < H)
+               ? __builtin_canonicalize(__hip_atomic_load(&F[static_cast<size_t>(gy) * W + gx],
+                                                          __ATOMIC_RELAXED,
+                                                          __HIP_MEMORY_SCOPE_AGENT))
+               : __builtin_huge_val();
+  };
+  for (int i = threadIdx.x; i < kFillReg * kFillReg; i += kFillBlock)
+    f_s[i] = load_f(x0 - 1 + i % kFillReg, y0 - 1 + i / kFillReg);
+  // this lane's 2 x 2 cells
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  const int lx = (wave % 4) * 16 + (lane % 8) * 2, ly = (wave / 4) * 16 + (lane / 8) * 2;
+  double hv[2][2];
+  bool inner[2][2];
 #pragma unroll
-  for (int k = 0; k < kPer; k++) {
-    const int i = k * kFillBlock + threadIdx.x;
-    const int gx = x0 + i % kFillTile, gy = y0 + i / kFillTile;
-    inner[k] = gx >= 2 && gx < W - 2 && gy >= 2 && gy < H - 2;
-    hv[k] = inner[k] ? h[static_cast<size_t>(gy) * W + gx] : 0.0;
-  }
-  if (threadIdx.x == 0) s_any = 0;
-  __syncthreads();
-  for (int sweep = 0; sweep < kFillSweeps; sweep++) {
-    if (threadIdx.x == 0) s_more = 0;
-    __syncthreads();
-    int more = 0;
+  for (int j = 0; j < 2; j++)
 #pragma unroll
-    for (int k = 0; k < kPer; k++) {
-      if (!inner[k]) continue;
-      const int i = k * kFillBlock + threadIdx.x;
-      const int r = (i / kFillTile + 1) * kFillReg + i % kFillTile + 1;
-      double m = f_s[r - kFillReg - 1];
-      m = fmin(m, f_s[r - kFillReg]);
-      m = fmin(m, f_s[r - kFillReg + 1]);
-      m = fmin(m, f_s[r - 1]);
-      m = fmin(m, f_s[r + 1]);
-      m = fmin(m, f_s[r + kFillReg - 1]);
-      m = fmin(m, f_s[r + kFillReg]);
-      m = fmin(m, f_s[r + kFillReg + 1]);
-      const double v = fmax(hv[k], next_up(m));
-      if (v < f_s[r]) {
-        f_s[r] = v;
-        more = 1;
-      }
+    for (int i = 0; i < 2; i++) {
+      const int gx = x0 + lx + i, gy = y0 + ly + j;
+      inner[j][i] = gx >= 2 && gx < W - 2 && gy >= 2 && gy < H - 2;
+      hv[j][i] = inner[j][i] ? h[static_cast<size_t>(gy) * W + gx] : 0.0;
     }
-    if (more) s_more = 1;
-    __syncthreads();
-    const int go = s_more;
-    if (go && threadIdx.x == 0) s_any = 1;
-    __syncthreads();
-    if (!go) break;
+  // the halo cell this thread looks after: the ring around the tile
+  constexpr int kRing = 4 * kFillReg - 4;
+  static_assert(kRing <= kFillBlock, "one halo cell per thread");
+  int halo = -1, hx = 0, hy = 0;
+  if (static_cast<int>(threadIdx.x) < kRing) {
+    const int q = threadIdx.x;
+    if (q < kFillReg) {
+      hx = q;
+    } else if (q < 2 * kFillReg) {
+      hx = q - kFillReg;
+      hy = kFillReg - 1;
+    } else {
+      hx = q < 3 * kFillReg - 2 ? 0 : kFillReg - 1;
+      hy = (q - 2 * kFillReg) % (kFillReg - 2) + 1;
+    }
+    halo = hy * kFillReg + hx;
   }
-  if (!s_any) return;
+  const bool border = lx == 0 || ly == 0 || lx + 2 == kFillTile || ly + 2 == kFillTile;
+  auto ld = [&](int i) {
+    return __hip_atomic_load(&f_s[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  };
+  const int c0 = (ly + 1) * kFillReg + lx + 1;
+  // the patches around this wave's
+  uint32_t around = 0;
 #pragma unroll
-  for (int k = 0; k < kPer; k++) {
-    if (!inner[k]) continue;
-    const int i = k * kFillBlock + threadIdx.x;
-    const int gx = x0 + i % kFillTile, gy = y0 + i / kFillTile;
-    const int r = (i / kFillTile + 1) * kFillReg + i % kFillTile + 1;
-    __hip_atomic_store(&F[static_cast<size_t>(gy) * W + gx], f_s[r], __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
+  for (int j = -1; j < 2; j++)
+#pragma unroll
+    for (int i = -1; i < 2; i++) {
+      const int px = wave % 4 + i, py = wave / 4 + j;
+      if ((i || j) && px >= 0 && px < 4 && py >= 0 && py < 4) around |= 1u << (4 * py + px);
+    }
+  // one relaxation of the lane's cells; true when one of them fell
+  auto relax = [&]() {
+    double f[4][4];
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) f[j][i] = f_s[c0 + (j - 1) * kFillReg + i - 1];
+    bool fell = false;
+#pragma unroll
+    for (int j = 1; j < 3; j++)
+#pragma unroll
+      for (int i = 1; i < 3; i++) {
+        const double a = raw_min(raw_min(f[j - 1][i - 1], f[j - 1][i]), f[j - 1][i + 1]);
+        const double b = raw_min(raw_min(f[j + 1][i - 1], f[j + 1][i]), f[j + 1][i + 1]);
+        const double m = raw_min(raw_min(a, b), raw_min(f[j][i - 1], f[j][i + 1]));
+        const double v = fmax(hv[j - 1][i - 1], next_up(m));
+        if (inner[j - 1][i - 1] && v < f[j][i]) {
+          f[j][i] = v;
+          fell = true;
+          f_s[c0 + (j - 1) * kFillReg + i - 1] = v;
+        }
+      }
+    asm volatile("" ::: "memory");   // the next relaxation reads LDS again
+    return fell;
+  };
+  auto store_cells = [&]() {
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+        if (inner[j][i])
+          __hip_atomic_store(&F[static_cast<size_t>(y0 + ly + j) * W + x0 + lx + i],
+                             ld(c0 + j * kFillReg + i), __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT);
+  };
+  // the neighbours' cell this thread looks after, read again; its news wakes
+  // the patches it touches
+  auto halo_news = [&]() {
+    if (halo < 0) return 0;
+    const double v = load_f(x0 - 1 + hx, y0 - 1 + hy);
+    if (!(v < ld(halo))) return 0;
+    __hip_atomic_store(&f_s[halo], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    uint32_t wake = 0;
+    for (int j = -1; j < 2; j++)
+      for (int i = -1; i < 2; i++) {
+        const int cx = hx - 1 + i, cy = hy - 1 + j;
+        if (cx >= 0 && cx < kFillTile && cy >= 0 && cy < kFillTile)
+          wake |= 1u << (4 * (cy / 16) + cx / 16);
+      }
+    atomicOr(&dirty, wake);
+    return 1;
+  };
+  bool ever = false;        // block-uniform: a cell fell in this launch
+  __syncthreads();
+  for (int votes = 0; votes < kFillVotes;) {
+    bool moved = false;     // block-uniform: since the last publication
+    for (; votes < kFillVotes; votes++) {
+      // a wave rests while neither it nor a patch around it has news
+      int fell = 0;
+      uint32_t mine = 0;
+      if (lane == 0) mine = atomicAnd(&dirty, ~(1u << wave)) >> wave & 1u;
+      if (__builtin_amdgcn_readfirstlane(mine)) {
+        bool now = true;
+        for (int k = 0; k < kFillInner && __any(now); k++) {
+          now = relax();
+          fell |= now ? 1 : 0;
+        }
+        const uint32_t wake = (__any(fell) ? around : 0u) | (__any(now) ? 1u << wave : 0u);
+        if (wake != 0 && lane == 0) atomicOr(&dirty, wake);
+      }
+      if (!__syncthreads_or(fell)) break;
+      moved = true;
+    }
+    if (moved) {
+      ever = true;
+      if (border) store_cells();
+    }
+    votes++;
+    if (!__syncthreads_or(halo_news())) break;
   }
+  if (!ever) return;
+  store_cells();
   if (threadIdx.x == 0) atomicOr(changed, 1);
 }
 
