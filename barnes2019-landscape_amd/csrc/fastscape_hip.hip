@@ -908,11 +908,10 @@ int ensure_graph(fs_model *m) {
   const size_t tiles = static_cast<size_t>((m->W + deep::kSide - 1) / deep::kSide) *
                        static_cast<size_t>((m->H + deep::kSide - 1) / deep::kSide);
   const size_t nodes = tiles * deep::kNodeCap;
-  int ncu = 0;
-  FS_HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, m->device));
-  m->graph_blocks = m->nmode == 1   ? deep::erode_grid<1>(ncu)
-                    : m->nmode == 2 ? deep::erode_grid<2>(ncu)
-                                    : deep::erode_grid<0>(ncu);
+  FS_HIP_TRY(hipDeviceGetAttribute(&m->ncu, hipDeviceAttributeMultiprocessorCount, m->device));
+  m->graph_blocks = m->nmode == 1   ? deep::erode_grid<1>(m->ncu)
+                    : m->nmode == 2 ? deep::erode_grid<2>(m->ncu)
+                                    : deep::erode_grid<0>(m->ncu);
   m->graph_queues = deep::erode_queues(m->graph_blocks);
   FS_TRY(fs::dev_alloc(&m->dinfo, N));
   FS_TRY(fs::dev_alloc(&m->link, N));
@@ -962,12 +961,12 @@ deep::GraphWork graph_work(fs_model *m) {
 
 // The counts' completion with the erosion of the root-tailed cells, then the
 // persistent erosion of the other tiers.
-template <int NMODE>
+template <int NMODE, bool kChain>
 int launch_graph_erosion(fs_model *m, int tiles) {
   hipStream_t s = m->stream;
   const deep::GraphWork w = graph_work(m);
   FS_TRY(kt_begin(m, FS_K_GRAPH_COUNTS));
-  hipLaunchKernelGGL(deep::k_deep_counts<NMODE>, dim3(tiles), dim3(deep::kCntBlock), 0, s, w, m->rcv,
+  hipLaunchKernelGGL((deep::k_deep_counts<NMODE, kChain>), dim3(tiles), dim3(deep::kCntBlock), 0, s, w, m->rcv,
                      m->cnt, m->dinfo, m->link, m->node_out, m->node_cell, m->node_tier,
                      m->nexit, m->tile_n0, m->cells, m->tcur, m->items, m->ftab, m->h, m->h_alt);
   FS_TRY(check_launch());
@@ -1018,9 +1017,11 @@ int graph_path(fs_model *m, const hipEvent_t *ev) {
   FS_TRY(kt_end(m));
   FS_TRY(mark(ev[4], s));
   FS_TRY(mark(ev[5], s));
-  if (m->nmode == 1) FS_TRY(launch_graph_erosion<1>(m, tiles));
-  else if (m->nmode == 2) FS_TRY(launch_graph_erosion<2>(m, tiles));
-  else FS_TRY(launch_graph_erosion<0>(m, tiles));
+  if (m->nmode == 1) FS_TRY((launch_graph_erosion<1, false>(m, tiles)));
+  else if (m->nmode == 2 && deep::counts_chain(tiles, m->ncu))
+    FS_TRY((launch_graph_erosion<2, true>(m, tiles)));
+  else if (m->nmode == 2) FS_TRY((launch_graph_erosion<2, false>(m, tiles)));
+  else FS_TRY((launch_graph_erosion<0, false>(m, tiles)));
   std::swap(m->h, m->h_alt);
   m->order_current = false;                 // levels, stack, donor masks on request
   m->cnt_stack = false;

@@ -216,16 +216,30 @@ __device__ __forceinline__ WorkTile work_tile(const GraphWork &w, int wi) {
   return r;
 }
 
-// The Newton solve in the grid's pow mode (NMODE < 0: chosen per grid).
+// The Newton solve in the grid's pow mode (NMODE < 0: chosen per grid), and
+// what it can do before the receiver is known.  kChain: for waves that wait
+// mostly for each other (newton_solve).  Else n = 2 takes the plain loop, which
+// is no slower where the vector units are busy: it stops at each lane's last
+// iteration, and its divisions' extra instructions are scalar ones by half.
 template <int NMODE>
-__device__ __forceinline__ double solve(int nm, double h0, double hn, double fact,
-                                        const ErodeConst &k, int32_t *hdr) {
+__device__ __forceinline__ NewtonPrep prepare(int nm, double h0, double fact, const ErodeConst &k) {
   if constexpr (NMODE >= 0) {
-    return newton_update<NMODE>(h0, hn, fact, k, hdr);
+    return newton_prep<NMODE>(h0, fact, k);
   } else {
-    if (nm == 1) return newton_update<1>(h0, hn, fact, k, hdr);
-    if (nm == 2) return newton_update<2>(h0, hn, fact, k, hdr);
-    return newton_update<0>(h0, hn, fact, k, hdr);
+    return nm == 1 ? newton_prep<1>(h0, fact, k) : newton_prep<2>(h0, fact, k);
+  }
+}
+template <int NMODE, bool kChain>
+__device__ __forceinline__ double solve(int nm, double h0, double hn, double fact,
+                                        const NewtonPrep &p, const ErodeConst &k, int32_t *hdr) {
+  if constexpr (NMODE == 1 || (NMODE == 2 && kChain)) {
+    return newton_solve<NMODE>(h0, hn, fact, p, k, hdr);
+  } else if constexpr (NMODE >= 0) {
+    return newton_plain<NMODE>(h0, hn, fact, k, hdr);
+  } else {
+    if (nm == 1) return solve<1, kChain>(nm, h0, hn, fact, p, k, hdr);
+    if (nm == 2) return solve<2, kChain>(nm, h0, hn, fact, p, k, hdr);
+    return solve<0, kChain>(nm, h0, hn, fact, p, k, hdr);
   }
 }
 
@@ -751,7 +765,7 @@ __device__ __forceinline__ int tier_rank(const int *sorted, int n, int tier) {
   return lo;
 }
 
-template <int NMODE>
+template <int NMODE, bool kChain>
 __global__ __launch_bounds__(kCntBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_deep_counts(
     GraphWork w, const uint8_t *__restrict__ rcv0, uint32_t *__restrict__ cnt0,
     const uint32_t *__restrict__ dinfo0, const uint32_t *__restrict__ link0,
@@ -1017,27 +1031,31 @@ __global__ __launch_bounds__(kCntBlock) __attribute__((amdgpu_waves_per_eu(6))) 
     const double fact = fnext;
     if (c + 1 < kCntPer && ci[c + 1] >= 0) fnext = fact_of(ci[c + 1]);
     const double h0 = h0s[c];
-    int spins = 0;
-    for (;;) {
-      const uint64_t rb = root ? 0
-                               : __hip_atomic_load(&hbits[ri], __ATOMIC_RELAXED,
-                                                   __HIP_MEMORY_SCOPE_WORKGROUP);
-      const bool ready = root || rb != kUnsolved;
-      const bool give_up = !ready && ++spins > kSpinCap;
-      if (ready || give_up) {
-        double hn = h0;
-        if (give_up) {
-          atomicOr(&hdr[2], kErrLookback);
-        } else if (root) {
-          const int gx = b.x0 + i % kSide, gy = b.y0 + i / kSide;
-          if (gx >= 2 && gx < W - 2 && gy >= 2 && gy < H - 2) hn += k.ud;
-        } else {
-          hn = solve<NMODE>(G.nmode, h0 + k.ud, __longlong_as_double(static_cast<long long>(rb)),
-                            fact, k, hdr);
+    const NewtonPrep prep = prepare<NMODE>(G.nmode, h0 + k.ud, fact, k);
+    // a wave-uniform loop: a lane publishes in the pass that solves it
+    bool open = true;
+    for (int spins = 0; __ballot(open) != 0; spins++) {
+      if (open) {
+        const uint64_t rb = root ? 0
+                                 : __hip_atomic_load(&hbits[ri], __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_WORKGROUP);
+        const bool ready = root || rb != kUnsolved, give_up = spins >= kSpinCap;
+        if (ready || give_up) {
+          open = false;
+          double hn = h0;
+          if (!ready) {
+            atomicOr(&hdr[2], kErrLookback);
+          } else if (root) {
+            const int gx = b.x0 + i % kSide, gy = b.y0 + i / kSide;
+            if (gx >= 2 && gx < W - 2 && gy >= 2 && gy < H - 2) hn += k.ud;
+          } else {
+            hn = solve<NMODE, kChain>(G.nmode, h0 + k.ud,
+                                        __longlong_as_double(static_cast<long long>(rb)), fact,
+                                        prep, k, hdr);
+          }
+          __hip_atomic_store(&hbits[i], static_cast<uint64_t>(__double_as_longlong(hn)),
+                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
-        __hip_atomic_store(&hbits[i], static_cast<uint64_t>(__double_as_longlong(hn)),
-                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        break;
       }
       __builtin_amdgcn_s_sleep(1);
     }
@@ -1059,8 +1077,7 @@ __global__ __launch_bounds__(kCntBlock) __attribute__((amdgpu_waves_per_eu(6))) 
 constexpr int kEroBlock = 256;   // items are small and latency-bound: many workgroups per CU
 constexpr int kWin = 1024;       // cells of an item held in LDS at once
 struct ErodeShared {
-  double hs[kWin];          // new elevation of each cell of the window, by position
-  uint8_t done[kWin];
+  unsigned long long hs[kWin];   // bits of each cell's new elevation by position in the window, or the mark
   uint64_t item;
 };
 
@@ -1126,12 +1143,11 @@ __global__ __launch_bounds__(kEroBlock) void k_deep_erode(
     const uint32_t *const tl = cells + static_cast<size_t>(wt.tg) * kCells + first;
     for (int w0 = 0; w0 < n; w0 += kWin) {
       const int wn = min(kWin, n - w0);
-      for (int q = threadIdx.x; q < wn; q += kEroBlock) sh.done[q] = 0;
+      for (int q = threadIdx.x; q < wn; q += kEroBlock) sh.hs[q] = kUnsolved;
       __syncthreads();
       // wavefront: each wave takes 64-cell chunks in order; a lane solves its
-      // cell as soon as its receiver is done.  The wait, the solve and the
-      // publication share one loop, so a lane whose receiver is on its own
-      // wave gets it on a later pass.
+      // cell as soon as its receiver is done, one on its own wave on a later
+      // pass
       for (int ch = wave; ch * kWave < wn; ch += kEroBlock / kWave) {
         const int q = ch * kWave + lane;
         if (q >= wn) continue;
@@ -1144,47 +1160,61 @@ __global__ __launch_bounds__(kEroBlock) void k_deep_erode(
         const uint8_t r = rcv[g];
         const double h0 = h_old[g];
         const double fact = ftab[2 * static_cast<size_t>(cnt[g]) + (r & 1)];
+        const NewtonPrep prep = prepare<NMODE>(G.nmode, h0 + k.ud, fact, k);
         const unsigned long long *rp_g = reinterpret_cast<const unsigned long long *>(
             h_new + static_cast<long long>(g) + dir_offset(r, W));
-        int spins = 0;
-        for (;;) {
-          bool ready;
-          double hr = 0.0;
-          if (local) {
-            ready = __hip_atomic_load(&sh.done[rp - w0], __ATOMIC_ACQUIRE,
-                                      __HIP_MEMORY_SCOPE_WORKGROUP) != 0;
-            if (ready) hr = sh.hs[rp - w0];
-          } else {
-            const unsigned long long v =
-                __hip_atomic_load(rp_g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            ready = v != kUnsolved;
-            hr = __longlong_as_double(static_cast<long long>(v));
+        // a wave-uniform loop, so that a lane publishes in the pass that solves
+        // it: as the exit of a loop that lanes leave one by one, the
+        // publication may be placed behind the loop, where lanes of the same
+        // wave would wait for it
+        bool open = true;
+        for (int spins = 0; __ballot(open) != 0; spins++) {
+          if (open) {
+            // one 64-bit read both signals the receiver's solve and delivers it
+            unsigned long long v;
+            if (local) {
+              v = __hip_atomic_load(&sh.hs[rp - w0], __ATOMIC_RELAXED,
+                                    __HIP_MEMORY_SCOPE_WORKGROUP);
+            } else {
+              v = __hip_atomic_load(rp_g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+              // waited for here: behind the branch, lanes that read LDS would
+              // wait for their wave's stores to memory as well
+              asm volatile("" : "+v"(v));
+            }
+            const bool ready = v != kUnsolved, give_up = spins >= kSpinCap;
+            if (ready || give_up) {
+              open = false;
+              double hn = h0;
+              if (ready)
+                hn = solve<NMODE, true>(G.nmode, h0 + k.ud,
+                                        __longlong_as_double(static_cast<long long>(v)), fact,
+                                        prep, k, hdr);
+              else
+                atomicOr(&hdr[2], kErrLookback);
+              const unsigned long long bits =
+                  static_cast<unsigned long long>(__double_as_longlong(hn));
+              __hip_atomic_store(&sh.hs[q], bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+              // every new elevation goes past this XCD's cache: border cells
+              // may be the receivers of other tiles' exits, and a cache line
+              // holds cells of two tiles wherever a row does not start on a
+              // line, so a plain store beside such a receiver would leave this
+              // XCD's L2 with a copy of the line that its polls could read
+              __hip_atomic_store(reinterpret_cast<unsigned long long *>(h_new + g), bits,
+                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
           }
-          const bool give_up = !ready && ++spins > kSpinCap;
-          if (ready || give_up) {
-            double hn = h0;
-            if (give_up) atomicOr(&hdr[2], kErrLookback);
-            else hn = solve<NMODE>(G.nmode, h0 + k.ud, hr, fact, k, hdr);
-            sh.hs[q] = hn;
-            __hip_atomic_store(&sh.done[q], static_cast<uint8_t>(1), __ATOMIC_RELEASE,
-                               __HIP_MEMORY_SCOPE_WORKGROUP);
-            // every new elevation goes past this XCD's cache: border cells
-            // may be the receivers of other tiles' exits, and a cache line
-            // holds cells of two tiles wherever a row does not start on a
-            // line, so a plain store beside such a receiver would leave this
-            // XCD's L2 with a copy of the line that its polls could read
-            __hip_atomic_store(reinterpret_cast<unsigned long long *>(h_new + g),
-                               static_cast<unsigned long long>(__double_as_longlong(hn)),
-                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            break;
-          }
-          __builtin_amdgcn_s_sleep(1);
         }
       }
       __syncthreads();
     }
   }
 }
+
+// Whether k_deep_counts runs the chain form of the solve for n = 2: with up
+// to four tiles per CU its waves wait for each other (reference constants, 501^2
+// 113 -> 93 us, 1000^2 115 -> 93, 2048^2 245 -> 205), with more the plain loop
+// is ahead (4097x3001 267 against 278, 10000^2 1140 against 1432).
+inline bool counts_chain(int tiles, int ncu) { return tiles <= 4 * ncu; }
 
 // The persistent erosion grid: as many workgroups as fit on the device at
 // once (host side).

@@ -338,7 +338,7 @@ int check_schedule(const fs_schedule &s) {
 // (fs_deep.h), on the same stream.  The host reads the list's tile count
 // (one wait per step, while the erosion runs) so every per-tile kernel is
 // launched with exactly one workgroup per tile.
-template <int NM>
+template <int NM, bool kChain>
 int graph_launches(fs_ensemble *e, const deep::GraphWork &w, int T) {
   hipStream_t s = e->stream;
   const double *h_old = e->h[e->cur];
@@ -357,7 +357,7 @@ int graph_launches(fs_ensemble *e, const deep::GraphWork &w, int T) {
                      e->node_kids, e->node_parent, e->nexit, e->node_out, e->tstat);
   hipLaunchKernelGGL(deep::k_deep_levels, dim3(T), dim3(deep::kBlock), 0, s, w, e->dinfo, e->link,
                      e->node_level);
-  hipLaunchKernelGGL(deep::k_deep_counts<NM>, dim3(T), dim3(deep::kCntBlock), 0, s, w, e->rcv,
+  hipLaunchKernelGGL((deep::k_deep_counts<NM, kChain>), dim3(T), dim3(deep::kCntBlock), 0, s, w, e->rcv,
                      e->cnt, e->dinfo, e->link, e->node_out, e->node_cell, e->node_tier, e->nexit,
                      e->tile_n0, e->cells_list, e->tcur, e->items, e->ftab, h_old, h_new);
   hipLaunchKernelGGL(deep::k_deep_erode<NM>, dim3(static_cast<unsigned>(e->graph_blocks)),
@@ -381,9 +381,11 @@ int graph_step(fs_ensemble *e) {
   w.which = e->tabG_real;
   w.size = e->tabG_size;
   e->graph_tiles += static_cast<uint64_t>(T);
-  if (e->nm_all == 1) return graph_launches<1>(e, w, T);
-  if (e->nm_all == 2) return graph_launches<2>(e, w, T);
-  return graph_launches<-1>(e, w, T);
+  if (e->nm_all == 1) return graph_launches<1, false>(e, w, T);
+  const bool chain = deep::counts_chain(T, e->ncu);
+  if (e->nm_all == 2)
+    return chain ? graph_launches<2, true>(e, w, T) : graph_launches<2, false>(e, w, T);
+  return chain ? graph_launches<-1, true>(e, w, T) : graph_launches<-1, false>(e, w, T);
 }
 
 // A grid of at least n workgroups (a grid of one row holds fewer than 2^32
