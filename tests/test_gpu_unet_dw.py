@@ -38,3 +38,22 @@ def test_batch_gradient_is_the_mean_of_the_samples(H, W, B):
             # power of two: 2^-8 a value, averaging out over the pixels
             tol = 2e-4 if B & (B - 1) == 0 else 2e-2
             assert np.linalg.norm(a - m) <= tol * np.linalg.norm(m), (i, what)
+
+
+@pytest.mark.parametrize("H,W,B", [(32, 32, 1), (32, 96, 5), (256, 256, 9)])
+def test_loss_and_head_bias_against_64_bits(H, W, B):
+    """Sums over all pixels, in FP32: a term is rounded three times, and is part
+    of at most (terms of a thread + 6 shuffles + 3 + one addition per workgroup,
+    at most 2048) additions: that many times 2^-24 of the sum of magnitudes."""
+    note("loss %dx%d batch %d" % (H, W, B))
+    terrain, params, target = sample(2 * H + W, B, H, W)
+    with fa.UNet(H, W, max_batch=B, seed=43) as net:
+        net.set_params(perturbed_params(net, 44))
+        y = net.forward(terrain, params).astype(np.float64).ravel()
+        loss, g = net.loss_grad(terrain, params, target)
+    M = B * H * W
+    e = y - target.astype(np.float64).ravel()
+    groups = min((4 * M + 255) // 256, 2048)
+    eps = (3 + -(-4 * M // (256 * groups)) + 9 + groups) * 2.0 ** -24
+    assert abs(loss - np.sum(e * e) / M) <= eps * np.sum(e * e) / M
+    assert abs(g[-1] - np.sum(2 * e) / M) <= eps * np.sum(2 * np.abs(e)) / M
