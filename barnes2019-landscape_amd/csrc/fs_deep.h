@@ -321,16 +321,20 @@ __device__ __forceinline__ int border_cell(int k, const Box &b) {
 // ---------------------------------------------------------------------------
 constexpr int kLocalBlock = 512;
 constexpr int kLocalPer = kCells / kLocalBlock;
+// jump words: a cell of the tile, or once a chain's end is reached its tail
+constexpr int kJumpEnd = 0x8000, kJumpExit = 0x4000, kJumpRoot = 0x2000;
+constexpr int kJumpRounds = 12;   // a chain has at most kCells - 1 hops
+static_assert(kCells <= 1 << kJumpRounds && kCells <= kJumpRoot, "jump words");
 __global__ __launch_bounds__(kLocalBlock) void k_deep_local(
     GraphWork w, const uint8_t *__restrict__ rcv0, uint32_t *__restrict__ cnt0,
     uint32_t *__restrict__ dinfo0, uint32_t *__restrict__ link0, uint64_t *__restrict__ node_word,
     uint32_t *__restrict__ node_kids, int32_t *__restrict__ node_cell,
     int32_t *__restrict__ nexit, int32_t *__restrict__ tile_n0, uint32_t *__restrict__ cells,
     double *__restrict__ h_new0, int32_t *__restrict__ tstat) {
-  __shared__ uint16_t nx[kCells];
-  // walk words: (next cell + 1) << 16 | local count; 0 in the top half at a
-  // tail (later the root list's counters)
-  __shared__ uint32_t jw[kCells];
+  __shared__ uint16_t jump[kCells];   // a cell some hops downstream; kJumpEnd: the tail
+  __shared__ uint16_t hop[kCells];    // hops to the tail, once it is known
+  __shared__ uint32_t sum[kCells];    // tile cells upstream so far (later the root list's counters)
+  __shared__ int more[kJumpRounds];
   __shared__ uint16_t slot_node[4 * kSide];   // node number of the exit at each border position
   __shared__ int wave_nodes[4 * kSide / kWave];
   __shared__ int maxhops, scan[kLocalBlock / kWave + 1];
@@ -352,6 +356,8 @@ __global__ __launch_bounds__(kLocalBlock) void k_deep_local(
   // receiver bytes, kept for the exits' marks; all requested before any is
   // used (a cell past a partial tile's edge reads one inside it)
   uint8_t rr[kLocalPer];
+  int cur[kLocalPer];
+  uint32_t up[kLocalPer], alive = 0;
 #pragma unroll
   for (int j = 0; j < kLocalPer; j++) {
     const int i = j * kLocalBlock + threadIdx.x;
@@ -365,43 +371,61 @@ __global__ __launch_bounds__(kLocalBlock) void k_deep_local(
     uint16_t n = kTermNone;
     if (lx < b.tw && ly < b.th) n = tile_next(rr[j], lx, ly, b);
     else rr[j] = 0xFF;
-    nx[i] = n;
-    jw[i] = n < kTermNone ? (static_cast<uint32_t>(n) + 1u) << 16 : 0u;
-  }
-  __syncthreads();
-  // every tile cell walks its in-tile chain to its tail, adding 1 to each
-  // cell it passes, itself included: one LDS atomic per step returns the
-  // cell's word, whose top half names the next cell.  The walk gives the
-  // cell's tail and hops, the adds every cell's local count (the tile cells
-  // upstream of it, itself included).  A thread's walks advance together,
-  // one step per round, with no barrier.
-  int cur[kLocalPer], hops[kLocalPer];
-  uint32_t alive = 0;
-#pragma unroll
-  for (int j = 0; j < kLocalPer; j++) {
-    const int i = j * kLocalBlock + threadIdx.x;
-    cur[j] = i;
-    hops[j] = 0;
-    if (i % kSide < b.tw && i / kSide < b.th) alive |= 1u << j;
-  }
-  for (int step = 0; alive != 0 && step < kCells; step++) {
-#pragma unroll
-    for (int j = 0; j < kLocalPer; j++) {
-      if (!(alive & (1u << j))) continue;
-      const uint32_t nxt = atomicAdd(&jw[cur[j]], 1u) >> 16;
-      if (nxt == 0) {
-        alive &= ~(1u << j);
-      } else {
-        cur[j] = static_cast<int>(nxt) - 1;
-        hops[j]++;
-      }
+    if (n < kTermNone) {
+      cur[j] = n;
+      alive |= 1u << j;
+    } else {
+      cur[j] = i | kJumpEnd | (n == kTermExit ? kJumpExit : 0) | (n == kTermRoot ? kJumpRoot : 0);
     }
+    jump[i] = static_cast<uint16_t>(cur[j]);
+    hop[i] = 0;
+    sum[i] = 1;
+    up[j] = 1;
+  }
+  if (threadIdx.x < kJumpRounds) more[threadIdx.x] = 0;
+  __syncthreads();
+  // every cell's tail, hops and local count (the tile cells upstream of it,
+  // itself included) by pointer doubling: after k rounds a cell knows the
+  // cell 2^k hops downstream, and the count of the cells less than 2^k hops
+  // upstream; those 2^k hops away and beyond add theirs in round k.  A tile
+  // takes log2 of its longest chain in rounds, and a cell log2 of its own in
+  // LDS atomics.  (Walking every chain, one returning atomic a hop, against
+  // doubling, in deep drainage: 62 and 24 us for the 64 tiles of a 501 x 501
+  // grid, 168 and 95 for 4097 x 3001, 790 and 617 for 10000 x 10000, which is
+  // bound by the LDS.)
+  for (int k = 0; k < kJumpRounds; k++) {
+    int nxt[kLocalPer];
+#pragma unroll
+    for (int j = 0; j < kLocalPer; j++)
+      if (alive & (1u << j)) {
+        nxt[j] = jump[cur[j]];
+        atomicAdd(&sum[cur[j]], up[j]);
+      }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kLocalPer; j++)
+      if (alive & (1u << j)) {
+        const int i = j * kLocalBlock + threadIdx.x;
+        up[j] = sum[i];
+        if (nxt[j] & kJumpEnd) {
+          hop[i] = static_cast<uint16_t>((1 << k) + hop[cur[j]]);
+          alive &= ~(1u << j);
+        }
+        cur[j] = nxt[j];
+        jump[i] = static_cast<uint16_t>(nxt[j]);
+      }
+    if (__any(alive != 0) && (threadIdx.x & (kWave - 1)) == 0) more[k] = 1;
+    __syncthreads();
+    if (!more[k]) break;   // the same for every thread
   }
   if (alive != 0) atomicOr(&tstat[kStErr], kErrChain);   // a receiver cycle
-  int mh = 0;
+  int hops[kLocalPer], mh = 0;
 #pragma unroll
-  for (int j = 0; j < kLocalPer; j++) mh = max(mh, hops[j]);
-  const int top = block_max(mh, &maxhops);   // its barrier ends every walk
+  for (int j = 0; j < kLocalPer; j++) {
+    hops[j] = hop[j * kLocalBlock + threadIdx.x];
+    mh = max(mh, hops[j]);
+  }
+  const int top = block_max(mh, &maxhops);
   // exits become the tile's nodes, numbered in border-position order: the
   // first four waves take one border position per lane
   constexpr int kSlotWaves = 4 * kSide / kWave;
@@ -409,7 +433,7 @@ __global__ __launch_bounds__(kLocalBlock) void k_deep_local(
   uint64_t slot_mask = 0;
   if (threadIdx.x < 4 * kSide) {
     slot_cell = border_cell(threadIdx.x, b);
-    const bool ex = slot_cell >= 0 && nx[slot_cell] == kTermExit;
+    const bool ex = slot_cell >= 0 && jump[slot_cell] == (slot_cell | kJumpEnd | kJumpExit);
     slot_mask = __ballot(ex);
     const int lane = threadIdx.x & (kWave - 1);
     slot_rank = ex ? __popcll(slot_mask & ((uint64_t{1} << lane) - 1)) : -1;
@@ -418,7 +442,7 @@ __global__ __launch_bounds__(kLocalBlock) void k_deep_local(
 #pragma unroll
   for (int j = 0; j < kLocalPer; j++) {   // the marks on the exits' receivers
     const int i = j * kLocalBlock + threadIdx.x;
-    if (nx[i] != kTermExit) continue;
+    if (cur[j] != (i | kJumpEnd | kJumpExit)) continue;
     const size_t g = static_cast<size_t>(b.y0 + i / kSide) * W + b.x0 + i % kSide;
     h_new[g + dir_offset(rr[j], W)] = __longlong_as_double(static_cast<long long>(kUnsolved));
   }
@@ -436,7 +460,7 @@ __global__ __launch_bounds__(kLocalBlock) void k_deep_local(
       slot_node[threadIdx.x] = static_cast<uint16_t>(k);
       const int id = t * kNodeCap + k;
       node_cell[id] = (b.y0 + slot_cell / kSide) * W + b.x0 + slot_cell % kSide;
-      node_word[id] = jw[slot_cell] & 0xFFFFu;
+      node_word[id] = sum[slot_cell];
       node_kids[id] = 0;
     }
   }
@@ -444,41 +468,40 @@ __global__ __launch_bounds__(kLocalBlock) void k_deep_local(
 #pragma unroll
   for (int j = 0; j < kLocalPer; j++) {
     const int i = j * kLocalBlock + threadIdx.x;
-    if (nx[i] == kTermNone) continue;
+    const int tail = cur[j] & (kCells - 1);
+    const bool exit_tail = (cur[j] & kJumpExit) != 0;
+    if (cur[j] == (i | kJumpEnd)) continue;   // beyond the grid
     const int lx = i % kSide, ly = i / kSide;
     const size_t g = static_cast<size_t>(b.y0 + ly) * W + b.x0 + lx;
-    const bool exit_tail = nx[cur[j]] == kTermExit;
-    cnt[g] = jw[i] & 0xFFFFu;
-    dinfo[g] = static_cast<uint32_t>(cur[j]) | (static_cast<uint32_t>(hops[j]) << 12) |
+    cnt[g] = sum[i];
+    dinfo[g] = static_cast<uint32_t>(tail) | (static_cast<uint32_t>(hops[j]) << 12) |
                (exit_tail ? kInfoExit : 0u);
     if (lx == 0 || ly == 0 || lx == b.tw - 1 || ly == b.th - 1)
       link[g] = exit_tail ? static_cast<uint32_t>(t * kNodeCap +
-                                                  slot_node[border_pos(cur[j] % kSide,
-                                                                       cur[j] / kSide, b)])
+                                                  slot_node[border_pos(tail % kSide, tail / kSide, b)])
                           : kNoNode;
   }
   if (threadIdx.x == 0) nexit[t] = nnode;   // every slot thread summed the same count
   // the cells with a root tail, sorted by hops, start the tile's cell list
-  // (jw is free once every count is stored: its words count the cells per
+  // (sum is free once every count is stored: its words count the cells per
   // hops)
   __syncthreads();
-  for (int q = threadIdx.x; q <= top; q += kLocalBlock) jw[q] = 0;
+  for (int q = threadIdx.x; q <= top; q += kLocalBlock) sum[q] = 0;
   __syncthreads();
   bool rooted[kLocalPer];
 #pragma unroll
   for (int j = 0; j < kLocalPer; j++) {
-    const int i = j * kLocalBlock + threadIdx.x;
-    rooted[j] = nx[i] != kTermNone && nx[cur[j]] == kTermRoot;
-    if (rooted[j]) atomicAdd(&jw[hops[j]], 1u);
+    rooted[j] = (cur[j] & kJumpRoot) != 0;
+    if (rooted[j]) atomicAdd(&sum[hops[j]], 1u);
   }
   __syncthreads();
   int carry = 0;
   for (int base = 0; base <= top; base += kLocalBlock) {
     const int q = base + threadIdx.x;
-    const int v = q <= top ? static_cast<int>(jw[q]) : 0;
+    const int v = q <= top ? static_cast<int>(sum[q]) : 0;
     int total;
     const int ex = block_scan<kLocalBlock>(v, scan, &total);
-    if (q <= top) jw[q] = static_cast<uint32_t>(carry + ex);
+    if (q <= top) sum[q] = static_cast<uint32_t>(carry + ex);
     carry += total;
   }
   __syncthreads();   // every cursor is set before any thread takes a slot
@@ -486,7 +509,7 @@ __global__ __launch_bounds__(kLocalBlock) void k_deep_local(
 #pragma unroll
   for (int j = 0; j < kLocalPer; j++)
     if (rooted[j])
-      list[atomicAdd(&jw[hops[j]], 1u)] =
+      list[atomicAdd(&sum[hops[j]], 1u)] =
           static_cast<uint32_t>(j * kLocalBlock + threadIdx.x) | kNoPos << kEntShift;
   // n0, and the tile's largest hops (which bounds the sort keys of k_deep_counts)
   if (threadIdx.x == 0) tile_n0[t] = carry | top << 16;
