@@ -158,7 +158,7 @@ struct fs_model {
   uint32_t *node_kids = nullptr, *node_parent = nullptr, *node_out = nullptr;
   int32_t *node_cell = nullptr, *nexit = nullptr;
   uint16_t *node_tier = nullptr;
-  int32_t *tile_n0 = nullptr;      // per tile: cells with a root tail | largest hops << 16
+  int32_t *tile_n0 = nullptr;      // per tile: cells with a root tail, and a cycle mark
   int32_t *thist = nullptr, *tcur = nullptr;   // per tier: work items, their cursor
   uint32_t *cells = nullptr;       // per tile: its cells sorted by tier (list entries)
   uint64_t *items = nullptr;       // work items in tier order
@@ -930,6 +930,7 @@ int ensure_graph(fs_model *m) {
   FS_TRY(fs::dev_alloc(&m->items, tiles * deep::kTiersPerTile));
   FS_TRY(fs::dev_alloc(&m->tstat, deep::kStWords));
   FS_HIP_TRY(hipMemsetAsync(m->thist, 0, tier_words * sizeof(int32_t), m->stream));
+  FS_HIP_TRY(hipMemsetAsync(m->tstat, 0, deep::kStWords * sizeof(int32_t), m->stream));
   deep::GraphGrid g{};
   g.off = 0;
   g.ftab_off = 0;
@@ -989,8 +990,6 @@ int graph_path(fs_model *m, const hipEvent_t *ev) {
   const int tiles = ((m->W + deep::kSide - 1) / deep::kSide) *
                     ((m->H + deep::kSide - 1) / deep::kSide);
   const deep::GraphWork w = graph_work(m);
-  hipLaunchKernelGGL(deep::k_deep_clear, dim3(1), dim3(64), 0, s, m->tstat);
-  FS_TRY(check_launch());
   FS_TRY(kt_begin(m, FS_K_GRAPH_LOCAL));
   hipLaunchKernelGGL(deep::k_deep_local, dim3(tiles), dim3(deep::kLocalBlock), 0, s, w, m->rcv, m->cnt,
                      m->dinfo, m->link, m->node_word, m->node_kids, m->node_cell, m->nexit,
@@ -1000,19 +999,14 @@ int graph_path(fs_model *m, const hipEvent_t *ev) {
   FS_TRY(mark(ev[2], s));
   FS_TRY(kt_begin(m, FS_K_GRAPH_NODES));
   hipLaunchKernelGGL(deep::k_deep_links, dim3(tiles), dim3(deep::kNodeCap), 0, s, w, m->rcv,
-                     m->link, m->dinfo, m->node_cell, m->nexit, m->node_parent, m->node_kids,
-                     static_cast<uint32_t *>(nullptr));
-  FS_TRY(check_launch());
-  hipLaunchKernelGGL(deep::k_deep_tiers, dim3(tiles), dim3(deep::kNodeCap), 0, s, w,
-                     m->node_parent, m->nexit, m->node_tier, static_cast<const uint32_t *>(nullptr),
-                     static_cast<uint32_t *>(nullptr), m->thist, m->tstat);
-  FS_TRY(check_launch());
-  hipLaunchKernelGGL(deep::k_deep_scan, dim3(1), dim3(deep::kBlock), 0, s, m->thist, m->tcur,
-                     m->tstat, m->graph_queues);
+                     m->link, m->dinfo, m->node_cell, m->nexit, m->tile_n0, m->node_parent,
+                     m->node_kids, static_cast<uint32_t *>(nullptr), m->tstat);
   FS_TRY(check_launch());
   FS_TRY(mark(ev[3], s));
-  hipLaunchKernelGGL(deep::k_deep_sum, dim3(tiles), dim3(deep::kNodeCap), 0, s, w, m->node_word,
-                     m->node_kids, m->node_parent, m->nexit, m->node_out, m->tstat);
+  hipLaunchKernelGGL(deep::k_deep_nodes, dim3(2 * tiles), dim3(deep::kNodeCap), 0, s, w,
+                     m->node_parent, m->nexit, m->node_tier, static_cast<const uint32_t *>(nullptr),
+                     static_cast<uint32_t *>(nullptr), m->thist, m->tcur, m->graph_queues,
+                     m->node_word, m->node_kids, m->node_out, m->tstat);
   FS_TRY(check_launch());
   FS_TRY(kt_end(m));
   FS_TRY(mark(ev[4], s));

@@ -21,13 +21,13 @@
 //                 new elevation field; the cells whose tail is a root start
 //                 the tile's cell list, sorted by hops
 //   k_deep_links  every node's parent, and the number of children per node
-//   k_deep_tiers  every node's tier (walking its parents), and the number of
-//                 (tile, tier) work items per tier
-//   k_deep_scan   the work items' offsets: up to 64 queues, each holding its
-//                 tiles' items in tier order (one workgroup)
-//   k_deep_sum    the count through every exit: its local count plus its
-//                 children's, leaf to root (the last child to arrive carries
-//                 the sum on, so each node is summed once)
+//   k_deep_nodes  half the workgroups: every node's tier (walking its
+//                 parents), the number of (tile, tier) work items per tier,
+//                 and from these (the last workgroup) the items' offsets: up
+//                 to 64 queues, each holding its tiles' items in tier order;
+//                 the other half: the count through every exit, its local
+//                 count plus its children's, leaf to root (the last child to
+//                 arrive carries the sum on, so each node is summed once)
 //   k_deep_counts per tile: the counts finished by the inflows of the ring
 //                 cells that drain into the tile (each walked down its
 //                 in-tile chain); the erosion of the cells with a root tail
@@ -81,15 +81,17 @@ __device__ __forceinline__ int shard_of(int t) {
   return static_cast<int>((static_cast<uint32_t>(t) * 2654435761u) >> 26);
 }
 static_assert(kShards == 1 << (32 - 26), "shard_of");
-// tstat words: error bits, deepest tier, items; the first item of each
-// queue (and the end of the last); each queue's cursor on a cache line of
-// its own (kQStride words apart).  Steps clear the first kStClear words.
-constexpr int kStErr = 0, kStMaxTier = 1, kStItems = 2, kStClear = 3;
+// tstat words: error bits, deepest tier, items, groups of tiles whose tiers
+// are counted; the first item of each queue (and the end of the last); each
+// queue's cursor, and beside it a count of finished tiles, on a cache line of
+// its own (kQStride words apart).  All are zero before the first step;
+// k_deep_local clears the first kStClear words.
+constexpr int kStErr = 0, kStMaxTier = 1, kStItems = 2, kStDone = 3, kStClear = 4;
 constexpr int kStQStart = 4;
 constexpr int kQStride = 32;
 constexpr int kStQCur = 128;
 constexpr int kStWords = kStQCur + kShards * kQStride;
-static_assert(kStQStart + kShards + 1 <= kStQCur, "queue starts fit before the cursors");
+static_assert(kStClear <= kStQStart && kStQStart + kShards + 1 <= kStQCur, "queue starts fit before the cursors");
 constexpr int32_t kErrTier = 1, kErrChain = 2;
 // the "not yet eroded" mark: a signalling NaN that no arithmetic produces
 constexpr unsigned long long kUnsolved = 0x7FF4A5A5A5A5A5A5ull;
@@ -328,6 +330,7 @@ __device__ __forceinline__ int border_cell(int k, const Box &b) {
 // ---------------------------------------------------------------------------
 constexpr int kLocalBlock = 512;
 constexpr int kLocalPer = kCells / kLocalBlock;
+constexpr int kTileCycle = 1 << 16;   // in tile_n0, beside the count: the tile's chains do not end
 // jump words: a cell of the tile, or once a chain's end is reached its tail
 constexpr int kJumpEnd = 0x8000, kJumpExit = 0x4000, kJumpRoot = 0x2000;
 constexpr int kJumpRounds = 12;   // a chain has at most kCells - 1 hops
@@ -356,6 +359,7 @@ __global__ __launch_bounds__(kLocalBlock) void k_deep_local(
   const int t = wt.tg;   // per-tile arrays and node ids
   const Box b = tile_box(wt.t, G.tiles_x, W, H);
   if (threadIdx.x == 0) maxhops = 0;
+  if (wi == 0 && threadIdx.x < kStClear) tstat[threadIdx.x] = 0;
   if (wt.t == 0 && G.levels) {   // the grid's level counts start from zero
     if (threadIdx.x == 0) G.hdr[0] = 0;
     for (int q = threadIdx.x; q < G.nlev; q += kLocalBlock) G.levels[q] = 0;
@@ -425,7 +429,7 @@ __global__ __launch_bounds__(kLocalBlock) void k_deep_local(
     __syncthreads();
     if (!more[k]) break;   // the same for every thread
   }
-  if (alive != 0) atomicOr(&tstat[kStErr], kErrChain);   // a receiver cycle
+  const bool cycle = more[kJumpRounds - 1] != 0;   // a receiver cycle: no chain is longer
   int hops[kLocalPer], mh = 0;
 #pragma unroll
   for (int j = 0; j < kLocalPer; j++) {
@@ -518,8 +522,7 @@ __global__ __launch_bounds__(kLocalBlock) void k_deep_local(
     if (rooted[j])
       list[atomicAdd(&sum[hops[j]], 1u)] =
           static_cast<uint32_t>(j * kLocalBlock + threadIdx.x) | kNoPos << kEntShift;
-  // n0, and the tile's largest hops (which bounds the sort keys of k_deep_counts)
-  if (threadIdx.x == 0) tile_n0[t] = carry | top << 16;
+  if (threadIdx.x == 0) tile_n0[t] = carry | (cycle ? kTileCycle : 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -530,12 +533,14 @@ __global__ __launch_bounds__(kLocalBlock) void k_deep_local(
 __global__ __launch_bounds__(kNodeCap) void k_deep_links(
     GraphWork w, const uint8_t *__restrict__ rcv0, const uint32_t *__restrict__ link0,
     const uint32_t *__restrict__ dinfo0, const int32_t *__restrict__ node_cell,
-    const int32_t *__restrict__ nexit, uint32_t *__restrict__ node_parent,
-    uint32_t *__restrict__ node_kids, uint32_t *__restrict__ node_up) {
+    const int32_t *__restrict__ nexit, const int32_t *__restrict__ tile_n0,
+    uint32_t *__restrict__ node_parent, uint32_t *__restrict__ node_kids,
+    uint32_t *__restrict__ node_up, int32_t *__restrict__ tstat) {
   const int k = threadIdx.x, wi = blockIdx.x;
   if (wi >= w.size[1]) return;
   const WorkTile wt = work_tile(w, wi);
   const int t = wt.tg;
+  if (k == 0 && (tile_n0[t] & kTileCycle)) atomicOr(&tstat[kStErr], kErrChain);
   if (k >= nexit[t]) return;
   const int id = t * kNodeCap + k;
   const int32_t g = node_cell[id];
@@ -547,17 +552,80 @@ __global__ __launch_bounds__(kNodeCap) void k_deep_links(
   if (node_up) node_up[id] = 1u + static_cast<uint32_t>(info_hops(dinfo0[wt.off + y]));
 }
 
-// Tier of every node, by walking its parents (a chain of tiles crossed by
-// one drainage path); per tier, the number of tiles holding cells of it.
-__global__ __launch_bounds__(kNodeCap) void k_deep_tiers(
+// Offsets of the work items: thist (counts per tier and shard) -> tcur
+// (the first slot of each (tier, shard), then the cursor k_deep_counts
+// appends at).  The items are laid out queue by queue -- queue q holds the
+// shards s with s % nq == q -- and each queue's tier by tier, so a queue
+// hands out its items in tier order.  Writes each queue's first item and
+// cursor, clears thist for the next step.  One workgroup of kNodeCap threads
+// in the kernel that counted: the counts of the other workgroups' atomics
+// are read past this XCD's cache; nq divides kShards.
+__device__ __forceinline__ void item_offsets(int32_t *__restrict__ thist,
+                                             int32_t *__restrict__ tcur,
+                                             int32_t *__restrict__ tstat, int nq, int *sh) {
+  constexpr int kWords = 4;   // consecutive words per thread
+  auto read = [](int32_t *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  const int spq = kShards / nq;                               // shards per queue
+  const int per_q = (read(&tstat[kStMaxTier]) + 1) * spq;     // (tier, shard) words per queue
+  const int n = nq * per_q;
+  int carry = 0;
+  for (int base = 0; base < n; base += kNodeCap * kWords) {
+    int idx[kWords], v[kWords], sum = 0;
+#pragma unroll
+    for (int j = 0; j < kWords; j++) {
+      const int k = base + threadIdx.x * kWords + j;
+      const int q = k / per_q, rem = k - q * per_q;
+      const int tier = rem / spq, s = q + (rem - tier * spq) * nq;
+      idx[j] = k < n ? tier * kShards + s : -1;
+      v[j] = idx[j] >= 0 ? read(&thist[idx[j]]) : 0;
+    }
+#pragma unroll
+    for (int j = 0; j < kWords; j++) sum += v[j];
+    int total;
+    int at = carry + block_scan<kNodeCap>(sum, sh, &total);
+#pragma unroll
+    for (int j = 0; j < kWords; j++) {
+      if (idx[j] < 0) continue;
+      const int k = base + threadIdx.x * kWords + j;
+      tcur[idx[j]] = at;
+      thist[idx[j]] = 0;
+      if (k % per_q == 0) {   // the queue's first word
+        tstat[kStQStart + k / per_q] = at;
+        tstat[kStQCur + (k / per_q) * kQStride] = at;
+      }
+      at += v[j];
+    }
+    carry += total;
+  }
+  if (threadIdx.x == 0) {
+    tstat[kStItems] = carry;
+    tstat[kStQStart + nq] = carry;
+  }
+}
+
+// Two workgroups of kNodeCap threads per tile.  The first size[1] workgroups:
+// the tier of every node, by walking its parents (a chain of tiles crossed by
+// one drainage path); per tier, the number of tiles holding cells of it; the
+// last of them to finish, the work items' offsets.  The others: the count
+// through every exit, leaf to root.  (As a launch each, the chains of memory
+// round trips one behind the other, all the node kernels took 23 us at 501 x
+// 501, 30 at 1000 x 1000 and 81 at 4097 x 3001 in deep drainage, 250 where 369
+// tiers lie in 250 x 250 cells; now 15, 21, 71 and 158.  Fences around the
+// ticks write every workgroup's L2 back: 299 us at 4097 x 3001.)
+__global__ __launch_bounds__(kNodeCap) void k_deep_nodes(
     GraphWork w, const uint32_t *__restrict__ node_parent, const int32_t *__restrict__ nexit,
     uint16_t *__restrict__ node_tier, const uint32_t *__restrict__ node_up,
-    uint32_t *__restrict__ node_level, int32_t *__restrict__ thist,
-    int32_t *__restrict__ tstat) {
+    uint32_t *__restrict__ node_level, int32_t *__restrict__ thist, int32_t *__restrict__ tcur,
+    int nq, uint64_t *__restrict__ node_word, const uint32_t *__restrict__ node_kids,
+    uint32_t *__restrict__ node_out, int32_t *__restrict__ tstat) {
   __shared__ uint32_t seen[(kTierCap + 32) / 32];   // tiers already counted for the tile
-  const int k = threadIdx.x, wi = blockIdx.x;
-  if (wi >= w.size[1]) return;
-  {
+  __shared__ int scan[kNodeCap / kWave + 1], last;
+  const int k = threadIdx.x, tiles = w.size[1];
+  int wi = blockIdx.x;
+  if (wi >= 2 * tiles) return;
+  if (wi < tiles) {
     const int t = work_tile(w, wi).tg;
     const int n = nexit[t];
     int tier = 0;
@@ -590,83 +658,49 @@ __global__ __launch_bounds__(kNodeCap) void k_deep_tiers(
         }
       }
     }
+    // the counts are atomics, performed past the caches: once a wave's have
+    // been acknowledged, its workgroup ticks, first among the tiles with the
+    // same low bits (tens of thousands of ticks stay off one address), the last of
+    // these for all of them
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-  }
-}
-
-// Offsets of the work items: thist (counts per tier and shard) -> tcur
-// (the first slot of each (tier, shard), then the cursor k_deep_counts
-// appends at).  The items are laid out queue by queue -- queue q holds the
-// shards s with s % nq == q -- and each queue's tier by tier, so a queue
-// hands out its items in tier order.  Writes each queue's first item and
-// cursor, clears thist for the next step.  One workgroup of kBlock threads;
-// nq divides kShards.
-__global__ __launch_bounds__(kBlock) void k_deep_scan(int32_t *__restrict__ thist,
-                                                      int32_t *__restrict__ tcur,
-                                                      int32_t *__restrict__ tstat, int nq) {
-  __shared__ int sh[kBlock / kWave + 1];
-  const int spq = kShards / nq;                       // shards per queue
-  const int per_q = (tstat[kStMaxTier] + 1) * spq;    // (tier, shard) words per queue
-  const int n = nq * per_q;
-  int carry = 0;
-  for (int base = 0; base < n; base += kBlock) {
-    const int k = base + threadIdx.x;
-    int idx = 0, v = 0;
-    if (k < n) {
-      const int q = k / per_q, rem = k - q * per_q;
-      const int tier = rem / spq, s = q + (rem - tier * spq) * nq;
-      idx = tier * kShards + s;
-      v = thist[idx];
-    }
-    int total;
-    const int ex = block_scan(v, sh, &total);
-    if (k < n) {
-      tcur[idx] = carry + ex;
-      thist[idx] = 0;
-      if (k % per_q == 0) {   // the queue's first word
-        tstat[kStQStart + k / per_q] = carry + ex;
-        tstat[kStQCur + (k / per_q) * kQStride] = carry + ex;
+    if (k == 0) {
+      const int g = wi & (kShards - 1), groups = min(tiles, kShards);
+      int32_t *const tick = &tstat[kStQCur + g * kQStride + 1];
+      last = 0;
+      if (atomicAdd(tick, 1) == (tiles - g + kShards - 1) / kShards - 1) {
+        *tick = 0;   // for the next step
+        last = atomicAdd(&tstat[kStDone], 1) == groups - 1;
       }
     }
-    carry += total;
+    __syncthreads();
+    if (!last) return;
+    item_offsets(thist, tcur, tstat, nq, scan);
+    return;
   }
-  if (threadIdx.x == 0) {
-    tstat[kStItems] = carry;
-    tstat[kStQStart + nq] = carry;
-  }
-}
-
-// Count through every exit, leaf to root.
-__global__ __launch_bounds__(kNodeCap) void k_deep_sum(
-    GraphWork w, uint64_t *__restrict__ node_word, const uint32_t *__restrict__ node_kids,
-    const uint32_t *__restrict__ node_parent, const int32_t *__restrict__ nexit,
-    uint32_t *__restrict__ node_out, int32_t *__restrict__ tstat) {
-  const int k = threadIdx.x, wi = blockIdx.x;
-  if (wi >= w.size[1]) return;
-  {
-    const int t = work_tile(w, wi).tg;
-    if (k >= nexit[t]) return;
-    uint32_t id = static_cast<uint32_t>(t * kNodeCap + k);
-    if (node_kids[id] != 0) return;          // summed by its last child's thread
-    uint64_t val = node_word[id] & kSumMask;
-    bool ended = false;
-    for (int guard = 0; guard <= kTierCap; guard++) {
-      node_out[id] = static_cast<uint32_t>(val);
-      const uint32_t p = node_parent[id];
-      if (p == kNoNode) {
-        ended = true;
-        break;
-      }
-      const uint64_t old = atomicAdd(&node_word[p], val + kOneArrival);
-      if ((old >> kSumShift) + 1 != node_kids[p]) {   // not the last child
-        ended = true;
-        break;
-      }
-      val += old & kSumMask;
-      id = p;
+  wi -= tiles;
+  const int t = work_tile(w, wi).tg;
+  if (k >= nexit[t]) return;
+  uint32_t id = static_cast<uint32_t>(t * kNodeCap + k);
+  if (node_kids[id] != 0) return;          // summed by its last child's thread
+  uint64_t val = node_word[id] & kSumMask;
+  bool ended = false;
+  for (int guard = 0; guard <= kTierCap; guard++) {
+    node_out[id] = static_cast<uint32_t>(val);
+    const uint32_t p = node_parent[id];
+    if (p == kNoNode) {
+      ended = true;
+      break;
     }
-    if (!ended) atomicOr(&tstat[kStErr], kErrChain);
+    const uint64_t old = atomicAdd(&node_word[p], val + kOneArrival);
+    if ((old >> kSumShift) + 1 != node_kids[p]) {   // not the last child
+      ended = true;
+      break;
+    }
+    val += old & kSumMask;
+    id = p;
   }
+  if (!ended) atomicOr(&tstat[kStErr], kErrChain);
 }
 
 // ---------------------------------------------------------------------------
@@ -1141,7 +1175,7 @@ __device__ __forceinline__ uint64_t next_item(int32_t *tstat, const uint64_t *__
 // field (final: stored before the window's barrier), one in another tile from
 // the field once its mark is replaced.
 //
-// The items come from nq queues (k_deep_scan's layout); a workgroup takes
+// The items come from nq queues (item_offsets' layout); a workgroup takes
 // one item at a time from queue blockIdx.x % nq and moves to the next queue
 // only when its own is empty.  An item waits only on items of lower tiers;
 // a queue hands out its items in tier order, and every queue keeps its own
@@ -1263,10 +1297,6 @@ int erode_grid(int ncu) {
       per_cu < 1)
     per_cu = 1;
   return per_cu * (ncu < 1 ? 1 : ncu);
-}
-
-__global__ void k_deep_clear(int32_t *tstat) {
-  if (threadIdx.x < kStClear) tstat[threadIdx.x] = 0;
 }
 
 // Queues for a persistent erosion grid of `blocks` workgroups: the largest

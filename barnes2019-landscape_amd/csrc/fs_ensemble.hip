@@ -343,18 +343,15 @@ int graph_launches(fs_ensemble *e, const deep::GraphWork &w, int T) {
   hipStream_t s = e->stream;
   const double *h_old = e->h[e->cur];
   double *h_new = e->h[e->cur ^ 1];
-  hipLaunchKernelGGL(deep::k_deep_clear, dim3(1), dim3(64), 0, s, e->tstat);
   hipLaunchKernelGGL(deep::k_deep_local, dim3(T), dim3(deep::kLocalBlock), 0, s, w, e->rcv, e->cnt,
                      e->dinfo, e->link, e->node_word, e->node_kids, e->node_cell, e->nexit,
                      e->tile_n0, e->cells_list, h_new, e->tstat);
   hipLaunchKernelGGL(deep::k_deep_links, dim3(T), dim3(deep::kNodeCap), 0, s, w, e->rcv, e->link,
-                     e->dinfo, e->node_cell, e->nexit, e->node_parent, e->node_kids, e->node_up);
-  hipLaunchKernelGGL(deep::k_deep_tiers, dim3(T), dim3(deep::kNodeCap), 0, s, w, e->node_parent,
-                     e->nexit, e->node_tier, e->node_up, e->node_level, e->thist, e->tstat);
-  hipLaunchKernelGGL(deep::k_deep_scan, dim3(1), dim3(deep::kBlock), 0, s, e->thist, e->tcur,
-                     e->tstat, e->graph_queues);
-  hipLaunchKernelGGL(deep::k_deep_sum, dim3(T), dim3(deep::kNodeCap), 0, s, w, e->node_word,
-                     e->node_kids, e->node_parent, e->nexit, e->node_out, e->tstat);
+                     e->dinfo, e->node_cell, e->nexit, e->tile_n0, e->node_parent, e->node_kids,
+                     e->node_up, e->tstat);
+  hipLaunchKernelGGL(deep::k_deep_nodes, dim3(2 * T), dim3(deep::kNodeCap), 0, s, w,
+                     e->node_parent, e->nexit, e->node_tier, e->node_up, e->node_level, e->thist,
+                     e->tcur, e->graph_queues, e->node_word, e->node_kids, e->node_out, e->tstat);
   hipLaunchKernelGGL(deep::k_deep_levels, dim3(T), dim3(deep::kBlock), 0, s, w, e->dinfo, e->link,
                      e->node_level);
   hipLaunchKernelGGL((deep::k_deep_counts<NM, kChain>), dim3(T), dim3(deep::kCntBlock), 0, s, w, e->rcv,
