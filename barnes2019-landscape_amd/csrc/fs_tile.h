@@ -73,9 +73,9 @@ __device__ __forceinline__ int region_offset(int r) {
 
 // Pass 1: upstream cell counts (ComputeFlowAcc, RB:262-279) and levels
 // (receiver hops to an outlet, the level GenerateOrder assigns, RB:213-254)
-// of the tile's cells.  Every region cell walks its receiver chain once and
-// adds 1 to each cell it passes, itself included, so a cell's count is the
-// number of region cells draining through it -- its whole upstream area when
+// of the tile's cells.  Every cell whose chain touches the tile walks it once
+// and adds 1 to each cell it passes, itself included, so a tile cell's count is
+// the number of region cells draining through it -- its whole upstream area when
 // every level is at most kHalo.  A tile cell deeper than that (or whose chain
 // leaves the region) raises the step's slot; a larger halo, the tile graph or
 // the level path then takes the step.
@@ -297,16 +297,24 @@ struct alignas(16) TilePlan {
   int32_t nhalo;
 };
 
+// Halo cells listed as draining into the tile, all waves' shares together.
+constexpr int kInflowCap = kHalo <= 16 ? 1024 : 4096;
+
 struct AccShared {
   alignas(16) uint32_t w_s[kRegCells];   // accumulation words
   uint32_t mark[kRegCells / 32];
-  uint16_t pre[kRegCells / 32];   // marks before each mark word
+  union {
+    uint16_t pre[kRegCells / 32];   // marks before each mark word
+    uint16_t inflow[kInflowCap];    // before them: halo cells that drain into the tile
+  };
   uint32_t scan[1];               // number of marks
   uint32_t nlist;                 // marked cells appended to hlist
   uint16_t hlist[kHaloCap];       // marked cells in marking order
   int over, maxlev;
+  int full;                       // a wave's share of the inflow list did not suffice
   int hist[kHalo + 1];
 };
+static_assert(sizeof(AccShared) * (kHalo <= 16 ? 4 : 2) <= 160 * 1024, "tiles per CU");
 
 // Slot of region cell c in the plan: a tile cell, or a marked halo cell.
 __device__ __forceinline__ int plan_slot(const uint32_t *mark, const uint16_t *pre, int c) {
@@ -323,6 +331,78 @@ __device__ __forceinline__ uint16_t plan_receiver(const uint32_t *w_s, const uin
   const int s = plan_slot(mark, pre, c + code);
   const bool diag = code != 1 && code != -1 && code != kReg && code != -kReg;
   return static_cast<uint16_t>(s | (diag ? kPlanDiag : 0u));
+}
+
+// One wave's part of the halo cells that drain into the tile: those whose
+// chains enter it from the wave's part of the ring around it.  From each
+// listed cell, eight lanes look at its neighbours for further ones.  Returns the
+// number listed, or -1 when they are more than cap.
+template <int BLOCK>
+__device__ __forceinline__ int list_inflow(const uint32_t *w_s, uint16_t *list, int cap) {
+  constexpr int kRing = 4 * kTile + 4, kShare = (kRing * kWave + BLOCK - 1) / BLOCK;
+  static_assert(kShare <= kWave, "one ring cell per lane");
+  const int lane = threadIdx.x & (kWave - 1);
+  auto below = [&](uint64_t m) { return __popcll(m & ((uint64_t{1} << lane) - 1)); };
+  const int q = static_cast<int>(threadIdx.x / kWave) * kShare + lane;
+  int c = 0;
+  bool in = lane < kShare && q < kRing;
+  if (in) {
+    constexpr int kSide = kTile + 2;
+    int x, y;   // from the ring's corner
+    if (q < kSide) {
+      x = q;
+      y = 0;
+    } else if (q < 2 * kSide) {
+      x = q - kSide;
+      y = kSide - 1;
+    } else {
+      const int k = q - 2 * kSide;
+      x = k < kTile ? 0 : kSide - 1;
+      y = 1 + (k < kTile ? k : k - kTile);
+    }
+    c = (kHalo - 1 + y) * kReg + kHalo - 1 + x;
+    const int code = acc_code(w_s[c]);
+    in = code > kStopMax && (w_s[c + code] & kAccTile) != 0;
+  }
+  uint64_t m = __ballot(in);
+  int n = __popcll(m);
+  if (n > cap) return -1;
+  if (in) list[below(m)] = static_cast<uint16_t>(c);
+  const int off = region_offset(lane & 7);
+  for (int head = 0; head < n;) {
+    __builtin_amdgcn_wave_barrier();   // the list is this wave's alone, and its LDS accesses in order
+    const int item = head + (lane >> 3);
+    c = -1;
+    if (item < n) {
+      c = reinterpret_cast<const volatile uint16_t *>(list)[item] + off;
+      // a step across the region's side leads to a cell whose own code would
+      // cross it back: such codes are kStopLeaves
+      if (static_cast<unsigned>(c) >= static_cast<unsigned>(kRegCells)) {
+        c = -1;
+      } else {
+        const uint32_t wd = w_s[c];
+        if ((wd & kAccTile) || acc_code(wd) != -off) c = -1;
+      }
+    }
+    head = min(head + 8, n);   // those listed now come next
+    m = __ballot(c >= 0);
+    const int found = __popcll(m);
+    if (n + found > cap) return -1;
+    if (c >= 0) list[n + below(m)] = static_cast<uint16_t>(c);
+    n += found;
+  }
+  __builtin_amdgcn_wave_barrier();
+  return n;
+}
+
+// One walk from region cell c (a byte address into w_s), as below.
+__device__ __forceinline__ void walk_chain(uint32_t *w_s, int xa) {
+  for (int round = 0; round <= kHalo; round++) {
+    uint32_t *w = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(w_s) + xa);
+    const int32_t wd = static_cast<int32_t>(atomicAdd(w, 1u));
+    if (wd <= kStopWordMax) break;
+    xa += wd >> 16;
+  }
 }
 
 // Returns nonzero (block-uniform) when a tile cell is deeper than kHalo or
@@ -345,7 +425,7 @@ __device__ __forceinline__ int tile_acc_body(AccShared &sh, const uint8_t *__res
   const int x0 = (t % tiles_x) * kTile, y0 = (t / tiles_x) * kTile;
   const int rx0 = x0 - kHalo, ry0 = y0 - kHalo;
   if (threadIdx.x == 0) {
-    sh.over = sh.maxlev = 0;
+    sh.over = sh.maxlev = sh.full = 0;
     sh.nlist = 0;
   }
   if (threadIdx.x < kHalo + 1) sh.hist[threadIdx.x] = 0;
@@ -360,20 +440,22 @@ __device__ __forceinline__ int tile_acc_body(AccShared &sh, const uint8_t *__res
   if (!done) load_region_words<BLOCK>(rcv, w_s, rx0, ry0, W, H);
   __syncthreads();
   const uint64_t t1 = ph ? wall_clock64() : 0;
-  // Every region cell walks its receiver chain and adds 1 to each cell it
+  // Every tile cell walks its receiver chain and adds 1 to each cell it
   // passes, itself included; the thread's chains advance together, one cell
   // per round.  A walker stops at an outlet (its level is the round it got
   // there), where its chain leaves the region, or after kHalo hops (kHalo + 1
   // rounds).  Walkers hold byte addresses into w_s; a stopped walker holds
   // the complement of the address of the cell that stopped it, so whether it
   // reached an outlet is read back from that cell's code afterwards.
-  constexpr int kPer = kRegCells / BLOCK;
-  static_assert(kPer <= 32, "walkers per thread (bits of live)");
+  constexpr int kPer = kTileCells / BLOCK;
+  static_assert(kPer <= 32 && BLOCK % kTile == 0, "walkers per thread (bits of live)");
+  const int tx = threadIdx.x % kTile, ty0 = threadIdx.x / kTile;   // slot j: row ty0 + j * kRows
+  constexpr int kRows = BLOCK / kTile;
   int xa[kPer], hops[kPer];
   uint32_t live = 0;
 #pragma unroll
   for (int j = 0; j < kPer; j++) {
-    const int i = j * BLOCK + threadIdx.x;
+    const int i = (kHalo + ty0 + j * kRows) * kReg + kHalo + tx;
     hops[j] = 0;
     if (acc_code(w_s[i]) != kStopOutside) {
       xa[j] = 4 * i;
@@ -397,27 +479,33 @@ __device__ __forceinline__ int tile_acc_body(AccShared &sh, const uint8_t *__res
       }
     }
   }
-  // the level of a cell is the length of its walk; only slots whose region
-  // rows can meet the tile's rows hold tile cells
-  int over = 0, deepest = 0;
-  constexpr int kJ0 = (kHalo * kReg) / BLOCK;
-  constexpr int kJ1 = ((kHalo + kTile) * kReg - 1) / BLOCK;
-  // region column and row of slot j's cell, stepped from slot kJ0's
-  constexpr int kStepY = BLOCK / kReg, kStepX = BLOCK % kReg;
-  int lx = (kJ0 * BLOCK + static_cast<int>(threadIdx.x)) % kReg;
-  int ly = (kJ0 * BLOCK + static_cast<int>(threadIdx.x)) / kReg;
-#pragma unroll
-  for (int j = kJ0; j <= kJ1; j++) {
-    const int tx = lx - kHalo, ty = ly - kHalo;
-    lx += kStepX;
-    ly += kStepY;
-    if (lx >= kReg) {
-      lx -= kReg;
-      ly++;
+  // Of the halo's cells, those walk that drain into the tile: about 107 of 5120
+  // on fresh terrain.  The walks are bound by the LDS's returning atomics, and
+  // those of the whole halo are more than half of them (10000 x 10000 after 5
+  // steps: 494 us with all of them, 390 now; with the deep halo, 6000 x 6000
+  // after 330 steps, 385 and 275, 1500 x 1101 48 and 30; 101 x 101, a tile or
+  // less per CU, 16.0 and 14.4).
+  // A wave whose list is full has the whole halo walk.
+  {
+    constexpr int kCap = kInflowCap * kWave / BLOCK;
+    uint16_t *const list = sh.inflow + (threadIdx.x / kWave) * kCap;
+    const int n = list_inflow<BLOCK>(w_s, list, kCap);
+    if (n < 0) sh.full = 1;
+    __syncthreads();
+    if (!sh.full) {
+      for (int q = threadIdx.x & (kWave - 1); q < n; q += kWave) walk_chain(w_s, 4 * list[q]);
+    } else {
+      for (int i = threadIdx.x; i < kRegCells; i += BLOCK) {
+        const uint32_t wd = w_s[i];
+        if (!(wd & kAccTile) && acc_code(wd) != kStopOutside) walk_chain(w_s, 4 * i);
+      }
     }
-    if (static_cast<unsigned>(tx) >= static_cast<unsigned>(kTile) ||
-        static_cast<unsigned>(ty) >= static_cast<unsigned>(kTile))
-      continue;
+  }
+  // the level of a cell is the length of its walk
+  int over = 0, deepest = 0;
+#pragma unroll
+  for (int j = 0; j < kPer; j++) {
+    const int ty = ty0 + j * kRows;
     if (x0 + tx >= W || y0 + ty >= H) continue;     // beyond the grid
     const bool rooted = xa[j] < 0 && acc_code(w_s[~xa[j] >> 2]) == kStopRoot;
     // a level when rooted; stored straight away (a wave's cells are a run of
