@@ -112,6 +112,12 @@ __device__ __forceinline__ u32x4 load_px(const char *row, int bytes, uint32_t of
       __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(row), 0, bytes, kRsrc),
       static_cast<int>(off), 0, 0);
 }
+// off: the lane's offset in bytes bytes, base: the wave's on top of it
+__device__ __forceinline__ u32x4 load_px_at(const char *p, int bytes, uint32_t off, int base) {
+  return __builtin_amdgcn_raw_buffer_load_b128(
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(p), 0, bytes, kRsrc),
+      static_cast<int>(off), base, 0);
+}
 // lane r's value from lane r-1 / r+1 of its 16; lanes 0 / 15 take edge's own
 __device__ __forceinline__ u32x4 from_left(u32x4 v, u32x4 edge) {
   u32x4 o;
@@ -387,9 +393,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void k_conv(ConvSrc src,
   }
 }
 
-// Levels smaller than 8 x 16: one wave per workgroup, 16 columns x 2 rows x 32
-// outputs, the loop over (tap, channel step) with kAhead iterations' operands
-// in flight.  cin is a multiple of 32.
+// Few tiles: one wave per workgroup, 16 columns x 2 rows x 32 outputs, no LDS,
+// the loop over (channel step, tap) or, for levels smaller than 8 x 16, over (tap,
+// channel step), with kAhead iterations' operands in flight.
+template <bool kTapOuter>
 __global__ __launch_bounds__(64) void k_conv_small(ConvSrc src, const uint16_t *__restrict__ wt,
                                                    const float *__restrict__ bias, int relu,
                                                    ConvDst dst, int nout, int H, int W,
@@ -398,34 +405,72 @@ __global__ __launch_bounds__(64) void k_conv_small(ConvSrc src, const uint16_t *
   const int lane = threadIdx.x, g = lane >> 4, r = lane & 15;
   const int n0 = blockIdx.y * kNB;
   const TileAt t = tile_at<R>(blockIdx.x, ntiles, tiles_x, tiles_y);
-  const int cin = src.ca + src.cb, csteps = cin / kKC, steps = 9 * csteps;
+  const int cin = src.ca + src.cb, csteps = (cin + kKC - 1) / kKC, steps = 9 * csteps;
+  // The wave is alone on its SIMD and bound by its instructions (12, 15 or 18
+  // iterations in flight are no faster than 9), so what a lane
+  // adds to an address is computed here, once, and the rest is the loads'
+  // scalar offset (8 x 8 levels of 160 channels: 12.6 us with every
+  // load's address computed anew, 9.5 now).  Columns beyond the image and
+  // channels beyond cin (the network's input has 8) lie out of range.
+  struct Side {
+    const char *img;
+    int bytes, rowbytes, up;
+    uint32_t x[3];
+  };
+  auto side_of = [&](const uint16_t *base, int C, int up) {
+    Side q;
+    q.up = up;
+    q.rowbytes = (W >> up) * C * 2;
+    q.bytes = (H >> up) * q.rowbytes;
+    q.img = reinterpret_cast<const char *>(base) + t.b * static_cast<long>(q.bytes);
+#pragma unroll
+    for (int dx = 0; dx < 3; dx++) {
+      const int x = t.x0 + r + dx - 1;
+      q.x[dx] = static_cast<unsigned>(x) < static_cast<unsigned>(W) && 8 * g < C
+                    ? static_cast<uint32_t>((x >> up) * C + 8 * g) * 2u
+                    : kOob;
+    }
+    return q;
+  };
+  const Side sa = side_of(src.a, src.ca, src.up), sb = side_of(src.b, src.cb, 0);
+  uint32_t wo[2];
+#pragma unroll
+  for (int nt = 0; nt < 2; nt++)
+    wo[nt] = 8 * g < cin ? static_cast<uint32_t>((n0 + frag_out(r, nt)) * cin + 8 * g) * 2u : kOob;
   u32x4 px[kAhead][R], wv[kAhead][2];
   int lt = 0, lc = 0;    // tap and first channel of the next iteration to load
   auto load = [&](int slot) {
-    const bool first_src = lc < src.ca, ok = lt < 9;
-    const int C = first_src ? src.ca : src.cb, c = first_src ? lc : lc - src.ca;
-    const int up = first_src ? src.up : 0;
-    const int rowbytes = (W >> up) * C * 2;
-    const char *base = reinterpret_cast<const char *>(first_src ? src.a : src.b) +
-                       t.b * (H >> up) * static_cast<long>(rowbytes);
-    const int tt = ok ? lt : 0;
-    const int x = t.x0 + r + tt % 3 - 1;
-    const uint32_t off = static_cast<uint32_t>((x >> up) * C + c + 8 * g) * 2u;
+    // iteration s is in slot s % 9; past the last one the first ones come again
+    const int tt = kTapOuter ? lt : slot;
+    const bool first_src = lc < src.ca;
+    const char *img = first_src ? sa.img : sb.img;
+    const int bytes = first_src ? sa.bytes : sb.bytes, up = first_src ? sa.up : 0;
+    const int rowbytes = first_src ? sa.rowbytes : sb.rowbytes;
+    const int c2 = 2 * (first_src ? lc : lc - src.ca);
+    const int dy = tt / 3, dx = tt - 3 * dy;
+    // selects by hand: an index into sa.x would put it into memory
+    const uint32_t x0 = first_src ? sa.x[0] : sb.x[0], x1 = first_src ? sa.x[1] : sb.x[1];
+    const uint32_t x2 = first_src ? sa.x[2] : sb.x[2];
+    const uint32_t x = dx == 0 ? x0 : dx == 1 ? x1 : x2;
 #pragma unroll
     for (int y = 0; y < R; y++) {
-      const int yy = t.y0 + y + tt / 3 - 1;
-      const bool in = ok && static_cast<unsigned>(yy) < static_cast<unsigned>(H);
-      px[slot][y] = load_px(base + static_cast<long>(in ? yy >> up : 0) * rowbytes,
-                            in ? rowbytes : 0, off);
+      const int yy = t.y0 + y + dy - 1;
+      const bool in = static_cast<unsigned>(yy) < static_cast<unsigned>(H);
+      px[slot][y] = load_px_at(img, in ? bytes : 0, x,
+                               in ? (yy >> up) * rowbytes + c2 : 0);
     }
 #pragma unroll
     for (int nt = 0; nt < 2; nt++)
-      wv[slot][nt] = *reinterpret_cast<const u32x4 *>(
-          wt + (static_cast<long>(tt) * nout + n0 + frag_out(r, nt)) * cin + lc + 8 * g);
-    lc += kKC;
-    if (lc >= cin) {
-      lc = 0;
-      lt++;
+      wv[slot][nt] = load_px_at(reinterpret_cast<const char *>(wt), 9 * nout * cin * 2, wo[nt],
+                                (tt * nout * cin + lc) * 2);
+    if (kTapOuter) {
+      lc += kKC;
+      if (lc >= cin) {
+        lc = 0;
+        lt = lt == 8 ? 0 : lt + 1;
+      }
+    } else if (slot == 8) {
+      lc = lc + kKC >= cin ? 0 : lc + kKC;
     }
   };
   f32x4 acc[R][2];
@@ -1099,15 +1144,25 @@ int launch_conv_rows(fs_unet *u, const ConvSrc &src, const uint16_t *wt, const f
 // dst = conv3x3(src) with weights wt [tap][nout][cin].
 int launch_conv(fs_unet *u, const ConvSrc &src, const uint16_t *wt, const float *bias,
                 const ConvDst &dst, int nout, int Hl, int Wl, int relu, int B) {
+  const int tx = (Wl + 15) / 16, ty = (Hl + 1) / 2, tiles = tx * ty * B;
   if (Hl < 8 || Wl < 16) {
-    const int tx = (Wl + 15) / 16, ty = (Hl + 1) / 2, tiles = tx * ty * B;
-    hipLaunchKernelGGL(k_conv_small, dim3(tiles, nout / kNB), dim3(64), 0, u->stream, src, wt, bias,
-                       relu, dst, nout, Hl, Wl, tx, ty, tiles);
+    hipLaunchKernelGGL(k_conv_small<true>, dim3(tiles, nout / kNB), dim3(64), 0, u->stream, src, wt,
+                       bias, relu, dst, nout, Hl, Wl, tx, ty, tiles);
+    return check_launch_u();
+  }
+  // Up to a wave per CU, waves by themselves: a workgroup of k_conv would have
+  // its four on one CU and wait for its weights in every step (one sample of 64
+  // x 64 180 us, by themselves 160; of 128 x 128 174 and 167).  With two or four
+  // waves per CU k_conv is level or ahead (four of 128 x 128: 198 against 204
+  // and 229).
+  if (static_cast<long>(tiles) * (nout / kNB) <= static_cast<long>(u->ncu)) {
+    hipLaunchKernelGGL(k_conv_small<false>, dim3(tiles, nout / kNB), dim3(64), 0, u->stream, src,
+                       wt, bias, relu, dst, nout, Hl, Wl, tx, ty, tiles);
     return check_launch_u();
   }
   // 8 rows a wave wherever that gives every SIMD a wave (1024 of them); below,
-  // 2 rows: one sample of 64 x 64 takes 187 us against 202 with 4 rows, and 32
-  // of 256 x 256 take as long with 4 rows as with 8
+  // 2 rows: four of 128 x 128 take 198 us; 32 of 256 x 256 take as long with 4
+  // rows as with 8
   const long waves = static_cast<long>((Wl + 15) / 16) * (Hl / 8) * B * (nout / kNB);
   if (waves >= 4l * u->ncu)
     return launch_conv_rows<8>(u, src, wt, bias, dst, nout, Hl, Wl, relu, B);
