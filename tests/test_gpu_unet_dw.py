@@ -57,3 +57,27 @@ def test_loss_and_head_bias_against_64_bits(H, W, B):
     eps = (3 + -(-4 * M // (256 * groups)) + 9 + groups) * 2.0 ** -24
     assert abs(loss - np.sum(e * e) / M) <= eps * np.sum(e * e) / M
     assert abs(g[-1] - np.sum(2 * e) / M) <= eps * np.sum(2 * np.abs(e)) / M
+
+
+@pytest.mark.parametrize("H,W", [(32, 64), (256, 256)])
+def test_calls_after_each_other_keep_their_targets(H, W):
+    """Targets and gradients are copied beside the kernels: every call of a
+    sequence with changing batches and targets gives what it gives on a new
+    network (the same kernels on the same inputs; sums by atomics, a handful of
+    whose orders differ, agree within 1e-5 of a layer's norm)."""
+    note("loss and gradients in sequence %dx%d" % (H, W))
+    calls = [(4, 1), (1, 2), (4, 3), (3, 4), (4, 1)]
+    with fa.UNet(H, W, max_batch=4, seed=45) as net:
+        p0 = perturbed_params(net, 46)
+        net.set_params(p0)
+        got = []
+        for B, k in calls:
+            terrain, params, target = sample(k, B, H, W)
+            got.append(net.loss_grad(terrain, params, k * target))
+    for (B, k), (loss, g) in zip(calls, got):
+        terrain, params, target = sample(k, B, H, W)
+        with fa.UNet(H, W, max_batch=4, seed=45) as net:
+            net.set_params(p0)
+            l1, g1 = net.loss_grad(terrain, params, k * target)
+        assert abs(loss - l1) <= 1e-5 * abs(l1)
+        assert np.linalg.norm(g - g1) <= 1e-5 * np.linalg.norm(g1)
