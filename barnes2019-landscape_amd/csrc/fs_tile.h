@@ -26,7 +26,6 @@ constexpr int kRegCells = kReg * kReg;
 constexpr int kAccBlock = kHalo <= 16 ? 512 : 1024;
 constexpr int kAccBlockWide = 1024;
 constexpr int kEroBlock = 1024;
-constexpr uint8_t kOutside = 0xFD;            // region cell beyond the grid
 constexpr uint8_t kEscaped = 0xFF;            // chain leaves the region
 constexpr int kFactCache = 256;               // erosion factors cached in LDS
 
@@ -93,8 +92,7 @@ __device__ __forceinline__ bool in_tile(int lx, int ly) {
 // of its receiver (the byte offset in the word array) or of a stop code.  One
 // atomic add both counts a walker's visit and tells it where to go next: the
 // returned word shifted right by 16 is the step of the walker's byte address.
-// The stop codes lie below every offset (-128..-126 for a 16-cell halo, so
-// that they also fit a byte).
+// The stop codes lie below every offset.
 constexpr uint32_t kAccCount = 0x7FFFu;
 constexpr uint32_t kAccTile = 1u << 15;
 constexpr int kStopRoot = -(kReg + 32);        // an outlet (NO_FLOW)
@@ -103,70 +101,11 @@ constexpr int kStopOutside = kStopRoot + 2;    // beyond the grid
 constexpr int kStopMax = kStopOutside;         // codes <= kStopMax end a walk
 static_assert(kRegCells <= static_cast<int>(kAccCount) && kReg + 1 < -kStopMax,
               "accumulation word layout");
-// offsets and stop codes fit one signed byte: the dword loader's lookups apply
-constexpr bool kByteCodes = kStopRoot >= -128;
-
 static_assert(4 * kStopRoot >= -32768, "byte offsets fit the word's top half");
 // words above this (as signed integers) carry an offset, not a stop code
 constexpr int32_t kStopWordMax = static_cast<int32_t>(
     static_cast<uint32_t>(4 * kStopMax) << 16 | 0xFFFFu);
 __device__ __forceinline__ int acc_code(uint32_t w) { return static_cast<int32_t>(w) >> 18; }
-__device__ __forceinline__ uint32_t acc_word(int code, bool tile) {
-  return static_cast<uint32_t>((4 * code) & 0xFFFF) << 16 | (tile ? kAccTile : 0u);
-}
-
-// Load the receivers of the region into accumulation words with zero counts
-// (every load of a thread is issued before the first LDS store).
-template <int BLOCK>
-__device__ __forceinline__ void load_region_words(const uint8_t *__restrict__ rcv,
-                                                  uint32_t *w_s, int rx0, int ry0, int W,
-                                                  int H) {
-  constexpr int kPer = kRegCells / BLOCK;
-  static_assert(kRegCells % BLOCK == 0, "region must split evenly over the block");
-  // a thread's cells are threadIdx.x + k * BLOCK: step the region column and
-  // row instead of dividing
-  constexpr int kStepY = BLOCK / kReg, kStepX = BLOCK % kReg;
-  const int lx0 = threadIdx.x % kReg, ly0 = threadIdx.x / kReg;
-  const bool inside = rx0 >= 0 && ry0 >= 0 && rx0 + kReg <= W && ry0 + kReg <= H;
-  uint8_t rv[kPer];
-  {
-    int lx = lx0, ly = ly0;
-#pragma unroll
-    for (int k = 0; k < kPer; k++) {
-      const int gx = rx0 + lx, gy = ry0 + ly;
-      const bool in = inside || (gx >= 0 && gx < W && gy >= 0 && gy < H);
-      rv[k] = in ? rcv[static_cast<size_t>(gy) * W + gx] : kOutside;
-      lx += kStepX;
-      ly += kStepY;
-      if (lx >= kReg) {
-        lx -= kReg;
-        ly++;
-      }
-    }
-  }
-  int lx = lx0, ly = ly0;
-#pragma unroll
-  for (int k = 0; k < kPer; k++) {
-    const int i = k * BLOCK + threadIdx.x;
-    const int r = rv[k];
-    int code;
-    if (r == kOutside) {
-      code = kStopOutside;
-    } else if (r >= 8) {
-      code = kStopRoot;
-    } else {
-      int nx = lx, ny = ly;
-      code = region_step(r, nx, ny) ? region_offset(r) : kStopLeaves;
-    }
-    w_s[i] = acc_word(code, in_tile(lx, ly));
-    lx += kStepX;
-    ly += kStepY;
-    if (lx >= kReg) {
-      lx -= kReg;
-      ly++;
-    }
-  }
-}
 
 // Bytes of a 4-entry table, first entry lowest.
 constexpr uint32_t pack4(int a, int b, int c, int d) {
@@ -174,64 +113,94 @@ constexpr uint32_t pack4(int a, int b, int c, int d) {
          static_cast<uint32_t>(c & 0xFF) << 16 | static_cast<uint32_t>(d & 0xFF) << 24;
 }
 
-// Same words as load_region_words, four cells per dword, for a region that
-// lies inside the grid.  Rows of any alignment: the memory takes a dword from
-// any byte address (k_tile_acc at 9999 x 9999: 482 us with the loader by bytes,
-// 398 by dwords; 390 at 10000 x 10000, whose rows are aligned).  v_perm_b32 looks bytes up
-// in an 8-entry table (selector 0..7; 12 gives 0): one lookup turns four
-// receiver directions into four offsets, four more flag the directions that
-// leave the region through its first/last column and row.
+// Load the receivers of the region into accumulation words with zero counts,
+// four cells per dword (every load of a thread is issued before the first LDS
+// store).  v_perm_b32 looks bytes up in an 8-entry table (selector 0..7; 12
+// gives 0): two lookups turn four receiver directions into the low and the high
+// bytes of four offsets, four more flag the directions that leave the region
+// through its first/last column and row, and one permutation puts each cell's
+// two bytes into its word.  Rows of any alignment: the memory takes a dword from
+// any byte address.  Byte by byte, k_tile_acc took 482 us at 9999 x 9999
+// against 398; at the grid's edges, which set the time of small grids, 16.3
+// at 1000 x 1000 and 14.4 at 101 x 101 against 14.6 and 12.8; and with the
+// deep halo 273 at 6000 x 6000 against 235.
 template <int BLOCK>
-__device__ __forceinline__ void load_region_words_x4(const uint8_t *__restrict__ rcv,
-                                                     uint32_t *w_s, int rx0, int ry0, int W) {
+__device__ __forceinline__ void load_region_words(const uint8_t *__restrict__ rcv, uint32_t *w_s,
+                                                  int rx0, int ry0, int W, int H) {
   constexpr int kRowWords = kReg / 4;
   constexpr int kWords = kRegCells / 4;
   constexpr int kIters = (kWords + BLOCK - 1) / BLOCK;
   static_assert(kReg % 4 == 0 && kHalo % 4 == 0 && kTile % 4 == 0, "dword cells");
-  // offsets of directions 0..3 (low table) and 4..7 (high table)
-  constexpr uint32_t kOffLo = pack4(-1, -kReg - 1, -kReg, -kReg + 1);
-  constexpr uint32_t kOffHi = pack4(1, kReg + 1, kReg, kReg - 1);
+  // byte offsets of directions 0..3 (low table) and 4..7 (high table)
+  constexpr int o0 = -4, o1 = 4 * (-kReg - 1), o2 = 4 * -kReg, o3 = 4 * (-kReg + 1);
+  constexpr int o4 = 4, o5 = 4 * (kReg + 1), o6 = 4 * kReg, o7 = 4 * (kReg - 1);
+  constexpr uint32_t kLowLo = pack4(o0, o1, o2, o3), kLowHi = pack4(o4, o5, o6, o7);
+  constexpr uint32_t kTopLo = pack4(o0 >> 8, o1 >> 8, o2 >> 8, o3 >> 8);
+  constexpr uint32_t kTopHi = pack4(o4 >> 8, o5 >> 8, o6 >> 8, o7 >> 8);
   // 0xFF for the directions that leave through each side
   constexpr uint32_t kWestLo = pack4(-1, -1, 0, 0), kWestHi = pack4(0, 0, 0, -1);
   constexpr uint32_t kEastLo = pack4(0, 0, 0, -1), kEastHi = pack4(-1, -1, 0, 0);
   constexpr uint32_t kNorthLo = pack4(0, -1, -1, -1), kNorthHi = 0u;
   constexpr uint32_t kSouthLo = 0u, kSouthHi = pack4(0, -1, -1, -1);
-  const uint8_t *base = rcv + static_cast<size_t>(ry0) * W + rx0;
-  uint32_t v[kIters];
+  // bytes of the stop codes, four times; the three share the high one
+  constexpr uint32_t kRootLow = 0x01010101u * static_cast<uint32_t>((4 * kStopRoot) & 0xFF);
+  constexpr uint32_t kLeavesLow = 0x01010101u * static_cast<uint32_t>((4 * kStopLeaves) & 0xFF);
+  constexpr uint32_t kStopTop = 0x01010101u * static_cast<uint32_t>((4 * kStopRoot >> 8) & 0xFF);
+  constexpr uint32_t kOutsideBits = 0x01010101u * (4 * (kStopOutside - kStopRoot));
+  static_assert((4 * kStopRoot >> 8) == (4 * kStopOutside >> 8) &&
+                    ((4 * kStopRoot) & (4 * (kStopOutside - kStopRoot))) == 0,
+                "stop codes differ in low bits");
+  const bool inside = rx0 >= 0 && ry0 >= 0 && rx0 + kReg <= W && ry0 + kReg <= H;
+  const uint8_t *const base = rcv + static_cast<ptrdiff_t>(ry0) * W + rx0;
+  uint32_t v[kIters], out[kIters];   // receivers; 0xFF for cells beyond the grid
 #pragma unroll
   for (int k = 0; k < kIters; k++) {
     const int d = k * BLOCK + threadIdx.x;
     const int row = d / kRowWords, col = d % kRowWords;
-    v[k] = 0u;
-    if (d < kWords) __builtin_memcpy(&v[k], base + static_cast<size_t>(row) * W + 4 * col, 4);
+    v[k] = out[k] = 0u;
+    if (inside) {
+      if (d < kWords)
+        __builtin_memcpy(&v[k], base + static_cast<ptrdiff_t>(row) * W + 4 * col, 4);
+    } else if (d < kWords) {
+      // rx0 is a multiple of 4, so only the grid's last column cuts a dword:
+      // the row's last four cells hold the part inside (W is at least 5)
+      const int gy = ry0 + row, gx = rx0 + 4 * col, cut = gx + 4 - W;
+      out[k] = ~0u;
+      if (static_cast<unsigned>(gy) < static_cast<unsigned>(H) && gx >= 0 && cut < 4) {
+        const int back = max(cut, 0);
+        __builtin_memcpy(&v[k], base + static_cast<ptrdiff_t>(row) * W + 4 * col - back, 4);
+        v[k] >>= 8 * back;
+        out[k] = back ? ~0u << (8 * (4 - back)) : 0u;
+      }
+    }
   }
 #pragma unroll
   for (int k = 0; k < kIters; k++) {
     const int d = k * BLOCK + threadIdx.x;
     if (d >= kWords) continue;
     const int row = d / kRowWords, col = d % kRowWords;
-    const uint32_t x = v[k];
+    const uint32_t x = v[k] | out[k];
     // outlets are 0xFF bytes: m is 0xFF in their byte lanes
     const uint32_t rb = (x >> 7) & 0x01010101u;
     const uint32_t m = (rb << 8) - rb;
     const uint32_t sel = (x & 0x07070707u & ~m) | (m & 0x0C0C0C0Cu);
-    uint32_t code = __builtin_amdgcn_perm(kOffHi, kOffLo, sel) | (rb << 7);
+    uint32_t low = __builtin_amdgcn_perm(kLowHi, kLowLo, sel) | (m & kRootLow);
+    uint32_t top = __builtin_amdgcn_perm(kTopHi, kTopLo, sel) | (m & kStopTop);
     uint32_t ex = 0;
     if (col == 0) ex |= __builtin_amdgcn_perm(kWestHi, kWestLo, sel) & 0x000000FFu;
     if (col == kRowWords - 1) ex |= __builtin_amdgcn_perm(kEastHi, kEastLo, sel) & 0xFF000000u;
     if (row == 0) ex |= __builtin_amdgcn_perm(kNorthHi, kNorthLo, sel);
     if (row == kReg - 1) ex |= __builtin_amdgcn_perm(kSouthHi, kSouthLo, sel);
-    constexpr uint32_t kLeaves4 = 0x01010101u * static_cast<uint32_t>(kStopLeaves & 0xFF);
-    code = (code & ~ex) | (ex & kLeaves4);
+    low = (low & ~ex) | (ex & kLeavesLow) | (out[k] & kOutsideBits);
+    top = (top & ~ex) | (ex & kStopTop);
     const bool tile = static_cast<unsigned>(row - kHalo) < static_cast<unsigned>(kTile) &&
                       static_cast<unsigned>(col - kHalo / 4) < static_cast<unsigned>(kTile / 4);
     const uint32_t t = tile ? kAccTile : 0u;
-    // byte b of code, sign-extended and times four, into bits 16-31 of word b
     uint4 q;
-    q.x = (static_cast<uint32_t>(static_cast<int32_t>(code << 24) >> 6) & 0xFFFC0000u) | t;
-    q.y = (static_cast<uint32_t>(static_cast<int32_t>(code << 16) >> 6) & 0xFFFC0000u) | t;
-    q.z = (static_cast<uint32_t>(static_cast<int32_t>(code << 8) >> 6) & 0xFFFC0000u) | t;
-    q.w = (static_cast<uint32_t>(static_cast<int32_t>(code) >> 6) & 0xFFFC0000u) | t;
+    q.x = __builtin_amdgcn_perm(top, low, 0x04000C0Cu) | t;
+    q.y = __builtin_amdgcn_perm(top, low, 0x05010C0Cu) | t;
+    q.z = __builtin_amdgcn_perm(top, low, 0x06020C0Cu) | t;
+    q.w = __builtin_amdgcn_perm(top, low, 0x07030C0Cu) | t;
     *reinterpret_cast<uint4 *>(&w_s[4 * d]) = q;
   }
 }
@@ -431,14 +400,7 @@ __device__ __forceinline__ int tile_acc_body(AccShared &sh, const uint8_t *__res
   }
   if (threadIdx.x < kHalo + 1) sh.hist[threadIdx.x] = 0;
   if (threadIdx.x < kRegCells / 32) sh.mark[threadIdx.x] = 0;
-  bool done = false;
-  if constexpr (kByteCodes) {
-    if (rx0 >= 0 && ry0 >= 0 && rx0 + kReg <= W && ry0 + kReg <= H) {
-      load_region_words_x4<BLOCK>(rcv, w_s, rx0, ry0, W);
-      done = true;
-    }
-  }
-  if (!done) load_region_words<BLOCK>(rcv, w_s, rx0, ry0, W, H);
+  load_region_words<BLOCK>(rcv, w_s, rx0, ry0, W, H);
   __syncthreads();
   const uint64_t t1 = ph ? wall_clock64() : 0;
   // Every tile cell walks its receiver chain and adds 1 to each cell it
