@@ -679,7 +679,9 @@ inline ErodeConst make_erode_const(const fs_params &p, int *nmode) {
   k.ud = p.ueq * p.dt;
   k.neq = p.neq;
   k.tol = p.tol;
-  *nmode = (p.neq == 1.0) ? 1 : (p.neq == 2.0) ? 2 : 0;
+  // the short forms of the solve take at least one iteration; with an infinite
+  // tolerance the reference's loop takes none, and neither does mode 0's
+  *nmode = !std::isfinite(p.tol) ? 0 : (p.neq == 1.0) ? 1 : (p.neq == 2.0) ? 2 : 0;
   return k;
 }
 
