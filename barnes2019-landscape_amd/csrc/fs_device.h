@@ -754,7 +754,8 @@ __device__ __forceinline__ double newton_plain(double h0, double hn, double fact
 // Control.  n = 1 is linear: the second iteration confirms the first.  n = 2
 // takes kNewtonFirst iterations before the wave first looks whether all its
 // lanes have converged (nearly every cell needs five to seven); a lane keeps
-// the iterate at which its own loop would have ended.
+// the iterate at which its own loop would have ended.  The iteration at which
+// the plain loop fails, converged or not, is left to it.
 __device__ __forceinline__ double refined_rcp(double b) {
   double y = __builtin_amdgcn_rcp(b);
   y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
@@ -815,7 +816,7 @@ __device__ __forceinline__ double newton_solve(double h0, double hn, double fact
 #pragma unroll
     for (int it = 0; it < kNewtonFirst; it++) iterate();
 #pragma nounroll
-    for (int it = kNewtonFirst; it < kNewtonCap && __ballot(!done) != 0; it++) iterate();
+    for (int it = kNewtonFirst; it < kNewtonCap - 1 && __ballot(!done) != 0; it++) iterate();
     if (p.ok & done & (fabs(hn) <= h0) & (fabs(res) >= kNewtonSmall)) return res;
     return newton_plain<2>(h0, hn, fact, k, hdr);
   } else {
