@@ -1208,6 +1208,29 @@ DwPlan dw_plan(int cout, int cin, int Hl, int Wl, int B) {
   return p;
 }
 
+// Pixels per chunk of the per-tap kernel, in whole 32s: up to 64 chunks, a few more
+// where rounding the chunk down leaves a rest.  The number of chunks therefore
+// does not always grow with the batch (352 x 352, level 2: 64 for 32 samples, 65 for
+// 22).
+struct TapChunks {
+  long chunk;
+  int n;
+};
+TapChunks tap_chunks(long M) {
+  const long chunk = std::max<long>(2048, (M + 63) / 64 / 32 * 32);
+  return {chunk, static_cast<int>((M + chunk - 1) / chunk)};
+}
+
+// Partial sums that the weight gradient of one layer needs for any batch up to
+// max_batch.
+size_t part_need(const Conv &c, int Hl, int Wl, int max_batch) {
+  const DwPlan dp = dw_plan(c.cout, c.cin, Hl, Wl, max_batch);
+  long chunks = dp.max_chunks;   // grows with the batch
+  for (int B = 1; !dp.tiled && B <= max_batch; B++)
+    chunks = std::max<long>(chunks, tap_chunks(static_cast<long>(B) * Hl * Wl).n);
+  return static_cast<size_t>(chunks) * 9 * c.cout * c.cin;
+}
+
 // Gradients of one conv layer from gz, the gradient of its output before the
 // ReLU: weight and bias gradients, and the input gradient into gin (if given).
 int conv_bwd(fs_unet *u, const Conv &c, const ConvSrc &in, const Tensor &gz, const ConvDst *gin,
@@ -1234,15 +1257,14 @@ int conv_bwd(fs_unet *u, const Conv &c, const ConvSrc &in, const Tensor &gz, con
                        dp.nchunks);
     FS_TRY(check_launch_u());
   } else {
-    const long chunk = std::max<long>(2048, (M + 63) / 64 / 32 * 32);
-    const int nchunks = static_cast<int>((M + chunk - 1) / chunk);
-    if (static_cast<size_t>(nchunks) * wn > u->part_n) return FS_ERR_INTERNAL;
+    const TapChunks tc = tap_chunks(M);
+    if (static_cast<size_t>(tc.n) * wn > u->part_n) return FS_ERR_INTERNAL;
     const int tiles = ((c.cout + 63) / 64) * ((c.cin + 63) / 64);
-    hipLaunchKernelGGL(k_conv3x3_dw, dim3(tiles, 9, nchunks), dim3(256), 0, u->stream, gz.d,
-                       c.cout, in, u->part, Hl, Wl, chunk, M);
+    hipLaunchKernelGGL(k_conv3x3_dw, dim3(tiles, 9, tc.n), dim3(256), 0, u->stream, gz.d,
+                       c.cout, in, u->part, Hl, Wl, tc.chunk, M);
     FS_TRY(check_launch_u());
     hipLaunchKernelGGL(k_reduce_chunks, dim3(grid_for(static_cast<long>(wn))), dim3(256), 0,
-                       u->stream, u->part, u->g + c.woff, static_cast<long>(wn), nchunks);
+                       u->stream, u->part, u->g + c.woff, static_cast<long>(wn), tc.n);
     FS_TRY(check_launch_u());
   }
   if (!dp.tiled) {
@@ -1470,13 +1492,8 @@ int fs_unet_create(int height, int width, int max_batch, uint64_t seed, int devi
     FS_TRY(fs::dev_alloc(&c.wb, 9ul * c.cout * c.cin));
   }
   size_t part = 0;
-  for (const Conv &c : u->conv) {
-    const long M = pixels(u, c.level, max_batch);
-    const long chunk = std::max<long>(2048, (M + 63) / 64 / 32 * 32);
-    part = std::max(part, static_cast<size_t>((M + chunk - 1) / chunk) * 9 * c.cout * c.cin);
-    const DwPlan dp = dw_plan(c.cout, c.cin, height >> c.level, width >> c.level, max_batch);
-    if (dp.tiled) part = std::max(part, static_cast<size_t>(dp.max_chunks) * 9 * c.cout * c.cin);
-  }
+  for (const Conv &c : u->conv)
+    part = std::max(part, part_need(c, height >> c.level, width >> c.level, max_batch));
   u->part_n = part;
   FS_TRY(fs::dev_alloc(&u->part, part));
   FS_TRY(alloc_tensor(u, u->x0, kInChannels, 0));
