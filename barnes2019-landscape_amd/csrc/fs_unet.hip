@@ -1609,12 +1609,12 @@ int fs_unet_loss_grad(fs_unet *u, const float *terrain, const float *params, con
   // gradients for 32 samples of 256 x 256: 4.08 ms one after the other, now
   // 3.55): the targets' while the forward pass, which does not read them, runs,
   // most of the gradients' during the last layers' backward pass.
-  FS_HIP_TRY(hipEventRecord(u->copy_ev[0], u->stream));
-  FS_TRY(upload_batch(u, terrain, params, nullptr, batch));
-  FS_TRY(forward(u, u->terrain, u->params_in, batch));
   const size_t npix = static_cast<size_t>(batch) * u->H * u->W;
   const size_t head = grad ? u->conv[enc(kDeepLevel, 0)].woff : 0;
   int st = [&] {
+    FS_HIP_TRY(hipEventRecord(u->copy_ev[0], u->stream));
+    FS_TRY(upload_batch(u, terrain, params, nullptr, batch));
+    FS_TRY(forward(u, u->terrain, u->params_in, batch));
     FS_HIP_TRY(hipStreamWaitEvent(u->copy, u->copy_ev[0], 0));
     FS_HIP_TRY(hipMemcpyAsync(u->tgt, tgt, npix * sizeof(float), hipMemcpyHostToDevice, u->copy));
     FS_HIP_TRY(hipEventRecord(u->copy_ev[1], u->copy));
@@ -1630,11 +1630,16 @@ int fs_unet_loss_grad(fs_unet *u, const float *terrain, const float *params, con
     FS_HIP_TRY(hipMemcpyAsync(loss, u->head_acc, sizeof(float), hipMemcpyDeviceToHost, u->stream));
     return FS_OK;
   }();
-  // the caller's arrays are free again, whatever happened
-  if (hipStreamSynchronize(u->copy) != hipSuccess && st == FS_OK) st = FS_ERR_HIP;
-  if (st != FS_OK) return st;
-  FS_HIP_TRY(hipStreamSynchronize(u->stream));
-  return FS_OK;
+  // the caller's arrays are free again, whatever happened: both streams are
+  // waited for, and the first failure is reported
+  for (hipStream_t s : {u->copy, u->stream}) {
+    const int waited = [&] {
+      FS_HIP_TRY(hipStreamSynchronize(s));
+      return FS_OK;
+    }();
+    if (st == FS_OK) st = waited;
+  }
+  return st;
 }
 
 int fs_unet_set_data(fs_unet *u, const float *terrain, const float *params, const float *tgt,

@@ -41,3 +41,11 @@ def test_every_batch_has_its_workspace(check, H, W, max_batch):
     """The partial sums of a smaller batch can need more chunks than those of
     the largest."""
     assert check("batches", H, W, max_batch) == [[str(max_batch)]]
+
+
+def test_a_failed_call_waits_for_its_copies(check):
+    """Whichever runtime call of loss_grad fails, no copy to or from the caller's
+    arrays is left behind, and the failure is reported."""
+    left = check("failures", 64, 64, 4)
+    assert left[:-1] == []
+    assert int(left[-1][0]) > 60
