@@ -26,6 +26,7 @@
 #include <string>
 #include <vector>
 
+#include "fs_conv_rows.h"
 #include "fs_internal.h"
 #include "fs_hostutil.h"
 
@@ -413,16 +414,21 @@ __global__ __launch_bounds__(64) void k_conv_small(ConvSrc src, const uint16_t *
   // load's address computed anew, 9.5 now).  Columns beyond the image and
   // channels beyond cin (the network's input has 8) lie out of range.
   struct Side {
-    const char *img;
-    int bytes, rowbytes, up;
+    const char *rows;      // the rows the tile reads (fs_conv_rows.h)
+    int bytes, up;
+    uint32_t rowbytes, skip;
     uint32_t x[3];
   };
   auto side_of = [&](const uint16_t *base, int C, int up) {
     Side q;
+    const int rowbytes = (W >> up) * C * 2;
+    const fs::ConvRows at = fs::conv_rows(t.y0, R, H, up, rowbytes);
     q.up = up;
-    q.rowbytes = (W >> up) * C * 2;
-    q.bytes = (H >> up) * q.rowbytes;
-    q.img = reinterpret_cast<const char *>(base) + t.b * static_cast<long>(q.bytes);
+    q.rowbytes = static_cast<uint32_t>(rowbytes);
+    q.skip = at.skip;
+    q.bytes = static_cast<int>(at.bytes);
+    q.rows = reinterpret_cast<const char *>(base) + t.b * (H >> up) * static_cast<long>(rowbytes) +
+             at.start;
 #pragma unroll
     for (int dx = 0; dx < 3; dx++) {
       const int x = t.x0 + r + dx - 1;
@@ -443,9 +449,10 @@ __global__ __launch_bounds__(64) void k_conv_small(ConvSrc src, const uint16_t *
     // iteration s is in slot s % 9; past the last one the first ones come again
     const int tt = kTapOuter ? lt : slot;
     const bool first_src = lc < src.ca;
-    const char *img = first_src ? sa.img : sb.img;
+    const char *rows = first_src ? sa.rows : sb.rows;
     const int bytes = first_src ? sa.bytes : sb.bytes, up = first_src ? sa.up : 0;
-    const int rowbytes = first_src ? sa.rowbytes : sb.rowbytes;
+    const uint32_t rowbytes = first_src ? sa.rowbytes : sb.rowbytes;
+    const uint32_t skip = first_src ? sa.skip : sb.skip;
     const int c2 = 2 * (first_src ? lc : lc - src.ca);
     const int dy = tt / 3, dx = tt - 3 * dy;
     // selects by hand: an index into sa.x would put it into memory
@@ -456,8 +463,9 @@ __global__ __launch_bounds__(64) void k_conv_small(ConvSrc src, const uint16_t *
     for (int y = 0; y < R; y++) {
       const int yy = t.y0 + y + dy - 1;
       const bool in = static_cast<unsigned>(yy) < static_cast<unsigned>(H);
-      px[slot][y] = load_px_at(img, in ? bytes : 0, x,
-                               in ? (yy >> up) * rowbytes + c2 : 0);
+      px[slot][y] = load_px_at(
+          rows, in ? bytes : 0, x,
+          in ? static_cast<int>(fs::conv_row_offset(yy, up, rowbytes, skip)) + c2 : 0);
     }
 #pragma unroll
     for (int nt = 0; nt < 2; nt++)
