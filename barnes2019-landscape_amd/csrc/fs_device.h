@@ -1105,10 +1105,26 @@ enum PhaseId {
 };
 static_assert(kPhCount <= kPhaseStride, "phase row");
 
-// This workgroup's phase row, or null when it is not sampled.
+// This workgroup's phase row, or null when it is not sampled.  Workgroups go to
+// the eight XCDs in turn: eight in a row are sampled, one on each.
 __device__ __forceinline__ unsigned long long *phase_row(unsigned long long *phase) {
-  if (!phase || blockIdx.x % kPhaseSample != 0) return nullptr;
-  return phase + (blockIdx.x / kPhaseSample % kPhaseSlots) * kPhaseStride;
+  const unsigned turn = blockIdx.x / 8;
+  if (!phase || turn % kPhaseSample != 0) return nullptr;
+  return phase + (8 * (turn / kPhaseSample) + blockIdx.x % 8) % kPhaseSlots * kPhaseStride;
+}
+// A sampled workgroup's clock at its k-th phase boundary, kept in LDS: in scalar
+// registers the times took the timed erosion from 70 to 82 of them, and beyond 80
+// a CU holds one workgroup of 1024 threads instead of two (1039 us against 610
+// at 10000 x 10000; with the times in LDS 609).
+__device__ __forceinline__ void phase_mark(const unsigned long long *row, uint64_t *clock, int k) {
+  if (row && threadIdx.x == 0) clock[k] = wall_clock64();
+}
+// Ends the last of the phases first .. first + 3, and adds them to the row.
+__device__ __forceinline__ void phase_end(unsigned long long *row, uint64_t *clock, int first) {
+  if (row && threadIdx.x == 0) {
+    clock[4] = wall_clock64();
+    for (int k = 0; k < 4; k++) atomicAdd(&row[first + k], clock[k + 1] - clock[k]);
+  }
 }
 
 // ---------------------------------------------------------------------------

@@ -283,6 +283,7 @@ struct AccShared {
   int over, maxlev;
   int full;                       // a wave's share of the inflow list did not suffice
   int hist[kHalo + 1];
+  uint64_t clock[5];              // phase boundaries of a sampled workgroup
 };
 static_assert(sizeof(AccShared) * (kHalo <= 16 ? 4 : 2) <= 160 * 1024, "tiles per CU");
 
@@ -391,7 +392,7 @@ __device__ __forceinline__ int tile_acc_body(AccShared &sh, const uint8_t *__res
   static_assert(kRegCells / 32 <= BLOCK && kHalo + 1 <= BLOCK, "one mark word per thread");
   uint32_t *w_s = sh.w_s;
   unsigned long long *const ph = phase_row(phase);
-  const uint64_t t0 = ph ? wall_clock64() : 0;
+  phase_mark(ph, sh.clock, 0);
   const int x0 = (t % tiles_x) * kTile, y0 = (t / tiles_x) * kTile;
   const int rx0 = x0 - kHalo, ry0 = y0 - kHalo;
   if (threadIdx.x == 0) {
@@ -402,7 +403,7 @@ __device__ __forceinline__ int tile_acc_body(AccShared &sh, const uint8_t *__res
   if (threadIdx.x < kRegCells / 32) sh.mark[threadIdx.x] = 0;
   load_region_words<BLOCK>(rcv, w_s, rx0, ry0, W, H);
   __syncthreads();
-  const uint64_t t1 = ph ? wall_clock64() : 0;
+  phase_mark(ph, sh.clock, 1);
   // Every tile cell walks its receiver chain and adds 1 to each cell it
   // passes, itself included; the thread's chains advance together, one cell
   // per round.  A walker stops at an outlet (its level is the round it got
@@ -487,11 +488,8 @@ __device__ __forceinline__ int tile_acc_body(AccShared &sh, const uint8_t *__res
     for (int d = 1; d < kWave; d <<= 1) deepest = max(deepest, __shfl_xor(deepest, d));
     if ((threadIdx.x & (kWave - 1)) == 0 && deepest > 0) atomicMax(&sh.maxlev, deepest);
   }
-  uint64_t t2 = 0;
-  if (ph) {
-    __syncthreads();
-    t2 = wall_clock64();
-  }
+  if (ph) __syncthreads();
+  phase_mark(ph, sh.clock, 2);
   mark_halo_chains<BLOCK>(w_s, sh.mark, sh.hlist, &sh.nlist);
   __syncthreads();
   // halo slot bases: one wave scans the mark words, kMarkRun per lane
@@ -566,11 +564,8 @@ __device__ __forceinline__ int tile_acc_body(AccShared &sh, const uint8_t *__res
     }
     if (threadIdx.x == 0) plan->nhalo = static_cast<int32_t>(nhalo);
   }
-  uint64_t t3 = 0;
-  if (ph) {
-    __syncthreads();
-    t3 = wall_clock64();
-  }
+  if (ph) __syncthreads();
+  phase_mark(ph, sh.clock, 3);
   for (int it = 0; it < kTileCells / BLOCK; it++) {
     const int i = it * BLOCK + threadIdx.x;
     const int tx = i % kTile, ty = i / kTile;
@@ -579,16 +574,8 @@ __device__ __forceinline__ int tile_acc_body(AccShared &sh, const uint8_t *__res
     const size_t gi = static_cast<size_t>(gy) * W + gx;
     cnt[gi] = w_s[(ty + kHalo) * kReg + tx + kHalo] & kAccCount;
   }
-  if (ph) {
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      const uint64_t t4 = wall_clock64();
-      atomicAdd(&ph[kPhAccLoad], t1 - t0);
-      atomicAdd(&ph[kPhAccWalk], t2 - t1);
-      atomicAdd(&ph[kPhAccPlan], t3 - t2);
-      atomicAdd(&ph[kPhAccStore], t4 - t3);
-    }
-  }
+  if (ph) __syncthreads();
+  phase_end(ph, sh.clock, kPhAccLoad);
   return tile_over;
 }
 
@@ -642,6 +629,7 @@ struct EroShared {
   uint32_t scan[kEroBlock / kWave + 1];
   int wcount[kHalo + 1][kEroBlock / kWave];
   int ltotal[kHalo + 1], loff[kHalo + 2];
+  uint64_t clock[5];            // phase boundaries of a sampled workgroup
 };
 
 template <int NMODE>
@@ -656,7 +644,7 @@ __device__ __forceinline__ void tile_erode_body(EroShared &sh, const double *__r
                                                 unsigned long long *phase = nullptr) {
   constexpr int kWaves = kEroBlock / kWave;
   unsigned long long *const ph = phase_row(phase);
-  const uint64_t t0 = ph ? wall_clock64() : 0;
+  phase_mark(ph, sh.clock, 0);
   constexpr int kKeys = kHalo + 1;
   constexpr int kTilePer = kTileCells / kEroBlock;
   constexpr int kSlotPer = (kSlots + kEroBlock - 1) / kEroBlock;
@@ -786,7 +774,7 @@ __device__ __forceinline__ void tile_erode_body(EroShared &sh, const double *__r
       list[e] = 0xFFFF;
   __syncthreads();
   const int nchunks = loff[kKeys] / kWave, root_chunks = loff[1] / kWave;
-  const uint64_t t1 = ph ? wall_clock64() : 0;
+  phase_mark(ph, sh.clock, 1);
   // level 0 first: uplift of the interior outlets; rings 0 and 1 stay fixed
   int ch = wave;
   for (; ch < root_chunks; ch += kWaves) {
@@ -804,11 +792,8 @@ __device__ __forceinline__ void tile_erode_body(EroShared &sh, const double *__r
     if (gx >= 2 && gx < W - 2 && gy >= 2 && gy < H - 2) hs[sl] += k.ud;
     __hip_atomic_store(&d_s[sl], kDone, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
   }
-  uint64_t tm = 0;
-  if (ph) {
-    __syncthreads();
-    tm = wall_clock64();
-  }
+  if (ph) __syncthreads();
+  phase_mark(ph, sh.clock, 2);
   // levels 1 and up, each cell as soon as its receiver is done
   for (; ch < nchunks; ch += kWaves) {
     const int sl = list[ch * kWave + lane];
@@ -842,7 +827,7 @@ __device__ __forceinline__ void tile_erode_body(EroShared &sh, const double *__r
     __hip_atomic_store(&d_s[sl], kDone, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
   }
   __syncthreads();
-  const uint64_t t2 = ph ? wall_clock64() : 0;
+  phase_mark(ph, sh.clock, 3);
 #pragma unroll
   for (int j = 0; j < kTilePer; j++) {
     const int tj = j * kEroBlock + threadIdx.x;
@@ -850,16 +835,8 @@ __device__ __forceinline__ void tile_erode_body(EroShared &sh, const double *__r
     if (gx >= W || gy >= H) continue;
     h_new[static_cast<size_t>(gy) * W + gx] = hs[tj];
   }
-  if (ph) {
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      const uint64_t t3 = wall_clock64();
-      atomicAdd(&ph[kPhEroBucket], t1 - t0);
-      atomicAdd(&ph[kPhEroRoots], tm - t1);
-      atomicAdd(&ph[kPhEroLoop], t2 - tm);
-      atomicAdd(&ph[kPhEroStore], t3 - t2);
-    }
-  }
+  if (ph) __syncthreads();
+  phase_end(ph, sh.clock, kPhEroBucket);
 }
 
 template <int NMODE, bool kTimed>
