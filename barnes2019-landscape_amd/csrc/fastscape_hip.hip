@@ -78,6 +78,13 @@ struct Span {
   bool small;
 };
 
+// How a tile step's time divides over its three kernels (receivers,
+// accumulation, erosion), and those of the two tile kernels over the stages.
+struct TileShares {
+  double kernel[3];
+  double acc[6], ero[6];   // FS_T_RECEIVERS + i
+};
+
 struct fs_model {
   int W = 0, H = 0;
   int32_t N = 0;
@@ -108,11 +115,11 @@ struct fs_model {
   unsigned long long *ticket = nullptr;
   unsigned long long *phase = nullptr;   // tile kernels' phase ticks (stage timers)
   int32_t *fill_flag = nullptr;          // per launch of a batch: it changed a cell
-  long long steps_in_call = 0;           // steps taken by the current fs_run / fs_step
   bool fill_mode = false;                // fill depressions before every step
 
   // host mirrors
   int32_t *hdr_h = nullptr;      // pinned: header + level counts
+  uint64_t *phase_h = nullptr;   // pinned: the phase ticks
   int32_t *levels_h = nullptr;   // pinned: levels uploaded each step
   std::vector<int32_t> counts, levels;
   int32_t nlevel = 0, maxdepth = 0, prev_maxdepth = FS_MAX_LEVELS;
@@ -134,12 +141,12 @@ struct fs_model {
   bool ev_pending[2] = {false, false};
   int ev_cur = 0;                     // level-path steps alternate the two sets
   // Tile and tile-graph steps are not bracketed by events one by one: a batch
-  // (or a run of tile-graph steps) is, and its first step's kernels are the
-  // sample its time is split by.
+  // is, and split by the shares of the last sampled step that was taken; a run
+  // of tile-graph steps by its first one's.
   hipEvent_t tev[5] = {};             // batch: start, the sampled step's kernels, end
-  double tile_ms = 0;                 // tile batches' time not yet split over the stages
-  double samp_ms[3] = {};             // sampled receivers, accumulation, erosion
-  long long since_sample = 0;         // tile steps since the last sampled one
+  TileShares shares{};                // of the last sample
+  uint64_t phase_seen[kPhaseStride] = {};   // the phase ticks' sums when last read
+  long long since_sample = kPhaseEvery;     // tile steps since the last sample
   hipEvent_t gev[8] = {};             // tile-graph run: its first step's stages, end
   bool graph_open = false, graph_pending = false;
   int batch = 4;                      // tile steps launched before the host looks
@@ -266,63 +273,56 @@ int graph_collect(fs_model *m) {
   return FS_OK;
 }
 
-// Split the tile batches' event time over the reference's stages: over the
-// three kernels in proportion to the sampled steps' event times, and the two
-// tile kernels' shares in proportion to the phase ticks their sampled
-// workgroups recorded on those steps:
+// The shares of a sampled step whose kernels took ms: the two tile kernels' by
+// the phase ticks that their sampled workgroups recorded in it:
 // k_tile_acc's region load -> DetermineDonors, its chain walks and
 // count/level stores -> FlowAcc, its halo-chain marking and erosion plan ->
 // GenerateOrder; k_tile_erode's level bucketing -> GenerateOrder, its outlet
 // uplift -> Uplift, its wavefront and stores -> Erosion.
-int split_tile_time(fs_model *m) {
-  if (m->tile_ms <= 0) return FS_OK;
-  double ph[kPhaseStride] = {};
-  if (m->phase) {
-    std::vector<unsigned long long> raw(static_cast<size_t>(kPhaseSlots) * kPhaseStride);
-    FS_HIP_TRY(hipSetDevice(m->device));
-    FS_HIP_TRY(hipStreamSynchronize(m->stream));
-    FS_HIP_TRY(hipMemcpy(raw.data(), m->phase, raw.size() * sizeof(raw[0]),
-                         hipMemcpyDeviceToHost));
-    for (int r = 0; r < kPhaseSlots; r++)
-      for (int i = 0; i < kPhaseStride; i++)
-        ph[i] += static_cast<double>(raw[static_cast<size_t>(r) * kPhaseStride + i]);
-    FS_HIP_TRY(hipMemset(m->phase, 0, raw.size() * sizeof(raw[0])));
-  }
-  const double samp = m->samp_ms[0] + m->samp_ms[1] + m->samp_ms[2];
-  const double per = samp > 0 ? m->tile_ms / samp : 0;
-  m->stage_ms[FS_T_RECEIVERS] += per * m->samp_ms[0];
-  const double acc_ms = per * m->samp_ms[1], ero_ms = per * m->samp_ms[2];
-  const double acc = ph[kPhAccLoad] + ph[kPhAccWalk] + ph[kPhAccPlan] + ph[kPhAccStore];
+TileShares tile_shares(const double (&ms)[3], const double *ticks) {
+  TileShares s{};
+  const double all = ms[0] + ms[1] + ms[2];
+  for (int i = 0; i < 3; i++) s.kernel[i] = all > 0 ? ms[i] / all : 1.0 / 3;
+  auto at = [](double *stage, int t) -> double & { return stage[t - FS_T_RECEIVERS]; };
+  const double acc =
+      ticks[kPhAccLoad] + ticks[kPhAccWalk] + ticks[kPhAccPlan] + ticks[kPhAccStore];
   if (acc > 0) {
-    m->stage_ms[FS_T_DONORS] += acc_ms * ph[kPhAccLoad] / acc;
-    m->stage_ms[FS_T_FLOWACC] += acc_ms * (ph[kPhAccWalk] + ph[kPhAccStore]) / acc;
-    m->stage_ms[FS_T_ORDER] += acc_ms * ph[kPhAccPlan] / acc;
+    at(s.acc, FS_T_DONORS) = ticks[kPhAccLoad] / acc;
+    at(s.acc, FS_T_FLOWACC) = (ticks[kPhAccWalk] + ticks[kPhAccStore]) / acc;
+    at(s.acc, FS_T_ORDER) = ticks[kPhAccPlan] / acc;
   } else {
-    m->stage_ms[FS_T_FLOWACC] += acc_ms;
+    at(s.acc, FS_T_FLOWACC) = 1;
   }
-  const double ero = ph[kPhEroBucket] + ph[kPhEroRoots] + ph[kPhEroLoop] + ph[kPhEroStore];
+  const double ero =
+      ticks[kPhEroBucket] + ticks[kPhEroRoots] + ticks[kPhEroLoop] + ticks[kPhEroStore];
   if (ero > 0) {
-    m->stage_ms[FS_T_ORDER] += ero_ms * ph[kPhEroBucket] / ero;
-    m->stage_ms[FS_T_UPLIFT] += ero_ms * ph[kPhEroRoots] / ero;
-    m->stage_ms[FS_T_EROSION] += ero_ms * (ph[kPhEroLoop] + ph[kPhEroStore]) / ero;
+    at(s.ero, FS_T_ORDER) = ticks[kPhEroBucket] / ero;
+    at(s.ero, FS_T_UPLIFT) = ticks[kPhEroRoots] / ero;
+    at(s.ero, FS_T_EROSION) = (ticks[kPhEroLoop] + ticks[kPhEroStore]) / ero;
   } else {
-    m->stage_ms[FS_T_EROSION] += ero_ms;
+    at(s.ero, FS_T_EROSION) = 1;
   }
-  m->tile_ms = 0;
-  for (double &v : m->samp_ms) v = 0;
-  return FS_OK;
+  return s;
 }
 
-// The stage times of every step so far, into the timers.
-int fold_timers(fs_model *m) {
-  FS_TRY(split_tile_time(m));
+// Divides ms over the stages by the shares of the kernels that ran.
+void add_tile_time(fs_model *m, double ms, const TileShares &s, bool recv, bool erode) {
+  const double k0 = recv ? s.kernel[0] : 0, k1 = s.kernel[1], k2 = erode ? s.kernel[2] : 0;
+  const double sum = k0 + k1 + k2;
+  if (!(sum > 0)) return;
+  m->stage_ms[FS_T_RECEIVERS] += ms * k0 / sum;
+  for (int i = 0; i < 6; i++)
+    m->stage_ms[FS_T_RECEIVERS + i] += ms * (k1 * s.acc[i] + k2 * s.ero[i]) / sum;
+}
+
+// Whole microseconds of the stage times so far into the timers.
+void fold_timers(fs_model *m) {
   for (int i = 0; i < 6; i++) {
     const double ms = m->stage_ms[FS_T_RECEIVERS + i];
     const uint64_t whole = static_cast<uint64_t>(ms * 1000.0);
     m->timer_us[FS_T_RECEIVERS + i] += whole;
     m->stage_ms[FS_T_RECEIVERS + i] = ms - static_cast<double>(whole) / 1000.0;
   }
-  return FS_OK;
 }
 
 int check_launch() {
@@ -373,6 +373,7 @@ void free_model(fs_model *m) {
                     static_cast<void *>(m->graph_grid), static_cast<void *>(m->graph_list)})
     if (ptr) (void)hipFree(ptr);
   if (m->hdr_h) (void)hipHostFree(m->hdr_h);
+  if (m->phase_h) (void)hipHostFree(m->phase_h);
   if (m->levels_h) (void)hipHostFree(m->levels_h);
   for (auto &set : m->ev)
     for (auto &e : set)
@@ -449,6 +450,9 @@ int create_model(int W, int H, const fs_params *p, const double *h_init, uint32_
   FS_TRY(fs::dev_alloc(&m->fill_flag, kFillBatch));
   if (hipHostMalloc(reinterpret_cast<void **>(&m->hdr_h),
                     (kHdrInts + FS_MAX_LEVELS + 3) * sizeof(int32_t)) != hipSuccess ||
+      hipHostMalloc(reinterpret_cast<void **>(&m->phase_h),
+                    static_cast<size_t>(kPhaseSlots) * kPhaseStride * sizeof(uint64_t)) !=
+          hipSuccess ||
       hipHostMalloc(reinterpret_cast<void **>(&m->levels_h),
                     (FS_MAX_LEVELS + 4) * sizeof(int32_t)) != hipSuccess) {
     fs::set_last_error("hipHostMalloc failed");
@@ -793,23 +797,57 @@ int launch_tile_step(fs_model *m, int halo, const double *h_in, double *h_out, i
   return kt_end(m);
 }
 
-// The outcome of the tile steps launched so far: waits for them, reads the
-// header and adds the batch's time (bracketed by tev[0] and tev[4]).
+// The outcome of the tile steps launched so far: waits for them and reads the
+// header and, of a sampled batch, the phase ticks.
 int finish_batch(fs_model *m, bool sampled) {
   FS_TRY(mark(m->tev[4], m->stream));
+  if (sampled)
+    FS_HIP_TRY(hipMemcpyAsync(m->phase_h, m->phase,
+                              static_cast<size_t>(kPhaseSlots) * kPhaseStride * sizeof(uint64_t),
+                              hipMemcpyDeviceToHost, m->stream));
   FS_TRY(fetch_header(m, 0));
   m->hdr_fresh = true;
-  if (m->tev[0]) {
-    float ms = 0.f;
-    FS_HIP_TRY(hipEventElapsedTime(&ms, m->tev[0], m->tev[4]));
-    m->tile_ms += ms;
-    for (int i = 0; i < 3 && sampled; i++) {
-      FS_HIP_TRY(hipEventElapsedTime(&ms, m->tev[i], m->tev[i + 1]));
-      m->samp_ms[i] += ms;
-    }
-  }
   FS_TRY(graph_collect(m));
   return kt_collect(m);
+}
+
+// The time of a finished batch (between tev[0] and tev[4]) for the stage timers.
+// sampled: its first step's kernels end at tev[1], tev[2] and tev[3]; taken: that
+// step was taken, and is the sample from now on.  One that was not has no
+// erosion: its events say what its kernels took, and the next step is sampled.
+// recv_ms: without receivers of its own (the same step with the deeper halo), what
+// those took.  Every batch is sampled until one has given shares.
+int account_batch(fs_model *m, bool sampled, bool taken, double *recv_ms, bool again) {
+  if (!m->tev[0]) return FS_OK;
+  float t = 0.f;
+  FS_HIP_TRY(hipEventElapsedTime(&t, m->tev[0], m->tev[4]));
+  const double all = t;
+  if (!sampled) {
+    add_tile_time(m, all, m->shares, !again, taken);
+    return FS_OK;
+  }
+  double ms[3] = {}, ticks[kPhaseStride];
+  for (int i = 0; i < 3; i++) {
+    FS_HIP_TRY(hipEventElapsedTime(&t, m->tev[i], m->tev[i + 1]));
+    ms[i] = t;
+  }
+  if (!again) *recv_ms = ms[0];
+  for (int k = 0; k < kPhaseStride; k++) {
+    uint64_t sum = 0;
+    for (int r = 0; r < kPhaseSlots; r++) sum += m->phase_h[r * kPhaseStride + k];
+    ticks[k] = static_cast<double>(sum - m->phase_seen[k]);
+    m->phase_seen[k] = sum;
+  }
+  if (taken) {
+    const double step[3] = {*recv_ms, again ? ms[0] + ms[1] : ms[1], ms[2]};
+    m->shares = tile_shares(step, ticks);
+    m->since_sample = 0;
+    add_tile_time(m, all, m->shares, !again, true);
+  } else {
+    const double step[3] = {again ? 0 : ms[0], all - (again ? 0 : ms[0]), 0};
+    add_tile_time(m, all, tile_shares(step, ticks), !again, false);
+  }
+  return FS_OK;
 }
 
 void take_tile_steps(fs_model *m, int n, int halo) {
@@ -845,8 +883,8 @@ int tile_steps(fs_model *m, long long want, int *done, bool *stuck) {
   const int n = m->ktiming || m->fill_mode
                     ? 1
                     : static_cast<int>(std::min<long long>(want, std::min(m->batch, kMaxBatch)));
-  // the first step of each call and then one in kPhaseEvery is the timers' sample
-  const bool sample = m->phase && (m->steps_in_call == 0 || m->since_sample >= kPhaseEvery);
+  // one step in kPhaseEvery is the timers' sample
+  const bool sample = m->phase && m->since_sample >= kPhaseEvery;
   const hipEvent_t none = nullptr;
   FS_TRY(mark(m->tev[0], m->stream));
   double *h_in = m->h, *h_out = m->h_alt;
@@ -868,8 +906,10 @@ int tile_steps(fs_model *m, long long want, int *done, bool *stuck) {
     taken++;
   take_tile_steps(m, taken, halo);   // a failed solve's step was taken, none behind it
   *done = taken;
+  double recv_ms = 0;
+  FS_TRY(account_batch(m, sample, taken > 0, &recv_ms, false));
+  m->since_sample += taken;
   FS_TRY(device_error_status(m->hdr_h[2]));
-  m->since_sample = sample ? n : m->since_sample + n;
   m->batch = taken == n ? std::min(2 * m->batch, kMaxBatch) : 4;
   if (taken == n || slots[taken * kSlotInts + kSlotStop] != 0) {
     // a 32-halo step whose levels all fit 16 tries the 16-cell halo next
@@ -882,16 +922,23 @@ int tile_steps(fs_model *m, long long want, int *done, bool *stuck) {
   if (halo == kHalo) {
     // the same step again with the 32-cell halo
     int32_t *slot = m->hdr + kHdrSlots;
+    const bool timed = sample && taken == 0;   // the sample is still to be had
     FS_TRY(mark(m->tev[0], m->stream));
     hipLaunchKernelGGL(k_slot_reset, dim3(1), dim3(64), 0, m->stream, slot);
     FS_TRY(check_launch());
-    FS_TRY(launch_tile_step(m, tile32::kHalo, m->h, m->h_alt, slot, false, none));
-    FS_TRY(finish_batch(m, false));
-    if (slots[kSlotOver] == 0) {
+    if (timed) FS_TRY(mark(m->tev[1], m->stream));
+    FS_TRY(launch_tile_step(m, tile32::kHalo, m->h, m->h_alt, slot, timed,
+                            timed ? m->tev[2] : none));
+    if (timed) FS_TRY(mark(m->tev[3], m->stream));
+    FS_TRY(finish_batch(m, timed));
+    const bool fits = slots[kSlotOver] == 0;
+    if (fits) {
       take_tile_steps(m, 1, tile32::kHalo);
       m->tile_halo = slots[kSlotDeepest] <= kHalo ? kHalo : tile32::kHalo;
       *done = taken + 1;
     }
+    FS_TRY(account_batch(m, timed, fits, &recv_ms, true));
+    if (fits) m->since_sample++;
     FS_TRY(device_error_status(m->hdr_h[2]));
     if (*done > taken) return FS_OK;
   }
@@ -1159,12 +1206,12 @@ int run_steps(fs_model *m, long long iterations) {
   int st = FS_OK;
   for (long long i = 0; i < iterations && st == FS_OK;) {
     int took = 0;
-    m->steps_in_call = i;
     st = advance(m, iterations - i, &took);
     i += took;
   }
   const int fst = finish(m);
   if (st == FS_OK) st = fst;
+  fold_timers(m);
   if (st != FS_OK) m->err_left = true;
   m->timer_us[FS_T_OVERALL] += static_cast<uint64_t>(
       std::chrono::duration_cast<std::chrono::microseconds>(std::chrono::steady_clock::now() - t0)
@@ -1265,14 +1312,13 @@ int fs_set_h(fs_model *m, const double *in, size_t count) {
 
 int fs_get_timers(fs_model *m, uint64_t us[FS_NUM_TIMERS]) {
   if (!m || !us) return FS_ERR_INVALID_ARGUMENT;
-  FS_TRY(fold_timers(m));
   for (int i = 0; i < FS_NUM_TIMERS; i++) us[i] = m->timer_us[i];
   return FS_OK;
 }
 
 int fs_reset_timers(fs_model *m) {
   if (!m) return FS_ERR_INVALID_ARGUMENT;
-  FS_TRY(fold_timers(m));
+  m->since_sample = kPhaseEvery;   // what is timed from here on has a sample of its own
   for (int i = 0; i < FS_NUM_TIMERS; i++) {
     m->timer_us[i] = 0;
     m->stage_ms[i] = 0;

@@ -1,0 +1,81 @@
+"""The stage timers' proportions against the kernels' own times, on models of their
+own (timing every kernel by itself changes how steps are launched).  Receivers are
+a kernel of their own; the tile erosion's time goes to GenerateOrder, Uplift and
+Erosion, GenerateOrder also gets a part of the accumulation's.  A sample of steps
+stands for the others: tolerance 4 points of the whole, of which the events
+around the sampled kernels take up to 2 at the smaller sizes (some 3 us of 150)."""
+import numpy as np
+import pytest
+
+import fastscape_amd as fa
+from conftest import cone_terrain
+from test_gpu_parity import note
+
+pytestmark = pytest.mark.gpu
+
+STAGES = fa.TIMER_NAMES[1:7]
+
+
+def kernel_shares(m, steps):
+    """Shares of the receivers and of the erosion kernels in `steps` steps."""
+    m.set_kernel_timing(True)
+    before = {k: v[0] for k, v in m.kernel_stats().items()}
+    m.step(steps)
+    ms = {k: v[0] - before[k] for k, v in m.kernel_stats().items()}
+    total = sum(ms.values())
+    return ms["k_receivers"] / total, ms["k_tile_erode"] / total
+
+
+def stage_shares(t):
+    total = sum(t[k] for k in STAGES)
+    return {k.split(": ")[1]: t[k] / total for k in STAGES}
+
+
+def check(stages, receivers, erode):
+    assert abs(stages["DetermineReceivers"] - receivers) <= 0.04, (stages, receivers)
+    order_on = stages["GenerateOrder"] + stages["Uplift"] + stages["Erosion"]
+    assert order_on >= erode - 0.04, (stages, erode)
+    assert stages["DetermineDonors"] + stages["FlowAcc"] <= 1 - receivers - erode + 0.04
+
+
+@pytest.mark.parametrize("side", [2048, 4096])
+def test_tile_steps(side):
+    note("timers %d^2" % side)
+    with fa.FastScape(side, side, fa.preset(fa.PRESET_BENCHMARK)) as m:
+        m.step(6)
+        receivers, erode = kernel_shares(m, 30)
+    with fa.FastScape(side, side, fa.preset(fa.PRESET_BENCHMARK)) as m:
+        m.step(6)
+        m.reset_timers()
+        m.step(60)
+        check(stage_shares(m.timers()), receivers, erode)
+
+
+def test_sampled_step_too_deep_for_the_first_halo():
+    """25 levels: the first step, sampled, does not erode with the 16-cell halo and
+    is taken with the 32-cell one."""
+    W, H = 2000, 1600
+    note("timers, 25 levels from the first step")
+    h = cone_terrain(W, H, 48, 0)
+    with fa.FastScape(W, H, fa.preset(fa.PRESET_BENCHMARK), h=h) as m:
+        receivers, erode = kernel_shares(m, 1)
+    with fa.FastScape(W, H, fa.preset(fa.PRESET_BENCHMARK), h=h) as m:
+        m.step(1)
+        assert m.tile_stats()["halo32"] == 1
+        check(stage_shares(m.timers()), receivers, erode)
+
+
+def test_every_call_is_accounted_for():
+    """Calls of one step, the timers read and reset behind each: every call's stages
+    share its time, whichever step was the sample."""
+    note("timers of single steps")
+    with fa.FastScape(1500, 1100, fa.preset(fa.PRESET_BENCHMARK)) as m:
+        m.step(1)
+        for i in range(40):
+            before = m.timers()
+            m.step(1)
+            t = m.timers()
+            part = np.array([t[k] - before[k] for k in STAGES], float)
+            assert part.sum() >= 20, (i, part)      # three kernels of 10 us and more
+            assert (part[[0, 1, 2, 3, 5]] > 0).all(), (i, part)
+            assert part.sum() <= t["Overall"] - before["Overall"], (i, part)
