@@ -142,13 +142,18 @@ struct fs_model {
   int ev_cur = 0;                     // level-path steps alternate the two sets
   // Tile and tile-graph steps are not bracketed by events one by one: a batch
   // is, and split by the shares of the last sampled step that was taken; a run
-  // of tile-graph steps by its first one's.
+  // of tile-graph steps by its first one's.  A step whose receivers a tile attempt
+  // has left in rcv launches none: it is a run of its own.
   hipEvent_t tev[5] = {};             // batch: start, the sampled step's kernels, end
   TileShares shares{};                // of the last sample
   uint64_t phase_seen[kPhaseStride] = {};   // the phase ticks' sums when last read
   long long since_sample = kPhaseEvery;     // tile steps since the last sample
-  hipEvent_t gev[8] = {};             // tile-graph run: its first step's stages, end
-  bool graph_open = false, graph_pending = false;
+  struct GraphRun {
+    hipEvent_t ev[8] = {};            // its first step's stages, its end
+    bool pending = false;             // ended, its time not yet collected
+  } grun[2];
+  int graph_open = -1;                // the run that goes on
+  bool graph_alone = false;           // it ends with its first step
   int batch = 4;                      // tile steps launched before the host looks
   bool hdr_fresh = false;             // hdr_h holds the header, nothing launched since
   bool err_left = false;              // the header may hold an earlier call's error bits
@@ -248,28 +253,51 @@ int stage_collect(fs_model *m, int set) {
 // Ends a run of tile-graph steps for the stage timers (its time is collected
 // once the stream has passed this point).
 int graph_close(fs_model *m) {
-  if (!m->graph_open) return FS_OK;
-  m->graph_open = false;
-  FS_HIP_TRY(hipEventRecord(m->gev[7], m->stream));
-  m->graph_pending = true;
+  if (m->graph_open < 0) return FS_OK;
+  fs_model::GraphRun &run = m->grun[m->graph_open];
+  m->graph_open = -1;
+  FS_HIP_TRY(hipEventRecord(run.ev[7], m->stream));
+  run.pending = true;
   return FS_OK;
 }
 
-// The time of a finished run of tile-graph steps, split over the stages in
-// proportion to its first step's.
+// The time of finished runs of tile-graph steps, split over the stages in
+// proportion to each one's first step.
 int graph_collect(fs_model *m) {
-  if (!m->graph_pending) return FS_OK;
-  FS_HIP_TRY(hipEventSynchronize(m->gev[7]));
-  m->graph_pending = false;
-  float ms[6] = {}, all = 0.f;
-  double sum = 0;
-  for (int i = 0; i < 6; i++) {
-    FS_HIP_TRY(hipEventElapsedTime(&ms[i], m->gev[i], m->gev[i + 1]));
-    sum += ms[i];
+  for (fs_model::GraphRun &run : m->grun) {
+    if (!run.pending) continue;
+    FS_HIP_TRY(hipEventSynchronize(run.ev[7]));
+    run.pending = false;
+    float ms[6] = {}, all = 0.f;
+    double sum = 0;
+    for (int i = 0; i < 6; i++) {
+      FS_HIP_TRY(hipEventElapsedTime(&ms[i], run.ev[i], run.ev[i + 1]));
+      sum += ms[i];
+    }
+    FS_HIP_TRY(hipEventElapsedTime(&all, run.ev[0], run.ev[7]));
+    for (int i = 0; i < 6 && sum > 0; i++)
+      m->stage_ms[FS_T_RECEIVERS + i] += static_cast<double>(all) * ms[i] / sum;
   }
-  FS_HIP_TRY(hipEventElapsedTime(&all, m->gev[0], m->gev[7]));
-  for (int i = 0; i < 6 && sum > 0; i++)
-    m->stage_ms[FS_T_RECEIVERS + i] += static_cast<double>(all) * ms[i] / sum;
+  return FS_OK;
+}
+
+// The events of a tile-graph step that begins a run, or null handles.  alone: its
+// receivers are there already.
+int graph_begin(fs_model *m, bool alone, const hipEvent_t **ev) {
+  static const hipEvent_t none[8] = {};
+  *ev = none;
+  const int last = m->graph_open;
+  if (last >= 0 && !m->graph_alone && !alone) return FS_OK;
+  FS_TRY(graph_close(m));
+  // a run at most waits to be collected here, behind one step alone: a tile
+  // attempt or the end of the call has collected those before
+  const int next = last == 0 ? 1 : 0;
+  if (m->grun[next].pending) FS_TRY(graph_collect(m));
+  for (auto &e : m->grun[next].ev)
+    if (!e) FS_HIP_TRY(hipEventCreate(&e));
+  m->graph_open = next;
+  m->graph_alone = alone;
+  *ev = m->grun[next].ev;
   return FS_OK;
 }
 
@@ -385,8 +413,9 @@ void free_model(fs_model *m) {
   for (auto e : m->kfree) (void)hipEventDestroy(e);
   for (auto e : m->tev)
     if (e) (void)hipEventDestroy(e);
-  for (auto e : m->gev)
-    if (e) (void)hipEventDestroy(e);
+  for (auto &run : m->grun)
+    for (auto e : run.ev)
+      if (e) (void)hipEventDestroy(e);
   if (m->stream) (void)hipStreamDestroy(m->stream);
   delete m;
 }
@@ -1138,16 +1167,8 @@ int advance(fs_model *m, long long want, int *took) {
   }
   m->hdr_fresh = false;
   if (m->path == FS_PATH_TILE_GRAPH || (m->path == FS_PATH_AUTO && m->owns_memory)) {
-    // the first of a run of tile-graph steps is the timers' sample
-    static const hipEvent_t none[8] = {};
-    const hipEvent_t *ev = none;
-    if (!m->graph_open) {
-      FS_TRY(graph_collect(m));
-      for (auto &e : m->gev)
-        if (!e) FS_HIP_TRY(hipEventCreate(&e));
-      m->graph_open = true;
-      ev = m->gev;
-    }
+    const hipEvent_t *ev;
+    FS_TRY(graph_begin(m, stuck, &ev));
     FS_TRY(mark(ev[0], m->stream));
     if (!stuck) FS_TRY(launch_receivers(m, m->h));
     FS_TRY(mark(ev[1], m->stream));

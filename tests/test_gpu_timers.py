@@ -79,3 +79,19 @@ def test_every_call_is_accounted_for():
             assert part.sum() >= 20, (i, part)      # three kernels of 10 us and more
             assert (part[[0, 1, 2, 3, 5]] > 0).all(), (i, part)
             assert part.sum() <= t["Overall"] - before["Overall"], (i, part)
+
+
+def test_graph_steps_behind_a_tile_attempt():
+    """49 levels: the first step's receivers come from the tile attempts, the later
+    ones' are the tile-graph steps' own."""
+    W, H, steps = 2000, 1600, 40
+    note("timers, 49 levels from the first step")
+    h = cone_terrain(W, H, 96, 0)
+    with fa.FastScape(W, H, fa.preset(fa.PRESET_BENCHMARK), h=h) as m:
+        receivers, _ = kernel_shares(m, steps)
+    with fa.FastScape(W, H, fa.preset(fa.PRESET_BENCHMARK), h=h) as m:
+        m.step(steps)
+        assert m.graph_stats()["steps"] == steps
+        share = stage_shares(m.timers())["DetermineReceivers"]
+        note("receivers %.4f of the stages, %.4f of the kernels" % (share, receivers))
+        assert 0.8 * receivers <= share <= 1.25 * receivers
