@@ -1159,7 +1159,10 @@ int fill_depressions(fs_model *m) {
 int advance(fs_model *m, long long want, int *took) {
   *took = 0;
   bool stuck = false;   // the step's receivers are in rcv
-  if (m->fill_mode) FS_TRY(fill_depressions(m));
+  if (m->fill_mode) {
+    FS_TRY(graph_close(m));   // the fill is no stage's time
+    FS_TRY(fill_depressions(m));
+  }
   if (m->path == FS_PATH_AUTO && m->tile_halo != 0) {
     FS_TRY(graph_close(m));
     FS_TRY(tile_steps(m, want, took, &stuck));

@@ -95,3 +95,23 @@ def test_graph_steps_behind_a_tile_attempt():
         share = stage_shares(m.timers())["DetermineReceivers"]
         note("receivers %.4f of the stages, %.4f of the kernels" % (share, receivers))
         assert 0.8 * receivers <= share <= 1.25 * receivers
+
+
+@pytest.mark.parametrize("path", [fa.PATH_AUTO, fa.PATH_TILE_GRAPH])
+def test_depression_filling_is_no_stage(path):
+    """Filling takes some ten times as long as a step here; the stages are the
+    steps' kernels, the gaps between them and no more."""
+    note("timers with depression filling, path %d" % path)
+    out = []
+    for timing in (True, False):
+        with fa.FastScape(700, 501, fa.preset(fa.PRESET_REFERENCE)) as m:
+            m.set_path(path)
+            m.set_depression_fill(True)
+            m.set_kernel_timing(timing)
+            m.step(8)
+            t = m.timers()
+            out.append((sum(v[0] for v in m.kernel_stats().values()) * 1e3,
+                        sum(t[k] for k in STAGES), t["Overall"] - t["Step1: Initialize"]))
+    kernels, stages, overall = out[0][0], out[1][1], out[1][2]
+    note("kernels %.0f us, stages %.0f, overall %.0f" % (kernels, stages, overall))
+    assert 0.5 * kernels <= stages <= 2 * kernels
