@@ -30,9 +30,8 @@
 // step in 64.
 //
 // A cell's elevation depends only on its own inputs and its receiver's final
-// value, and upstream counts are integers, so the order of the work is free.
-// (fs_schedule's work item sizes were the persistent kernel's; they are
-// accepted and have no effect.)
+// value, and upstream counts are integers, so the order of the work is free: the
+// schedule (fs_schedule) says how much of it a workgroup takes.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -57,6 +56,7 @@ namespace {
 constexpr int kEnsBlock = 1024;                     // k_ens_lists
 constexpr int kHistLen = kHalo + 1;
 constexpr int kRecvRows = 16;                       // schedules name multiples of this
+constexpr int kRecvPerBlock = 64;                   // rows named per receiver block
 constexpr int kMaxRealizations = 1 << 20;
 
 // per-realization state words (kRH ints each)
@@ -132,12 +132,10 @@ __device__ __forceinline__ int ens_block() {
   return static_cast<int>(blockIdx.y * gridDim.x + blockIdx.x);
 }
 
-// recv_real: each workgroup's realization (nblocks of them).
-__global__ __launch_bounds__(256) void k_ens_receivers(EnsArgs a,
-                                                       const int32_t *__restrict__ recv_real,
-                                                       int nblocks) {
-  const int b = ens_block();
-  if (b >= nblocks) return;
+// Receivers of block b: 64 columns x kRecvShort * kRecvGroups rows of
+// realization recv_real[b].
+__device__ __forceinline__ void ens_recv_block(const EnsArgs &a,
+                                               const int32_t *__restrict__ recv_real, int b) {
   const int r = recv_real[b];
   const EnsReal &g = a.real[r];
   const int local = b - g.recv_first;
@@ -152,6 +150,23 @@ __global__ __launch_bounds__(256) void k_ens_receivers(EnsArgs a,
   ShortRows v;
   load_short(v, a.h_old + g.off, g.W, g.H, x, group);
   decide_short(v, a.rcv + g.off, g.W, g.H, x, group, g.d_card, g.d_diag);
+}
+
+// A workgroup takes per_group of the nblocks blocks (kMany), or one: the loop
+// over them costs registers (92 instead of 76).
+template <bool kMany>
+__global__ __launch_bounds__(256) void k_ens_receivers(EnsArgs a,
+                                                       const int32_t *__restrict__ recv_real,
+                                                       int nblocks, int per_group) {
+  if constexpr (kMany) {
+    const long long first = static_cast<long long>(ens_block()) * per_group;
+    const int end = static_cast<int>(min(static_cast<long long>(nblocks), first + per_group));
+    for (int b = static_cast<int>(min(first, static_cast<long long>(end))); b < end; b++)
+      ens_recv_block(a, recv_real, b);
+  } else {
+    const int b = ens_block();
+    if (b < nblocks) ens_recv_block(a, recv_real, b);
+  }
 }
 
 // tile_real: each tile's realization (tiles numbered across realizations).
@@ -210,16 +225,8 @@ __global__ __launch_bounds__(kEnsBlock) void k_ens_lists(EnsArgs a, int32_t *tab
 }
 
 template <int NM>
-__global__ __launch_bounds__(kEroBlock) void k_ens_erode(EnsArgs a,
-                                                         const int32_t *__restrict__ tile_real,
-                                                         int ntiles) {
-  __shared__ EroShared sh;
-  const int b = ens_block();
-  if (b >= ntiles) return;
-  const int tile = xcd_tile(b, ntiles);
-  const int r = tile_real[tile];
-  int32_t *const q = a.rh + static_cast<size_t>(r) * kRH;
-  if (q[kRhPath] != 1) return;
+__device__ __forceinline__ void ens_erode_tile(EroShared &sh, const EnsArgs &a, int r,
+                                               int32_t *q, int tile) {
   const EnsReal &g = a.real[r];
   const ErodeConst ek = g.ek;
   with_nmode<NM>(g.nmode, [&](auto c) {
@@ -229,6 +236,34 @@ __global__ __launch_bounds__(kEroBlock) void k_ens_erode(EnsArgs a,
   });
 }
 
+// A workgroup takes per_group of the ntiles tiles, one after another (kMany), or
+// one: the loop over them would take 94 registers where two workgroups per CU
+// have 64 (held to these it spills 60 bytes a lane).
+template <int NM, bool kMany>
+__global__ __launch_bounds__(kEroBlock, kMany ? 8 : 1) void k_ens_erode(
+    EnsArgs a, const int32_t *__restrict__ tile_real, int ntiles, int per_group) {
+  __shared__ EroShared sh;
+  const int b = ens_block();
+  if constexpr (kMany) {
+    const int groups = (ntiles - 1) / per_group + 1;
+    if (b >= groups) return;
+    const int first = xcd_tile(b, groups) * per_group, n = min(ntiles - first, per_group);
+    for (int j = 0; j < n; j++) {
+      const int r = tile_real[first + j];
+      int32_t *const q = a.rh + static_cast<size_t>(r) * kRH;
+      if (q[kRhPath] != 1) continue;
+      __syncthreads();   // the LDS of the tile before is free
+      ens_erode_tile<NM>(sh, a, r, q, first + j);
+    }
+  } else {
+    if (b >= ntiles) return;
+    const int tile = xcd_tile(b, ntiles);
+    const int r = tile_real[tile];
+    int32_t *const q = a.rh + static_cast<size_t>(r) * kRH;
+    if (q[kRhPath] != 1) return;
+    ens_erode_tile<NM>(sh, a, r, q, tile);
+  }
+}
 
 }  // namespace
 
@@ -392,6 +427,18 @@ dim3 ens_grid(int n) {
   return dim3(x, (static_cast<unsigned>(n) + x - 1) / x);
 }
 
+template <int NM>
+void launch_ens_erode(fs_ensemble *e, const EnsArgs &a) {
+  const int per = e->sched.tiles_per_claim;
+  const dim3 grid = ens_grid((e->tiles - 1) / per + 1);
+  if (per > 1)
+    hipLaunchKernelGGL((k_ens_erode<NM, true>), grid, dim3(kEroBlock), 0, e->stream, a,
+                       e->tile_real, e->tiles, per);
+  else
+    hipLaunchKernelGGL((k_ens_erode<NM, false>), grid, dim3(kEroBlock), 0, e->stream, a,
+                       e->tile_real, e->tiles, per);
+}
+
 int tile_launches(fs_ensemble *e) {
   hipStream_t s = e->stream;
   EnsArgs a{};
@@ -406,8 +453,14 @@ int tile_launches(fs_ensemble *e) {
   a.ftab = e->ftab;
   a.rh = e->rh;
   a.hist = e->hist;
-  hipLaunchKernelGGL(k_ens_receivers, ens_grid(e->recv_blocks), dim3(256), 0, s, a,
-                     e->recv_real, e->recv_blocks);
+  const int recv = std::max(1, e->sched.recv_rows / kRecvPerBlock);
+  const dim3 recv_grid = ens_grid((e->recv_blocks - 1) / recv + 1);
+  if (recv > 1)
+    hipLaunchKernelGGL(k_ens_receivers<true>, recv_grid, dim3(256), 0, s, a, e->recv_real,
+                       e->recv_blocks, recv);
+  else
+    hipLaunchKernelGGL(k_ens_receivers<false>, recv_grid, dim3(256), 0, s, a, e->recv_real,
+                       e->recv_blocks, recv);
   // as for one grid: 1024-thread workgroups where there are fewer tiles than
   // four per CU
   if (e->tiles < 4 * e->ncu)
@@ -419,15 +472,9 @@ int tile_launches(fs_ensemble *e) {
   hipLaunchKernelGGL(k_ens_lists, dim3(1), dim3(kEnsBlock), 0, s, a, e->tabG_off, e->tabG_real,
                      e->tabG_size, e->graph_n_h);
   FS_HIP_TRY(hipEventRecord(e->listed, s));
-  if (e->nm_all == 1)
-    hipLaunchKernelGGL(k_ens_erode<1>, ens_grid(e->tiles), dim3(kEroBlock), 0, s, a, e->tile_real,
-                       e->tiles);
-  else if (e->nm_all == 2)
-    hipLaunchKernelGGL(k_ens_erode<2>, ens_grid(e->tiles), dim3(kEroBlock), 0, s, a, e->tile_real,
-                       e->tiles);
-  else
-    hipLaunchKernelGGL(k_ens_erode<-1>, ens_grid(e->tiles), dim3(kEroBlock), 0, s, a, e->tile_real,
-                       e->tiles);
+  if (e->nm_all == 1) launch_ens_erode<1>(e, a);
+  else if (e->nm_all == 2) launch_ens_erode<2>(e, a);
+  else launch_ens_erode<-1>(e, a);
   FS_HIP_TRY(hipGetLastError());
   return FS_OK;
 }
@@ -491,37 +538,33 @@ int timed_steps(fs_ensemble *e, const fs_schedule &s, int steps, double *ms_per_
 }
 
 // Coordinate search over the schedule knobs, each candidate timed on
-// tune_trial real steps; stops early when `budget` steps are used.
-// Returns the number of steps taken in *used.
+// tune_trial real steps; stops early when `budget` steps are used.  A candidate
+// has to be ahead by more than one step's time varies (3%); a knob is done with
+// its first value that is not, since more work per workgroup then only costs
+// more.  Returns the number of steps taken in *used.
 int autotune(fs_ensemble *e, int budget, int *used) {
   *used = 0;
-  const std::vector<int> rows_vals = {16, 64, 256};
-  const std::vector<int> tpc_vals = {1, 2, 4};
   fs_schedule best = e->sched;
   double best_ms = -1;
-  for (int knob = 1; knob < 3; knob++) {
-    const std::vector<int> &vals = knob == 1 ? rows_vals : tpc_vals;
-    for (int v : vals) {
-      if (*used + e->tune_trial > budget) {
-        e->sched = best;
-        return FS_OK;
-      }
+  auto search = [&](int fs_schedule::*knob, std::initializer_list<int> values) {
+    for (int v : values) {
       fs_schedule c = best;
-      (knob == 0 ? c.group_cells : knob == 1 ? c.recv_rows : c.tiles_per_claim) = v;
-      if (best_ms >= 0 && c.group_cells == best.group_cells && c.recv_rows == best.recv_rows &&
-          c.tiles_per_claim == best.tiles_per_claim)
-        continue;
+      c.*knob = v;
+      if (best_ms >= 0 && c.*knob == best.*knob) continue;   // timed already
+      if (*used + e->tune_trial > budget) return FS_OK;
       double ms = 0;
       FS_TRY(timed_steps(e, c, e->tune_trial, &ms));
       *used += e->tune_trial;
       e->tune_cand.push_back(c);
       e->tune_ms.push_back(ms);
-      if (best_ms < 0 || ms < best_ms) {
-        best_ms = ms;
-        best = c;
-      }
+      if (best_ms >= 0 && !(ms < 0.97 * best_ms)) return FS_OK;
+      best_ms = ms;
+      best = c;
     }
-  }
+    return FS_OK;
+  };
+  FS_TRY(search(&fs_schedule::recv_rows, {kRecvPerBlock, 2 * kRecvPerBlock, 4 * kRecvPerBlock}));
+  FS_TRY(search(&fs_schedule::tiles_per_claim, {1, 2, 4}));
   e->sched = best;
   return FS_OK;
 }

@@ -282,11 +282,12 @@ typedef struct fs_realization {
   uint32_t engine_seed;
 } fs_realization;
 
-/* Work schedule of a step.  The fields are checked and kept and have no
- * effect: the work is laid out by the realizations' sizes.
- *   recv_rows        16..256, a multiple of 16
- *   tiles_per_claim  1..16
- *   group_cells      >= 0 */
+/* Work schedule of a step; every schedule gives the same results.
+ *   recv_rows        16..256, a multiple of 16: a receiver workgroup takes one
+ *                    block of 64 columns x 24 rows for every 64 of it (at least one)
+ *   tiles_per_claim  1..16: 64x64 tiles per erosion workgroup
+ *   group_cells      accepted (>= 0) and without effect: deep realizations take
+ *                    the tile-graph step, whose work spreads over every CU */
 typedef struct fs_schedule {
   int recv_rows;
   int tiles_per_claim;

@@ -6,26 +6,28 @@ import os
 import re
 import subprocess
 
+import pytest
+
 from conftest import ROOT
 
 CSRC = os.path.join(ROOT, "barnes2019-landscape_amd", "csrc")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 
-def test_two_erosion_workgroups_per_cu(tmp_path):
+# k_tile_erode<n, timed> with both halos; k_ens_erode<n, many>
+@pytest.mark.parametrize("source,kernel,count", [
+    ("fastscape_hip.hip", "k_tile_erode", 8), ("fs_ensemble.hip", "k_ens_erode", 4)])
+def test_two_erosion_workgroups_per_cu(tmp_path, source, kernel, count):
     r = subprocess.run(
         [HIPCC, "-O3", "-std=c++17", "-ffp-contract=off", "-w", "--offload-arch=gfx950", "-Xclang",
          "-target-feature", "-Xclang", "-packed-fp32-ops", "-I" + os.path.join(ROOT, "include"),
-         "-I" + CSRC, "--cuda-device-only", "-S", os.path.join(CSRC, "fastscape_hip.hip"), "-o",
+         "-I" + CSRC, "--cuda-device-only", "-S", os.path.join(CSRC, source), "-o",
          str(tmp_path / "out.s"), "-Rpass-analysis=kernel-resource-usage"],
         check=True, capture_output=True, text=True)
     used = {}
     for part in r.stderr.split("Function Name: ")[1:]:
-        # k_tile_erode<n, timed>, both halos
-        name = re.match(r"\S*k_tile_erodeILi([12])ELb([01])E", part)
-        if name:
-            tile32 = "tile32" in part.split()[0]
-            used[tile32, name.group(1), name.group(2)] = tuple(
-                int(re.search(k + r": (\d+)", part).group(1)) for k in (r"\bVGPRs", "TotalSGPRs"))
-    assert len(used) == 8, used
+        if re.match(r"\S*" + kernel + r"ILi[12]ELb[01]E", part):
+            used[part.split()[0]] = tuple(int(re.search(k + r": (\d+)", part).group(1))
+                                          for k in (r"\bVGPRs", "TotalSGPRs"))
+    assert len(used) == count, used
     assert all(v <= 64 and s <= 80 for v, s in used.values()), used
