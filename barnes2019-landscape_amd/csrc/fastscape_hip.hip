@@ -1111,7 +1111,8 @@ int graph_status(fs_model *m) {
     return FS_ERR_LEVEL_OVERFLOW;
   }
   if (err) {
-    fs::set_last_error("tile-graph path: receivers do not form a forest");
+    fs::set_last_error(err & deep::kErrCount ? "tile-graph path: work items were not all counted"
+                                             : "tile-graph path: receivers do not form a forest");
     return FS_ERR_INTERNAL;
   }
   return FS_OK;

@@ -81,18 +81,20 @@ __device__ __forceinline__ int shard_of(int t) {
   return static_cast<int>((static_cast<uint32_t>(t) * 2654435761u) >> 26);
 }
 static_assert(kShards == 1 << (32 - 26), "shard_of");
-// tstat words: error bits, deepest tier, items, groups of tiles whose tiers
-// are counted; the first item of each queue (and the end of the last); each
-// queue's cursor, and beside it a count of finished tiles, on a cache line of
-// its own (kQStride words apart).  All are zero before the first step;
-// k_deep_local clears the first kStClear words.
-constexpr int kStErr = 0, kStMaxTier = 1, kStItems = 2, kStDone = 3, kStClear = 4;
+// tstat words: error bits, deepest tier, items; the first item of each queue (and
+// the end of the last); each queue's cursor on a cache line of its own (kQStride
+// words apart), and on these lines, as 64-bit words, a group's finished tiles
+// and their items and (the first line) the finished groups and theirs.  All are
+// zero before the first step; k_deep_local clears the first kStClear words,
+// k_deep_nodes the 64-bit ones.
+constexpr int kStErr = 0, kStMaxTier = 1, kStItems = 2, kStClear = 3;
+constexpr int kStTick = 2, kStAll = 4;   // from a cursor's word
 constexpr int kStQStart = 4;
 constexpr int kQStride = 32;
 constexpr int kStQCur = 128;
 constexpr int kStWords = kStQCur + kShards * kQStride;
 static_assert(kStClear <= kStQStart && kStQStart + kShards + 1 <= kStQCur, "queue starts fit before the cursors");
-constexpr int32_t kErrTier = 1, kErrChain = 2;
+constexpr int32_t kErrTier = 1, kErrChain = 2, kErrCount = 4;
 // the "not yet eroded" mark: a signalling NaN that no arithmetic produces
 constexpr unsigned long long kUnsolved = 0x7FF4A5A5A5A5A5A5ull;
 constexpr int kSpinCap = 1 << 24;
@@ -558,48 +560,61 @@ __global__ __launch_bounds__(kNodeCap) void k_deep_links(
 // shards s with s % nq == q -- and each queue's tier by tier, so a queue
 // hands out its items in tier order.  Writes each queue's first item and
 // cursor, clears thist for the next step.  One workgroup of kNodeCap threads
-// in the kernel that counted: the counts of the other workgroups' atomics
-// are read past this XCD's cache; nq divides kShards.
-__device__ __forceinline__ void item_offsets(int32_t *__restrict__ thist,
-                                             int32_t *__restrict__ tcur,
-                                             int32_t *__restrict__ tstat, int nq, int *sh) {
-  constexpr int kWords = 4;   // consecutive words per thread
+// in the kernel that counts; nq divides kShards.  Nothing orders the other
+// workgroups' atomics before this one's reads: `items` is the number they have
+// added in all.  A count only grows, so counts that sum up to that number are
+// all final, the deepest tier with them; otherwise they are read again.
+__device__ __forceinline__ void item_offsets(int32_t *thist, int32_t *__restrict__ tcur,
+                                             int32_t *tstat, int nq, int items, int *sh) {
+  constexpr int kWords = 4;             // consecutive words per thread
+  constexpr int kCountTries = 1 << 16;  // each a few microseconds
   auto read = [](int32_t *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   };
-  const int spq = kShards / nq;                               // shards per queue
-  const int per_q = (read(&tstat[kStMaxTier]) + 1) * spq;     // (tier, shard) words per queue
-  const int n = nq * per_q;
-  int carry = 0;
-  for (int base = 0; base < n; base += kNodeCap * kWords) {
-    int idx[kWords], v[kWords], sum = 0;
+  const int spq = kShards / nq;   // shards per queue
+  int n = 0, carry = 0;
+  for (int tries = 0;; tries++) {
+    __syncthreads();
+    if (threadIdx.x == 0) sh[0] = read(&tstat[kStMaxTier]);
+    __syncthreads();
+    const int per_q = (sh[0] + 1) * spq;   // (tier, shard) words per queue
+    __syncthreads();
+    n = nq * per_q;
+    carry = 0;
+    for (int base = 0; base < n; base += kNodeCap * kWords) {
+      int idx[kWords], v[kWords], sum = 0;
 #pragma unroll
-    for (int j = 0; j < kWords; j++) {
-      const int k = base + threadIdx.x * kWords + j;
-      const int q = k / per_q, rem = k - q * per_q;
-      const int tier = rem / spq, s = q + (rem - tier * spq) * nq;
-      idx[j] = k < n ? tier * kShards + s : -1;
-      v[j] = idx[j] >= 0 ? read(&thist[idx[j]]) : 0;
-    }
-#pragma unroll
-    for (int j = 0; j < kWords; j++) sum += v[j];
-    int total;
-    int at = carry + block_scan<kNodeCap>(sum, sh, &total);
-#pragma unroll
-    for (int j = 0; j < kWords; j++) {
-      if (idx[j] < 0) continue;
-      const int k = base + threadIdx.x * kWords + j;
-      tcur[idx[j]] = at;
-      thist[idx[j]] = 0;
-      if (k % per_q == 0) {   // the queue's first word
-        tstat[kStQStart + k / per_q] = at;
-        tstat[kStQCur + (k / per_q) * kQStride] = at;
+      for (int j = 0; j < kWords; j++) {
+        const int k = base + threadIdx.x * kWords + j;
+        const int q = k / per_q, rem = k - q * per_q;
+        const int tier = rem / spq, s = q + (rem - tier * spq) * nq;
+        idx[j] = k < n ? tier * kShards + s : -1;
+        v[j] = idx[j] >= 0 ? read(&thist[idx[j]]) : 0;
       }
-      at += v[j];
+#pragma unroll
+      for (int j = 0; j < kWords; j++) sum += v[j];
+      int total;
+      int at = carry + block_scan<kNodeCap>(sum, sh, &total);
+#pragma unroll
+      for (int j = 0; j < kWords; j++) {
+        if (idx[j] < 0) continue;
+        const int k = base + threadIdx.x * kWords + j;
+        tcur[idx[j]] = at;
+        if (k % per_q == 0) {   // the queue's first word
+          tstat[kStQStart + k / per_q] = at;
+          tstat[kStQCur + (k / per_q) * kQStride] = at;
+        }
+        at += v[j];
+      }
+      carry += total;
     }
-    carry += total;
+    if (carry == items || tries >= kCountTries) break;   // the same for every thread
+    __builtin_amdgcn_s_sleep(8);
   }
+  for (int k = threadIdx.x; k < n; k += kNodeCap)   // the words of tiers 0 .. the deepest
+    __hip_atomic_store(&thist[k], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (threadIdx.x == 0) {
+    if (carry != items) atomicOr(&tstat[kStErr], kErrCount);
     tstat[kStItems] = carry;
     tstat[kStQStart + nq] = carry;
   }
@@ -612,16 +627,17 @@ __device__ __forceinline__ void item_offsets(int32_t *__restrict__ thist,
 // through every exit, leaf to root.  (As a launch each, the chains of memory
 // round trips one behind the other, all the node kernels took 23 us at 501 x
 // 501, 30 at 1000 x 1000 and 81 at 4097 x 3001 in deep drainage, 250 where 369
-// tiers lie in 250 x 250 cells; now 15, 21, 71 and 158.  Fences around the
-// ticks write every workgroup's L2 back: 299 us at 4097 x 3001.)
+// tiers lie in 250 x 250 cells; now 15, 21, 71 and 158.  Release and acquire
+// around the ticks would order the counts, but write every workgroup's L2 back:
+// 299 us at 4097 x 3001.)
 __global__ __launch_bounds__(kNodeCap) void k_deep_nodes(
     GraphWork w, const uint32_t *__restrict__ node_parent, const int32_t *__restrict__ nexit,
     uint16_t *__restrict__ node_tier, const uint32_t *__restrict__ node_up,
-    uint32_t *__restrict__ node_level, int32_t *__restrict__ thist, int32_t *__restrict__ tcur,
+    uint32_t *__restrict__ node_level, int32_t *thist, int32_t *__restrict__ tcur,
     int nq, uint64_t *__restrict__ node_word, const uint32_t *__restrict__ node_kids,
-    uint32_t *__restrict__ node_out, int32_t *__restrict__ tstat) {
+    uint32_t *__restrict__ node_out, int32_t *tstat) {
   __shared__ uint32_t seen[(kTierCap + 32) / 32];   // tiers already counted for the tile
-  __shared__ int scan[kNodeCap / kWave + 1], last;
+  __shared__ int scan[kNodeCap / kWave + 1], found, items;
   const int k = threadIdx.x, tiles = w.size[1];
   int wi = blockIdx.x;
   if (wi >= 2 * tiles) return;
@@ -644,6 +660,7 @@ __global__ __launch_bounds__(kNodeCap) void k_deep_nodes(
     }
     // clear the words the tile's tiers can touch (the block's own entries)
     if (k < n && tier <= kTierCap) seen[tier >> 5] = 0;
+    if (k == 0) found = 0;
     __syncthreads();
     if (k < n) {
       if (tier > kTierCap) {
@@ -652,30 +669,38 @@ __global__ __launch_bounds__(kNodeCap) void k_deep_nodes(
         const uint32_t bit = 1u << (tier & 31);
         if (!(atomicOr(&seen[tier >> 5], bit) & bit)) {   // the tile's first node of the tier
           atomicAdd(&thist[tier * kShards + shard_of(t)], 1);
+          atomicAdd(&found, 1);
           if (tier > __hip_atomic_load(&tstat[kStMaxTier], __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_AGENT))
             atomicMax(&tstat[kStMaxTier], tier);
         }
       }
     }
-    // the counts are atomics, performed past the caches: once a wave's have
-    // been acknowledged, its workgroup ticks, first among the tiles with the
-    // same low bits (tens of thousands of ticks stay off one address), the last of
+    // the workgroup ticks and adds its items, first among the tiles with the same
+    // low bits (tens of thousands of ticks stay off one address), the last of
     // these for all of them
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (k == 0) {
-      const int g = wi & (kShards - 1), groups = min(tiles, kShards);
-      int32_t *const tick = &tstat[kStQCur + g * kQStride + 1];
-      last = 0;
-      if (atomicAdd(tick, 1) == (tiles - g + kShards - 1) / kShards - 1) {
-        *tick = 0;   // for the next step
-        last = atomicAdd(&tstat[kStDone], 1) == groups - 1;
-      }
+      constexpr uint64_t kOne = uint64_t{1} << 32;   // ticks above, items below
+      auto word = [&](int at) { return reinterpret_cast<unsigned long long *>(&tstat[at]); };
+      auto add = [&](unsigned long long *p, uint64_t v, int of, uint64_t *sum) {
+        *sum = atomicAdd(p, static_cast<unsigned long long>(v)) + v;
+        if ((*sum >> 32) != static_cast<uint64_t>(of)) return false;
+        // the last one clears it for the next step
+        __hip_atomic_store(p, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return true;
+      };
+      const int g = wi & (kShards - 1);
+      uint64_t sum = 0;
+      items = -1;
+      if (add(word(kStQCur + g * kQStride + kStTick), kOne + static_cast<uint32_t>(found),
+              (tiles - g + kShards - 1) / kShards, &sum) &&
+          add(word(kStQCur + kStAll), kOne + static_cast<uint32_t>(sum), min(tiles, kShards), &sum))
+        items = static_cast<int>(static_cast<uint32_t>(sum));
     }
     __syncthreads();
-    if (!last) return;
-    item_offsets(thist, tcur, tstat, nq, scan);
+    if (items < 0) return;
+    item_offsets(thist, tcur, tstat, nq, items, scan);
     return;
   }
   wi -= tiles;

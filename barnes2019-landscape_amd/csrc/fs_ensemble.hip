@@ -501,6 +501,8 @@ int ensemble_errors(fs_ensemble *e) {
     e->broken = true;
     fs::set_last_error(ts[deep::kStErr] & deep::kErrTier
                            ? "tile-graph step: a drainage path crosses more tile borders than levels allow"
+                       : ts[deep::kStErr] & deep::kErrCount
+                           ? "tile-graph step: work items were not all counted"
                            : "tile-graph step: receivers do not form a forest");
     return ts[deep::kStErr] & deep::kErrTier ? FS_ERR_LEVEL_OVERFLOW : FS_ERR_INTERNAL;
   }
