@@ -685,11 +685,16 @@ inline ErodeConst make_erode_const(const fs_params &p, int *nmode) {
   return k;
 }
 
-// v_min_f64 as it is, without the instruction per operand that fmin spends on
-// quieting signalling NaNs
+// v_min_f64 and v_max_f64 as they are, without the instruction per operand that
+// fmin and fmax spend on quieting signalling NaNs
 __device__ __forceinline__ double raw_min(double a, double b) {
   double r;
   asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ double raw_max(double a, double b) {
+  double r;
+  asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
   return r;
 }
 // The implicit update of one cell (RB:313-326), operation for operation.
@@ -959,7 +964,7 @@ __global__ __launch_bounds__(kFillBlock) void k_fill(const double *__restrict__ 
     for (int i = 0; i < 2; i++) {
       const int gx = x0 + lx + i, gy = y0 + ly + j;
       inner[j][i] = gx >= 2 && gx < W - 2 && gy >= 2 && gy < H - 2;
-      hv[j][i] = inner[j][i] ? h[static_cast<size_t>(gy) * W + gx] : 0.0;
+      hv[j][i] = inner[j][i] ? __builtin_canonicalize(h[static_cast<size_t>(gy) * W + gx]) : 0.0;
     }
   // the halo cell this thread looks after: the ring around the tile
   constexpr int kRing = 4 * kFillReg - 4;
@@ -982,6 +987,18 @@ __global__ __launch_bounds__(kFillBlock) void k_fill(const double *__restrict__ 
   auto ld = [&](int i) {
     return __hip_atomic_load(&f_s[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   };
+  auto st = [&](int i, double v) {
+    __hip_atomic_store(&f_s[i], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  };
+  // news is published behind the values it stands for, and taken before they are
+  // read
+  auto publish = [&](uint32_t patches) {
+    __hip_atomic_fetch_or(&dirty, patches, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+  };
+  auto take = [&](uint32_t patch) {
+    return __hip_atomic_fetch_and(&dirty, ~patch, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) &
+           patch;
+  };
   const int c0 = (ly + 1) * kFillReg + lx + 1;
   // the patches around this wave's
   uint32_t around = 0;
@@ -992,13 +1009,17 @@ __global__ __launch_bounds__(kFillBlock) void k_fill(const double *__restrict__ 
       const int px = wave % 4 + i, py = wave / 4 + j;
       if ((i || j) && px >= 0 && px < 4 && py >= 0 && py < 4) around |= 1u << (4 * py + px);
     }
-  // one relaxation of the lane's cells; true when one of them fell
+  // the lane's cells, which it alone writes
+  double own[2][2];
+  // one relaxation of them; true when one fell
   auto relax = [&]() {
     double f[4][4];
 #pragma unroll
     for (int j = 0; j < 4; j++)
 #pragma unroll
-      for (int i = 0; i < 4; i++) f[j][i] = f_s[c0 + (j - 1) * kFillReg + i - 1];
+      for (int i = 0; i < 4; i++)
+        f[j][i] = j % 3 && i % 3 ? own[(j - 1) & 1][(i - 1) & 1]
+                                 : ld(c0 + (j - 1) * kFillReg + i - 1);
     bool fell = false;
 #pragma unroll
     for (int j = 1; j < 3; j++)
@@ -1007,14 +1028,13 @@ __global__ __launch_bounds__(kFillBlock) void k_fill(const double *__restrict__ 
         const double a = raw_min(raw_min(f[j - 1][i - 1], f[j - 1][i]), f[j - 1][i + 1]);
         const double b = raw_min(raw_min(f[j + 1][i - 1], f[j + 1][i]), f[j + 1][i + 1]);
         const double m = raw_min(raw_min(a, b), raw_min(f[j][i - 1], f[j][i + 1]));
-        const double v = fmax(hv[j - 1][i - 1], next_up(m));
+        const double v = raw_max(hv[j - 1][i - 1], next_up(m));
         if (inner[j - 1][i - 1] && v < f[j][i]) {
-          f[j][i] = v;
+          f[j][i] = own[j - 1][i - 1] = v;
           fell = true;
-          f_s[c0 + (j - 1) * kFillReg + i - 1] = v;
+          st(c0 + (j - 1) * kFillReg + i - 1, v);
         }
       }
-    asm volatile("" ::: "memory");   // the next relaxation reads LDS again
     return fell;
   };
   auto store_cells = [&]() {
@@ -1024,8 +1044,7 @@ __global__ __launch_bounds__(kFillBlock) void k_fill(const double *__restrict__ 
       for (int i = 0; i < 2; i++)
         if (inner[j][i])
           __hip_atomic_store(&F[static_cast<size_t>(y0 + ly + j) * W + x0 + lx + i],
-                             ld(c0 + j * kFillReg + i), __ATOMIC_RELAXED,
-                             __HIP_MEMORY_SCOPE_AGENT);
+                             own[j][i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   };
   // the neighbours' cell this thread looks after, read again; its news wakes
   // the patches it touches
@@ -1033,7 +1052,7 @@ __global__ __launch_bounds__(kFillBlock) void k_fill(const double *__restrict__ 
     if (halo < 0) return 0;
     const double v = load_f(x0 - 1 + hx, y0 - 1 + hy);
     if (!(v < ld(halo))) return 0;
-    __hip_atomic_store(&f_s[halo], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    st(halo, v);
     uint32_t wake = 0;
     for (int j = -1; j < 2; j++)
       for (int i = -1; i < 2; i++) {
@@ -1041,18 +1060,22 @@ __global__ __launch_bounds__(kFillBlock) void k_fill(const double *__restrict__ 
         if (cx >= 0 && cx < kFillTile && cy >= 0 && cy < kFillTile)
           wake |= 1u << (4 * (cy / 16) + cx / 16);
       }
-    atomicOr(&dirty, wake);
+    publish(wake);
     return 1;
   };
   bool ever = false;        // block-uniform: a cell fell in this launch
   __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 2; j++)
+#pragma unroll
+    for (int i = 0; i < 2; i++) own[j][i] = ld(c0 + j * kFillReg + i);
   for (int votes = 0; votes < kFillVotes;) {
     bool moved = false;     // block-uniform: since the last publication
     for (; votes < kFillVotes; votes++) {
       // a wave rests while neither it nor a patch around it has news
       int fell = 0;
       uint32_t mine = 0;
-      if (lane == 0) mine = atomicAnd(&dirty, ~(1u << wave)) >> wave & 1u;
+      if (lane == 0) mine = take(1u << wave);
       if (__builtin_amdgcn_readfirstlane(mine)) {
         bool now = true;
         for (int k = 0; k < kFillInner && __any(now); k++) {
@@ -1060,7 +1083,7 @@ __global__ __launch_bounds__(kFillBlock) void k_fill(const double *__restrict__ 
           fell |= now ? 1 : 0;
         }
         const uint32_t wake = (__any(fell) ? around : 0u) | (__any(now) ? 1u << wave : 0u);
-        if (wake != 0 && lane == 0) atomicOr(&dirty, wake);
+        if (wake != 0 && lane == 0) publish(wake);
       }
       if (!__syncthreads_or(fell)) break;
       moved = true;
