@@ -750,8 +750,39 @@ __global__ __launch_bounds__(kDwThreads, 2) void k_conv_dw(
   const int strip = 2 * kh + (g >> 1), pix = 8 * (g & 1) + (r >> 2);
   const uint16_t *const xl = &xs[(strip * S::kXPix + pix) * S::kXS + 16 * cih + 4 * (r & 3)];
   const uint16_t *const zl = &zs[(strip * S::kZPix + pix) * S::kZS + 32 * coh + 4 * (r & 3)];
+  // this lane's sums in part, by 32-bit offsets from the chunk's (inputs beyond cin:
+  // beyond them all)
+  const __amdgpu_buffer_rsrc_t sums = __builtin_amdgcn_make_buffer_rsrc(
+      part + static_cast<long>(blockIdx.y) * 9 * cout * cin, 0, 36 * cout * cin, kRsrc);
+  const uint32_t sum_at = ci0 + 16 * cih + r < cin
+                              ? static_cast<uint32_t>((co0 + 32 * coh + 4 * g) * cin + ci0 +
+                                                      16 * cih + r) * 4u
+                              : kOob;
+  auto each_sum = [&](auto f) {
+#pragma unroll
+    for (int t = 0; t < 9; t++)
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) f(t, h, i, 4 * (t * cout + 16 * h + i) * cin);
+  };
+  auto store_sum = [&](int t, int h, int i, int at) {
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[t][h][i]), sums,
+                                          static_cast<int>(sum_at), at, 0);
+  };
+  // Where one wave sums all of the workgroup's pixels, its sums go to memory
+  // halfway and start again from zero: an accumulator's rounding error grows with
+  // its sum's length (against sums in 32 times as many chunks, the 288 -> 128 layer
+  // of 32 samples of 256 x 256 is off by 2.4e-7 of its norm in one go, by 2.0e-7
+  // this way).  It costs the loss and gradients of that batch 2.5%.
+  const long half = NK == 1 && u1 - u0 > 1 ? u0 + (u1 - u0 + 1) / 2 : u1;
   if (u0 < u1) fetch(u0);
   for (long unit = u0; unit < u1; unit++) {
+    if (NK == 1 && unit == half) {
+      each_sum(store_sum);
+#pragma unroll
+      for (int t = 0; t < 9; t++) acc[t][0] = acc[t][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
     stage();
     __syncthreads();
     if (unit + 1 < u1) fetch(unit + 1);
@@ -809,17 +840,12 @@ __global__ __launch_bounds__(kDwThreads, 2) void k_conv_dw(
       atomicAdd(&db[co0 + threadIdx.x], sum);
     }
   }
-  if (kh == 0 && ci0 + 16 * cih + r < cin) {
-    float *const dst = part + static_cast<long>(blockIdx.y) * 9 * cout * cin;
-#pragma unroll
-    for (int t = 0; t < 9; t++)
-#pragma unroll
-      for (int h = 0; h < 2; h++)
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-          dst[(static_cast<long>(t) * cout + co0 + 32 * coh + 16 * h + 4 * g + i) * cin + ci0 +
-              16 * cih + r] = acc[t][h][i];
-  }
+  if (half < u1)
+    each_sum([&](int t, int h, int i, int at) {
+      acc[t][h][i] += __uint_as_float(
+          __builtin_amdgcn_raw_buffer_load_b32(sums, static_cast<int>(sum_at), at, 0));
+    });
+  if (kh == 0) each_sum(store_sum);
 }
 
 // dw[i] = sum over chunks of part[chunk][i]; 64 elements x 16 chunk lanes per
@@ -1190,8 +1216,8 @@ int conv_fwd(fs_unet *u, const Conv &c, const ConvSrc &in, Tensor &out, const Te
 
 // Work split of the nine-tap weight-gradient kernel: about kDwTargetGroups
 // workgroups per layer, the two that fit on every CU (1024 of them: 4.47 ms
-// against 4.29 for the loss and gradients of 32 samples).  Levels whose size is not a multiple of the strips use
-// k_conv3x3_dw.
+// against 4.29 for the loss and gradients of 32 samples).  Levels whose size is
+// not a multiple of the strips use k_conv3x3_dw.
 constexpr long kDwTargetGroups = 512;
 struct DwPlan {
   bool tiled = false;
