@@ -541,25 +541,43 @@ int timed_steps(fs_ensemble *e, const fs_schedule &s, int steps, double *ms_per_
 
 // Coordinate search over the schedule knobs, each candidate timed on
 // tune_trial real steps; stops early when `budget` steps are used.  A candidate
-// has to be ahead by more than one step's time varies (3%); a knob is done with
-// its first value that is not, since more work per workgroup then only costs
-// more.  Returns the number of steps taken in *used.
+// has to be ahead of the best so far by more than one step's time varies (3%),
+// both as timed before it and as timed again behind it: the first steps of a run
+// are its slowest, and what comes later would win by that alone.  A knob is done
+// with its first value that is not ahead, since more work per workgroup then only
+// costs more.  Returns the number of steps taken in *used.
 int autotune(fs_ensemble *e, int budget, int *used) {
   *used = 0;
   fs_schedule best = e->sched;
   double best_ms = -1;
+  bool open = true;   // steps are left
+  auto trial = [&](const fs_schedule &c, double *ms) {
+    open = *used + e->tune_trial <= budget;
+    if (!open) return FS_OK;
+    FS_TRY(timed_steps(e, c, e->tune_trial, ms));
+    *used += e->tune_trial;
+    e->tune_cand.push_back(c);
+    e->tune_ms.push_back(*ms);
+    return FS_OK;
+  };
   auto search = [&](int fs_schedule::*knob, std::initializer_list<int> values) {
     for (int v : values) {
       fs_schedule c = best;
       c.*knob = v;
       if (best_ms >= 0 && c.*knob == best.*knob) continue;   // timed already
-      if (*used + e->tune_trial > budget) return FS_OK;
-      double ms = 0;
-      FS_TRY(timed_steps(e, c, e->tune_trial, &ms));
-      *used += e->tune_trial;
-      e->tune_cand.push_back(c);
-      e->tune_ms.push_back(ms);
-      if (best_ms >= 0 && !(ms < 0.97 * best_ms)) return FS_OK;
+      double ms = 0, again = 0;
+      FS_TRY(trial(c, &ms));
+      if (!open) return FS_OK;
+      if (best_ms < 0) {
+        best_ms = ms;
+        best = c;
+        continue;
+      }
+      if (!(ms < 0.97 * best_ms)) return FS_OK;
+      FS_TRY(trial(best, &again));
+      if (!open) return FS_OK;
+      best_ms = std::min(best_ms, again);
+      if (!(ms < 0.97 * best_ms)) return FS_OK;
       best_ms = ms;
       best = c;
     }

@@ -80,8 +80,9 @@ __device__ __forceinline__ f32x4 mfma16(uint4 a, uint4 b, f32x4 c) {
 //
 // Each accumulator adds its taps in order 0..8 within a step and the
 // steps in order, so the sums are those of a plain loop over (channel step,
-// tap), bit for bit, at every R.  kTapOuter (levels smaller than 8 x 16,
-// few and latency-bound): the loop over (tap, channel step).
+// tap), bit for bit, at every R.  kTapOuter (levels smaller than 8 x 16): those
+// of the loop over (tap, channel step), the order these levels have always been
+// summed in; their outputs keep their bits.
 // ---------------------------------------------------------------------------
 constexpr int kNB = 32;            // outputs per wave
 constexpr int kKC = 32;            // input channels per step

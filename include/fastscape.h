@@ -142,17 +142,18 @@ int fs_get_h(fs_model *m, double *out, size_t count);
 int fs_set_h(fs_model *m, const double *in, size_t count);
 
 /* Per-stage times in microseconds, in FS_T_* order (RB:380-387).  Stage
- * times are device time between HIP events; Overall is
- * host wall time of fs_run / fs_step plus construction.  On the level path
- * events bracket each stage.  On the tile path
- * (below) donors, levels and accumulation are one kernel and uplift and
- * erosion another, and events bracket batches of steps; their time is split
- * over the stages by phase timestamps
- * that the kernels record on one step in 32.  On the tile-graph path,
- * events bracket a run of steps and the stages of its first one, which split
- * the run's time: DetermineDonors is the in-tile structure, GenerateOrder the
- * links between tiles, FlowAcc the tiers of and sums over them, Uplift is
- * fused into Erosion (which also finishes the counts).  FS_PATH_LEVELS gives the reference's stage split. */
+ * times are device time between HIP events, complete when fs_run / fs_step
+ * returns; Overall is host wall time of fs_run / fs_step plus construction.
+ * On the level path events bracket each stage.  On the tile path (below)
+ * donors, levels and accumulation are one kernel and uplift and erosion
+ * another, and events bracket batches of steps; their time is split by the
+ * latest sampled step (one in 32, counted across calls, and the first after
+ * fs_reset_timers): its kernels' event times, and phase timestamps that its
+ * kernels record.  On the tile-graph path, events bracket a run of steps and
+ * the stages of its first one, which split the run's time: DetermineDonors is
+ * the in-tile structure, GenerateOrder the links between tiles, FlowAcc the
+ * tiers of and sums over them, Uplift is fused into Erosion (which also
+ * finishes the counts).  FS_PATH_LEVELS gives the reference's stage split. */
 int fs_get_timers(fs_model *m, uint64_t us[FS_NUM_TIMERS]);
 int fs_reset_timers(fs_model *m);
 

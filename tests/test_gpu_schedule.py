@@ -42,6 +42,19 @@ def test_search_leaves_a_bad_schedule():
         assert ens.get_schedule().as_dict()["tiles_per_claim"] < 16
 
 
+def test_slow_first_steps_pick_no_schedule():
+    """A run's first steps are its slowest (code and memory are touched for the first
+    time, drainage is new); two tiles a workgroup take half as long again as one."""
+    note("search from a fresh start")
+    specs = [(160, 160, bench(keq=1e-5 * (1 + i % 7)), i) for i in range(28)]   # 252 tiles
+    for _ in range(5):
+        with make(specs) as ens:
+            ens.autotune(1)
+            ens.run(19)
+            note("%s" % ens.tune_log())
+            assert ens.get_schedule().as_dict()["tiles_per_claim"] == 1
+
+
 # the last workgroup's share: whole, one item, all but one, and more than there are
 @pytest.mark.parametrize("per", [2, 3, 5, 16])
 @pytest.mark.parametrize("specs", [
