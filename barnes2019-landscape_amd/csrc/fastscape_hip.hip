@@ -146,6 +146,8 @@ struct fs_model {
   // has left in rcv launches none: it is a run of its own.
   hipEvent_t tev[5] = {};             // batch: start, the sampled step's kernels, end
   TileShares shares{};                // of the last sample
+  bool warm = false;                  // it was not the model's first
+  double unsplit_ms = 0;              // of batches before a warm sample
   uint64_t phase_seen[kPhaseStride] = {};   // the phase ticks' sums when last read
   long long since_sample = kPhaseEvery;     // tile steps since the last sample
   struct GraphRun {
@@ -287,6 +289,8 @@ int graph_begin(fs_model *m, bool alone, const hipEvent_t **ev) {
   static const hipEvent_t none[8] = {};
   *ev = none;
   const int last = m->graph_open;
+  // a model's first tile-graph step may hold the loading of the kernels
+  alone = alone || m->graph_steps == 0;
   if (last >= 0 && !m->graph_alone && !alone) return FS_OK;
   FS_TRY(graph_close(m));
   // a run at most waits to be collected here, behind one step alone: a tile
@@ -343,8 +347,15 @@ void add_tile_time(fs_model *m, double ms, const TileShares &s, bool recv, bool 
     m->stage_ms[FS_T_RECEIVERS + i] += ms * (k1 * s.acc[i] + k2 * s.ero[i]) / sum;
 }
 
+// The time of steps that waited for a warm sample.
+void split_rest(fs_model *m) {
+  if (m->unsplit_ms > 0) add_tile_time(m, m->unsplit_ms, m->shares, true, true);
+  m->unsplit_ms = 0;
+}
+
 // Whole microseconds of the stage times so far into the timers.
 void fold_timers(fs_model *m) {
+  split_rest(m);
   for (int i = 0; i < 6; i++) {
     const double ms = m->stage_ms[FS_T_RECEIVERS + i];
     const uint64_t whole = static_cast<uint64_t>(ms * 1000.0);
@@ -845,7 +856,9 @@ int finish_batch(fs_model *m, bool sampled) {
 // step was taken, and is the sample from now on.  One that was not has no
 // erosion: its events say what its kernels took, and the next step is sampled.
 // recv_ms: without receivers of its own (the same step with the deeper halo), what
-// those took.  Every batch is sampled until one has given shares.
+// those took.  Every batch is sampled until one has given shares; a model's first
+// sample may hold the loading of the kernels (30 ms), so it stands for itself
+// alone, and the next batch is sampled again.
 int account_batch(fs_model *m, bool sampled, bool taken, double *recv_ms, bool again) {
   if (!m->tev[0]) return FS_OK;
   float t = 0.f;
@@ -867,15 +880,21 @@ int account_batch(fs_model *m, bool sampled, bool taken, double *recv_ms, bool a
     ticks[k] = static_cast<double>(sum - m->phase_seen[k]);
     m->phase_seen[k] = sum;
   }
-  if (taken) {
-    const double step[3] = {*recv_ms, again ? ms[0] + ms[1] : ms[1], ms[2]};
-    m->shares = tile_shares(step, ticks);
-    m->since_sample = 0;
-    add_tile_time(m, all, m->shares, !again, true);
-  } else {
+  if (!taken) {
     const double step[3] = {again ? 0 : ms[0], all - (again ? 0 : ms[0]), 0};
     add_tile_time(m, all, tile_shares(step, ticks), !again, false);
+    return FS_OK;
   }
+  const double step[3] = {*recv_ms, again ? ms[0] + ms[1] : ms[1], ms[2]};
+  const double own = std::min(all, ms[0] + ms[1] + ms[2]);
+  m->shares = tile_shares(step, ticks);
+  add_tile_time(m, own, m->shares, !again, true);
+  m->unsplit_ms += all - own;
+  if (m->warm) {
+    split_rest(m);
+    m->since_sample = 0;
+  }
+  m->warm = true;
   return FS_OK;
 }
 
@@ -1344,6 +1363,7 @@ int fs_get_timers(fs_model *m, uint64_t us[FS_NUM_TIMERS]) {
 int fs_reset_timers(fs_model *m) {
   if (!m) return FS_ERR_INVALID_ARGUMENT;
   m->since_sample = kPhaseEvery;   // what is timed from here on has a sample of its own
+  m->unsplit_ms = 0;
   for (int i = 0; i < FS_NUM_TIMERS; i++) {
     m->timer_us[i] = 0;
     m->stage_ms[i] = 0;

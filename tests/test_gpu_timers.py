@@ -4,12 +4,14 @@ a kernel of their own; the tile erosion's time goes to GenerateOrder, Uplift and
 Erosion, GenerateOrder also gets a part of the accumulation's.  A sample of steps
 stands for the others: tolerance 4 points of the whole, of which the events
 around the sampled kernels take up to 2 at the smaller sizes (some 3 us of 150)."""
+import subprocess
+
 import numpy as np
 import pytest
 
 import fastscape_amd as fa
 from conftest import cone_terrain
-from test_gpu_parity import note
+from test_gpu_parity import CLI, note
 
 pytestmark = pytest.mark.gpu
 
@@ -115,3 +117,19 @@ def test_depression_filling_is_no_stage(path):
     kernels, stages, overall = out[0][0], out[1][1], out[1][2]
     note("kernels %.0f us, stages %.0f, overall %.0f" % (kernels, stages, overall))
     assert 0.5 * kernels <= stages <= 2 * kernels
+
+
+@pytest.mark.parametrize("side,steps", [(101, 60), (1001, 60)])
+def test_first_step_of_a_process(tmp_path, side, steps):
+    """Loading the kernels takes some 30 ms of a process's first step; that step does
+    not stand for the others, whose accumulation takes 8 us and erosion 10 at least."""
+    note("timers of a process of its own, %d^2" % side)
+    r = subprocess.run([CLI, "--preset=benchmark", str(side), str(steps), str(tmp_path / "o.dem"),
+                        "1"], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr
+    t = dict(line[2:].split("=")[:2] for line in r.stdout.splitlines() if line.startswith("t "))
+    us = {k.strip().split(": ")[-1]: int(v.split()[0]) for k, v in t.items()}
+    note("%s" % us)
+    assert us["DetermineDonors"] + us["FlowAcc"] + us["GenerateOrder"] + us["Uplift"] + \
+        us["Erosion"] >= 18 * steps
+    assert us["Uplift"] > 0
