@@ -113,13 +113,14 @@ struct fs_model {
   tile32::TilePlan *plan32 = nullptr;  // the same for the 32-cell halo (on first use)
   uint64_t *status = nullptr;
   unsigned long long *ticket = nullptr;
-  unsigned long long *phase = nullptr;   // tile kernels' phase ticks (stage timers)
+  unsigned long long *phase = nullptr;   // tile kernels' phase ticks (stage timers); right
+                                         // before hdr, so that one copy fetches both
   int32_t *fill_flag = nullptr;          // per launch of a batch: it changed a cell
   bool fill_mode = false;                // fill depressions before every step
 
   // host mirrors
   int32_t *hdr_h = nullptr;      // pinned: header + level counts
-  uint64_t *phase_h = nullptr;   // pinned: the phase ticks
+  uint64_t *phase_h = nullptr;   // pinned: the phase ticks, right before hdr_h
   int32_t *levels_h = nullptr;   // pinned: levels uploaded each step
   std::vector<int32_t> counts, levels;
   int32_t nlevel = 0, maxdepth = 0, prev_maxdepth = FS_MAX_LEVELS;
@@ -144,7 +145,9 @@ struct fs_model {
   // is, and split by the shares of the last sampled step that was taken; a run
   // of tile-graph steps by its first one's.  A step whose receivers a tile attempt
   // has left in rcv launches none: it is a run of its own.
-  hipEvent_t tev[5] = {};             // batch: start, the sampled step's kernels, end
+  // batch: start; the sampled step's kernels; end; the sampled step's start unless
+  // it is the batch's
+  hipEvent_t tev[6] = {};
   TileShares shares{};                // of the last sample
   bool warm = false;                  // it was not the model's first
   double unsplit_ms = 0;              // of batches before a warm sample
@@ -394,7 +397,7 @@ void free_model(fs_model *m) {
                     static_cast<void *>(m->dmask), static_cast<void *>(m->lvl),
                     static_cast<void *>(m->depth),
                     static_cast<void *>(m->jump), static_cast<void *>(m->list),
-                    static_cast<void *>(m->stack), static_cast<void *>(m->hdr),
+                    static_cast<void *>(m->stack),
                     static_cast<void *>(m->rdir), static_cast<void *>(m->fdon),
                     static_cast<void *>(m->ndon), static_cast<void *>(m->cnt_s),
                     static_cast<void *>(m->levels_d), static_cast<void *>(m->cnt),
@@ -411,7 +414,6 @@ void free_model(fs_model *m) {
                     static_cast<void *>(m->cells), static_cast<void *>(m->items),
                     static_cast<void *>(m->graph_grid), static_cast<void *>(m->graph_list)})
     if (ptr) (void)hipFree(ptr);
-  if (m->hdr_h) (void)hipHostFree(m->hdr_h);
   if (m->phase_h) (void)hipHostFree(m->phase_h);
   if (m->levels_h) (void)hipHostFree(m->levels_h);
   for (auto &set : m->ev)
@@ -479,32 +481,30 @@ int create_model(int W, int H, const fs_params *p, const double *h_init, uint32_
   // at least kFactCache counts, so the tile kernels' LDS cache stays in bounds
   const size_t kmax = std::max<size_t>(N, kFactCache - 1);
   FS_TRY(fs::dev_alloc(&m->ftab, 2 * (kmax + 1)));
-  FS_TRY(fs::dev_alloc(&m->hdr, kHdrAlloc));
+  FS_TRY(fs::dev_alloc(&m->phase, kPhaseWords + (kHdrAlloc + 1) / 2));
+  m->hdr = reinterpret_cast<int32_t *>(m->phase + kPhaseWords);
   FS_TRY(fs::dev_alloc(&m->levels_d, FS_MAX_LEVELS + 4));
   FS_TRY(fs::dev_alloc(&m->status, ntiles));
   FS_TRY(fs::dev_alloc(&m->ticket, 1));
   const size_t plan_tiles = static_cast<size_t>((m->W + kTile - 1) / kTile) *
                             static_cast<size_t>((m->H + kTile - 1) / kTile);
   FS_TRY(fs::dev_alloc(&m->plan, plan_tiles));
-  FS_TRY(fs::dev_alloc(&m->phase, static_cast<size_t>(kPhaseSlots) * kPhaseStride));
   FS_TRY(fs::dev_alloc(&m->fill_flag, kFillBatch));
-  if (hipHostMalloc(reinterpret_cast<void **>(&m->hdr_h),
-                    (kHdrInts + FS_MAX_LEVELS + 3) * sizeof(int32_t)) != hipSuccess ||
-      hipHostMalloc(reinterpret_cast<void **>(&m->phase_h),
-                    static_cast<size_t>(kPhaseSlots) * kPhaseStride * sizeof(uint64_t)) !=
-          hipSuccess ||
+  if (hipHostMalloc(reinterpret_cast<void **>(&m->phase_h),
+                    kPhaseWords * sizeof(uint64_t) +
+                        (kHdrInts + FS_MAX_LEVELS + 3) * sizeof(int32_t)) != hipSuccess ||
       hipHostMalloc(reinterpret_cast<void **>(&m->levels_h),
                     (FS_MAX_LEVELS + 4) * sizeof(int32_t)) != hipSuccess) {
     fs::set_last_error("hipHostMalloc failed");
     return FS_ERR_OUT_OF_MEMORY;
   }
+  m->hdr_h = reinterpret_cast<int32_t *>(m->phase_h + kPhaseWords);
   FS_HIP_TRY(hipMemsetAsync(m->rcv, 0xFF, N + 16, m->stream));   // RB:361-362
-  FS_HIP_TRY(hipMemsetAsync(m->hdr, 0, kHdrAlloc * sizeof(int32_t), m->stream));
   FS_HIP_TRY(hipMemsetAsync(m->status, 0, ntiles * sizeof(uint64_t), m->stream));
   FS_HIP_TRY(hipMemsetAsync(m->ticket, 0, sizeof(unsigned long long), m->stream));
   FS_HIP_TRY(hipMemsetAsync(m->plan, 0, plan_tiles * sizeof(TilePlan), m->stream));
   FS_HIP_TRY(hipMemsetAsync(m->phase, 0,
-                            static_cast<size_t>(kPhaseSlots) * kPhaseStride * sizeof(uint64_t),
+                            kPhaseWords * sizeof(uint64_t) + kHdrAlloc * sizeof(int32_t),
                             m->stream));
   FS_HIP_TRY(hipMemsetAsync(m->cnt, 0, N * sizeof(uint32_t), m->stream));
   {
@@ -542,10 +542,14 @@ int create_model(int W, int H, const fs_params *p, const double *h_init, uint32_
 
 // Read the header (max level, unfinished count, error bits) and the level
 // histogram; synchronises the stream.
-int fetch_header(fs_model *m, int ncounts) {
+int fetch_header(fs_model *m, int ncounts, bool phase = false) {
   ncounts = std::min(ncounts, FS_MAX_LEVELS + 3);
-  FS_HIP_TRY(hipMemcpyAsync(m->hdr_h, m->hdr, (kHdrInts + ncounts) * sizeof(int32_t),
-                            hipMemcpyDeviceToHost, m->stream));
+  const size_t hdr = (kHdrInts + ncounts) * sizeof(int32_t);
+  if (phase)
+    FS_HIP_TRY(hipMemcpyAsync(m->phase_h, m->phase, kPhaseWords * sizeof(uint64_t) + hdr,
+                              hipMemcpyDeviceToHost, m->stream));
+  else
+    FS_HIP_TRY(hipMemcpyAsync(m->hdr_h, m->hdr, hdr, hipMemcpyDeviceToHost, m->stream));
   FS_HIP_TRY(hipStreamSynchronize(m->stream));
   return FS_OK;
 }
@@ -841,52 +845,53 @@ int launch_tile_step(fs_model *m, int halo, const double *h_in, double *h_out, i
 // header and, of a sampled batch, the phase ticks.
 int finish_batch(fs_model *m, bool sampled) {
   FS_TRY(mark(m->tev[4], m->stream));
-  if (sampled)
-    FS_HIP_TRY(hipMemcpyAsync(m->phase_h, m->phase,
-                              static_cast<size_t>(kPhaseSlots) * kPhaseStride * sizeof(uint64_t),
-                              hipMemcpyDeviceToHost, m->stream));
-  FS_TRY(fetch_header(m, 0));
+  FS_TRY(fetch_header(m, 0, sampled));
   m->hdr_fresh = true;
   FS_TRY(graph_collect(m));
   return kt_collect(m);
 }
 
-// The time of a finished batch (between tev[0] and tev[4]) for the stage timers.
-// sampled: its first step's kernels end at tev[1], tev[2] and tev[3]; taken: that
-// step was taken, and is the sample from now on.  One that was not has no
-// erosion: its events say what its kernels took, and the next step is sampled.
-// recv_ms: without receivers of its own (the same step with the deeper halo), what
-// those took.  Every batch is sampled until one has given shares; a model's first
-// sample may hold the loading of the kernels (30 ms), so it stands for itself
-// alone, and the next batch is sampled again.
-int account_batch(fs_model *m, bool sampled, bool taken, double *recv_ms, bool again) {
+// The time of a finished batch (between tev[0] and tev[4]), of which the first
+// `taken` steps were taken, for the stage timers.  at: the sampled step, whose
+// kernels end at tev[1], tev[2] and tev[3], or -1.  If it was taken, it is the
+// sample from now on.  One that was too deep has no erosion: its events say what
+// its kernels took, and the next batch is sampled.  recv_ms: without receivers of
+// its own (`again`: the same step with the deeper halo), what those took.  Every
+// batch is sampled until one has given shares; a model's first sample may hold the
+// loading of the kernels (30 ms), so it stands for itself alone, and the next batch
+// is sampled again.
+int account_batch(fs_model *m, int at, int taken, double *recv_ms, bool again) {
   if (!m->tev[0]) return FS_OK;
   float t = 0.f;
   FS_HIP_TRY(hipEventElapsedTime(&t, m->tev[0], m->tev[4]));
   const double all = t;
-  if (!sampled) {
-    add_tile_time(m, all, m->shares, !again, taken);
+  double ms[3] = {}, ticks[kPhaseStride];
+  if (at >= 0) {
+    for (int i = 0; i < 3; i++) {
+      FS_HIP_TRY(hipEventElapsedTime(&t, m->tev[i == 0 && at > 0 ? 5 : i], m->tev[i + 1]));
+      ms[i] = t;
+    }
+    if (!again) *recv_ms = ms[0];
+    for (int k = 0; k < kPhaseStride; k++) {
+      uint64_t sum = 0;
+      for (int r = 0; r < kPhaseSlots; r++) sum += m->phase_h[r * kPhaseStride + k];
+      ticks[k] = static_cast<double>(sum - m->phase_seen[k]);
+      m->phase_seen[k] = sum;
+    }
+  }
+  if (at < 0 || taken < at) {
+    add_tile_time(m, all, m->shares, !again, taken > 0);
     return FS_OK;
   }
-  double ms[3] = {}, ticks[kPhaseStride];
-  for (int i = 0; i < 3; i++) {
-    FS_HIP_TRY(hipEventElapsedTime(&t, m->tev[i], m->tev[i + 1]));
-    ms[i] = t;
-  }
-  if (!again) *recv_ms = ms[0];
-  for (int k = 0; k < kPhaseStride; k++) {
-    uint64_t sum = 0;
-    for (int r = 0; r < kPhaseSlots; r++) sum += m->phase_h[r * kPhaseStride + k];
-    ticks[k] = static_cast<double>(sum - m->phase_seen[k]);
-    m->phase_seen[k] = sum;
-  }
-  if (!taken) {
-    const double step[3] = {again ? 0 : ms[0], all - (again ? 0 : ms[0]), 0};
-    add_tile_time(m, all, tile_shares(step, ticks), !again, false);
+  const double own = std::min(all, ms[0] + ms[1] + ms[2]);
+  if (taken == at) {
+    const double step[3] = {again ? 0 : ms[0], ms[1] + ms[2] + (again ? ms[0] : 0), 0};
+    const TileShares failed = tile_shares(step, ticks);
+    add_tile_time(m, own, failed, !again, false);
+    add_tile_time(m, all - own, at > 0 ? m->shares : failed, !again, at > 0);
     return FS_OK;
   }
   const double step[3] = {*recv_ms, again ? ms[0] + ms[1] : ms[1], ms[2]};
-  const double own = std::min(all, ms[0] + ms[1] + ms[2]);
   m->shares = tile_shares(step, ticks);
   add_tile_time(m, own, m->shares, !again, true);
   m->unsplit_ms += all - own;
@@ -931,14 +936,18 @@ int tile_steps(fs_model *m, long long want, int *done, bool *stuck) {
   const int n = m->ktiming || m->fill_mode
                     ? 1
                     : static_cast<int>(std::min<long long>(want, std::min(m->batch, kMaxBatch)));
-  // one step in kPhaseEvery is the timers' sample
+  // one step in kPhaseEvery is the timers' sample: a batch's second, if it has one
+  // (the first one's receivers wait for the launches, 10 us of 42 at 4096^2), but
+  // never the second until there are shares
   const bool sample = m->phase && m->since_sample >= kPhaseEvery;
+  const int at = !sample ? -1 : m->warm && n > 1 ? 1 : 0;
   const hipEvent_t none = nullptr;
   FS_TRY(mark(m->tev[0], m->stream));
   double *h_in = m->h, *h_out = m->h_alt;
   for (int i = 0; i < n; i++) {
     int32_t *slot = m->hdr + kHdrSlots + i * kSlotInts;
-    const bool timed = sample && i == 0;
+    const bool timed = i == at;
+    if (timed && i > 0) FS_TRY(mark(m->tev[5], m->stream));
     FS_TRY(launch_receivers(m, h_in, i ? slot - kSlotInts : nullptr, slot,
                             halo == kHalo ? -1 : kHalo));
     if (timed) FS_TRY(mark(m->tev[1], m->stream));
@@ -955,7 +964,7 @@ int tile_steps(fs_model *m, long long want, int *done, bool *stuck) {
   take_tile_steps(m, taken, halo);   // a failed solve's step was taken, none behind it
   *done = taken;
   double recv_ms = 0;
-  FS_TRY(account_batch(m, sample, taken > 0, &recv_ms, false));
+  FS_TRY(account_batch(m, at, taken, &recv_ms, false));
   m->since_sample += taken;
   FS_TRY(device_error_status(m->hdr_h[2]));
   m->batch = taken == n ? std::min(2 * m->batch, kMaxBatch) : 4;
@@ -970,7 +979,7 @@ int tile_steps(fs_model *m, long long want, int *done, bool *stuck) {
   if (halo == kHalo) {
     // the same step again with the 32-cell halo
     int32_t *slot = m->hdr + kHdrSlots;
-    const bool timed = sample && taken == 0;   // the sample is still to be had
+    const bool timed = at == 0 && taken == 0;   // the sample is still to be had
     FS_TRY(mark(m->tev[0], m->stream));
     hipLaunchKernelGGL(k_slot_reset, dim3(1), dim3(64), 0, m->stream, slot);
     FS_TRY(check_launch());
@@ -985,7 +994,7 @@ int tile_steps(fs_model *m, long long want, int *done, bool *stuck) {
       m->tile_halo = slots[kSlotDeepest] <= kHalo ? kHalo : tile32::kHalo;
       *done = taken + 1;
     }
-    FS_TRY(account_batch(m, timed, fits, &recv_ms, true));
+    FS_TRY(account_batch(m, timed ? 0 : -1, fits ? 1 : 0, &recv_ms, true));
     if (fits) m->since_sample++;
     FS_TRY(device_error_status(m->hdr_h[2]));
     if (*done > taken) return FS_OK;

@@ -1115,6 +1115,7 @@ constexpr int kPhaseSample = 16;     // workgroups per sampled one in a timed la
 constexpr int kPhaseEvery = 32;      // tile steps per timed step
 constexpr int kPhaseSlots = 32;
 constexpr int kPhaseStride = 8;
+constexpr size_t kPhaseWords = static_cast<size_t>(kPhaseSlots) * kPhaseStride;
 enum PhaseId {
   kPhAccLoad = 0,    // receivers -> region words (the donor structure)   Donors
   kPhAccWalk,        // receiver-chain walks: counts and levels          FlowAcc
