@@ -229,8 +229,8 @@ __device__ __forceinline__ void load_cols(__amdgpu_buffer_rsrc_t r, uint32_t xo,
 // 16 at every size: 19.1 -> 9.0 us at 1000^2, 22.4 -> 15.9 at 2048^2, 93.5 ->
 // 86.3 at 6000^2, 227 -> 223.5 at 10000^2 (HIP events, their own 4 us
 // included); four rows read 1.5 rows per row decided (241 us at 10000^2),
-// sixteen leave too few waves (12.1 at 1000^2).  Bound by VALU issue at the
-// largest sizes (1.04 GB in 0.22 ms).
+// sixteen leave too few waves (12.1 at 1000^2).  Bound by memory at the
+// largest sizes (1.23 GB in 0.22 ms, a copy's rate; VALU active 71% of the cycles).
 // On the tile path it also opens its step's slot.  prev is the slot of the
 // batch's previous step (null for its first): when that step was not taken, a
 // solve failed, or its drainage was no deeper than `shallow` levels (the

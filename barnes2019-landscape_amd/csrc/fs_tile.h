@@ -444,7 +444,8 @@ __device__ __forceinline__ int tile_acc_body(AccShared &sh, const uint8_t *__res
     }
   }
   // Of the halo's cells, those walk that drain into the tile: about 107 of 5120
-  // on fresh terrain.  The walks are bound by the LDS's returning atomics, and
+  // on fresh terrain.  The walks are bound by their instructions (VALU active 95% of
+  // the kernel's cycles) and the LDS's returning atomics, and
   // those of the whole halo are more than half of them (10000 x 10000 after 5
   // steps: 494 us with all of them, 390 now; with the deep halo, 6000 x 6000
   // after 330 steps, 385 and 275, 1500 x 1101 48 and 30; 101 x 101, a tile or

@@ -76,7 +76,9 @@ __device__ __forceinline__ f32x4 mfma16(uint4 a, uint4 b, f32x4 c) {
 // the finished tile, so none of them is a pass over memory of its own.
 // Ranking 256 candidates at 256 x 256: 12.75 -> 7.43 ms (391 -> 672 TFLOP/s);
 // the widest layers run at 820 to 990 TFLOP/s, the 32-channel layers of the
-// top level at 3.4 TB/s, bound by memory.
+// top level at 3.4 TB/s.  Over all layers of a training step the matrix units are
+// busy 27% of the cycles, LDS 8%, and waves wait 46% of theirs: two share a SIMD
+// (253 registers), and the latency of their rows bounds them.
 //
 // Each accumulator adds its taps in order 0..8 within a step and the
 // steps in order, so the sums are those of a plain loop over (channel step,
@@ -609,7 +611,10 @@ __global__ __launch_bounds__(256) void k_reduce_chunks(const float *__restrict__
 //
 // With 8 x 8 transposes in registers, three shifted copies of the patch and
 // three waves per workgroup, the weight gradients took 1.95 ms of the backward
-// pass of 32 samples of 256 x 256 (321 TFLOP/s); they take 1.10 (570).
+// pass of 32 samples of 256 x 256 (321 TFLOP/s); they take 1.20 (523).  <2, 1> moves
+// its bytes at 5.5 TB/s, a copy's rate (every block of inputs reads the gradients
+// again); <1, 2> is bound by no one unit (matrix units busy 18% of the cycles, LDS
+// 24%, 3.8 TB/s).
 // ---------------------------------------------------------------------------
 typedef short i16x4 __attribute__((ext_vector_type(4)));
 constexpr int kDwThreads = 256;

@@ -360,7 +360,7 @@ def bench_inversion(args, fa):
                          "final_loss": float(hist[-1]), "tflops": train_tflops},
             "roofline": {"bound": "mfma", "achieved": round(inf_tflops, 2), "peak": 2500.0,
                          "unit": "TFLOP/s", "frac": round(inf_tflops / 2500.0, 4),
-                         "traffic": None, "kernel": "U-Net inference (k_conv3x3)",
+                         "traffic": None, "kernel": "U-Net inference (k_conv)",
                          "inference_seconds": t_inf},
             "cpu_baseline": cpu}
     print(json.dumps(line))
@@ -402,7 +402,7 @@ def bench_unet(args, fa):
                        "training_tflops": tr, "training_samples": tr_samples},
             "roofline": {"bound": "mfma", "achieved": round(inf, 2), "peak": 2500.0,
                          "unit": "TFLOP/s", "frac": round(inf / 2500.0, 4), "traffic": None,
-                         "kernel": "U-Net forward (k_conv3x3)"},
+                         "kernel": "U-Net forward (k_conv)"},
             "cpu_baseline": None}
     print(json.dumps(line))
 
